@@ -28,6 +28,7 @@ UNITS = [
     ("afx_implicit.hip", ["-ffp-contract=off"]),
     ("afx_adjoint.hip", ["-ffp-contract=off"]),
     ("afx_adjoint_sa.hip", ["-ffp-contract=off"]),
+    ("afx_exchange.hip", ["-ffp-contract=off"]),   # vectors crossing the C ABI: layout kernels, staging
     ("afx_mapper.hip", ["-ffp-contract=off"]),   # multigrid level prolongation
     ("afx_capi.hip", ["-ffp-contract=off"]),
     ("afx_vlm.hip", ["-ffp-contract=fast"]),    # vortex lattice, FP32 LU, FP64 refinement

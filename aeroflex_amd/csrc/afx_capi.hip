@@ -24,6 +24,7 @@
 #include "afx_tiles.hpp"
 #include "afx_implicit.hpp"
 #include "afx_adjoint_kernels.hpp"
+#include "afx_exchange.hpp"
 #include "afx_mapper.hpp"
 #include "afx_post.hpp"
 
@@ -85,6 +86,8 @@ struct afx_rans {
     double cfl = 1.0;
 
     std::vector<int32_t> c_new2old, c_old2new, f_new2old, f_old2new;
+    DBuf<int32_t> o2n;   // c_old2new on the device
+    DBuf<double> xrows;  // rows of a vector too large for the direct exchange (afx_exchange.hpp)
 
     // geometry (FP64 and FP32 copies)
     DBuf<double> xc, yc, area, fnx, fny, flen, fxf, fyf, fgw, lsq;
@@ -198,8 +201,10 @@ struct afx_rans {
     std::vector<double> bface_vars;        // 4 per boundary face: mach angle T p
     bool q32_valid = false;
 
+    afx_rans() { staging_retain(); }
     ~afx_rans() {
         if (stream) (void)hipStreamDestroy(stream);
+        staging_release();
     }
 
     CellsT<double> cells64() const {
@@ -275,60 +280,105 @@ std::vector<T> to_device_order_faces(const afx_rans* h, const std::vector<double
     return out;
 }
 
-// device SoA [NV][nT] -> reference AoS q(4*i+k)
-int download_aos(afx_rans* h, const double* d, double* out, int nv = NV) {
-    std::vector<double> tmp((size_t)nv * h->nT);
-    HIPCHK(hipMemcpyAsync(tmp.data(), d, tmp.size() * 8, hipMemcpyDeviceToHost, h->stream));
-    HIPCHK(hipStreamSynchronize(h->stream));
-    for (int32_t i = 0; i < h->nT; ++i) {
-        int32_t o = h->c_new2old[i];
-        for (int k = 0; k < nv; ++k) out[(size_t)nv * o + k] = tmp[(size_t)k * h->nT + i];
+int ensure_rows(afx_rans* h, int nv) {
+    if (h->xrows.n >= (size_t)nv * h->nT) return AFX_OK;
+    if (h->xrows.p) { (void)hipFree(h->xrows.p); h->xrows.p = nullptr; h->xrows.n = 0; }
+    const hipError_t e = h->xrows.alloc((size_t)nv * h->nT);
+    if (e != hipSuccess) { h->xrows.p = nullptr; h->xrows.n = 0; }
+    HIPCHK(e);
+    return AFX_OK;
+}
+// device cells (planes of double or float, or one float4 per cell) -> nv values
+// per reference cell in the caller's memory (nv 4: q(4*i+k)); waits.  The call's staging
+// buffer st may carry scalars that earlier kernels of the call wrote.
+template <typename T>
+int fetch_rows(afx_rans* h, const Staging& st, const T* d, int nv, double* out) {
+    const size_t bytes = (size_t)nv * h->nT * sizeof(double);
+    const bool pinned = st.status() == hipSuccess;
+    if (pinned && bytes <= kDirectBytes) {
+        HIPCHK(launch_export_rows(h->stream, d, h->o2n.p, h->nT, nv, reinterpret_cast<double*>(st.piece(0))));
+        HIPCHK(hipStreamSynchronize(h->stream));
+        std::memcpy(out, st.piece(0), bytes);
+        return AFX_OK;
+    }
+    int rc = ensure_rows(h, nv);
+    if (rc) return rc;
+    HIPCHK(launch_export_rows(h->stream, d, h->o2n.p, h->nT, nv, h->xrows.p));
+    if (pinned) {
+        HIPCHK(st.to_host(h->stream, h->xrows.p, out, bytes));
+    } else {   // no pinned memory to be had
+        HIPCHK(hipMemcpyAsync(out, h->xrows.p, bytes, hipMemcpyDeviceToHost, h->stream));
+        HIPCHK(hipStreamSynchronize(h->stream));
     }
     return AFX_OK;
 }
-int download_aos32(afx_rans* h, const float* d, double* out) {
-    std::vector<float> tmp((size_t)NV * h->nT);
-    HIPCHK(hipMemcpyAsync(tmp.data(), d, tmp.size() * 4, hipMemcpyDeviceToHost, h->stream));
-    HIPCHK(hipStreamSynchronize(h->stream));
-    for (int32_t i = 0; i < h->nT; ++i) {
-        int32_t o = h->c_new2old[i];
-        for (int k = 0; k < NV; ++k) out[(size_t)NV * o + k] = (double)tmp[(size_t)k * h->nT + i];
+// the other way: nv values per reference cell -> planes; waits
+int send_rows(afx_rans* h, const Staging& st, const double* in, int nv, double* d) {
+    const size_t bytes = (size_t)nv * h->nT * sizeof(double);
+    const bool pinned = st.status() == hipSuccess;
+    if (pinned && bytes <= kDirectBytes) {
+        std::memcpy(st.piece(0), in, bytes);
+        HIPCHK(launch_import_rows(h->stream, reinterpret_cast<const double*>(st.piece(0)), h->o2n.p, h->nT, nv, d));
+        HIPCHK(hipStreamSynchronize(h->stream));
+        return AFX_OK;
     }
-    return AFX_OK;
-}
-int upload_aos(afx_rans* h, const double* in, double* d) {
-    std::vector<double> tmp((size_t)NV * h->nT);
-    for (int32_t i = 0; i < h->nT; ++i) {
-        int32_t o = h->c_new2old[i];
-        for (int k = 0; k < NV; ++k) tmp[(size_t)k * h->nT + i] = in[(size_t)NV * o + k];
-    }
-    HIPCHK(hipMemcpyAsync(d, tmp.data(), tmp.size() * 8, hipMemcpyHostToDevice, h->stream));
+    int rc = ensure_rows(h, nv);
+    if (rc) return rc;
+    if (pinned)
+        HIPCHK(st.to_device(h->stream, in, h->xrows.p, bytes));
+    else
+        HIPCHK(hipMemcpyAsync(h->xrows.p, in, bytes, hipMemcpyHostToDevice, h->stream));
+    HIPCHK(launch_import_rows(h->stream, h->xrows.p, h->o2n.p, h->nT, nv, d));
     HIPCHK(hipStreamSynchronize(h->stream));
-    return AFX_OK;
-}
-int download_cells(afx_rans* h, const double* d, double* out) {
-    std::vector<double> tmp(h->nT);
-    HIPCHK(hipMemcpyAsync(tmp.data(), d, tmp.size() * 8, hipMemcpyDeviceToHost, h->stream));
-    HIPCHK(hipStreamSynchronize(h->stream));
-    for (int32_t i = 0; i < h->nT; ++i) out[h->c_new2old[i]] = tmp[i];
     return AFX_OK;
 }
 
-int norm_of(afx_rans* h, const double* x, int64_t ld, int nrows, double* out) {
-    HIPCHK(launch_sumsq(h->stream, x, ld, ld, nrows, h->partial.p, h->nblk_red));
-    HIPCHK(launch_final_sum(h->stream, h->partial.p, h->nblk_red, h->sum1.p));
-    double s = 0;
-    HIPCHK(hipMemcpyAsync(&s, h->sum1.p, 8, hipMemcpyDeviceToHost, h->stream));
+// device SoA [NV][nT] -> reference AoS q(4*i+k)
+int download_aos(afx_rans* h, const double* d, double* out) { return fetch_rows(h, Staging(), d, NV, out); }
+int download_aos32(afx_rans* h, const float* d, double* out) { return fetch_rows(h, Staging(), d, NV, out); }
+int download_cells(afx_rans* h, const double* d, double* out) { return fetch_rows(h, Staging(), d, 1, out); }
+int upload_aos(afx_rans* h, const double* in, double* d) { return send_rows(h, Staging(), in, NV, d); }
+int upload_cells(afx_rans* h, const double* in, double* d) { return send_rows(h, Staging(), in, 1, d); }
+// the rho nu~ plane from the caller's vector, zero without one
+int upload_nu(afx_rans* h, const double* in, double* d) {
+    if (in) return upload_cells(h, in, d);
+    HIPCHK(hipMemsetAsync(d, 0, (size_t)h->nT * sizeof(double), h->stream));
     HIPCHK(hipStreamSynchronize(h->stream));
-    *out = std::sqrt(s);
     return AFX_OK;
 }
-int norm_of32(afx_rans* h, const float* x, int64_t ld, int nrows, double* out) {
+
+// enqueue |x|^2 (nrows rows of length ld) into *out, device or pinned memory
+int enqueue_sumsq(afx_rans* h, const double* x, int64_t ld, int nrows, double* out) {
+    HIPCHK(launch_sumsq(h->stream, x, ld, ld, nrows, h->partial.p, h->nblk_red));
+    HIPCHK(launch_final_sum(h->stream, h->partial.p, h->nblk_red, out));
+    return AFX_OK;
+}
+int enqueue_sumsq(afx_rans* h, const float* x, int64_t ld, int nrows, double* out) {
     HIPCHK(launch_sumsq_f32(h->stream, x, ld, ld, nrows, h->partial.p, h->nblk_red));
-    HIPCHK(launch_final_sum(h->stream, h->partial.p, h->nblk_red, h->sum1.p));
-    double s = 0;
-    HIPCHK(hipMemcpyAsync(&s, h->sum1.p, 8, hipMemcpyDeviceToHost, h->stream));
+    HIPCHK(launch_final_sum(h->stream, h->partial.p, h->nblk_red, out));
+    return AFX_OK;
+}
+// where a call's kernels leave its scalars: the staging buffer's pinned tail, or
+// sum1 and a copy when there is no pinned memory
+double* scalar_slot(afx_rans* h, const Staging& st) {
+    return st.status() == hipSuccess ? st.scalars() : h->sum1.p;
+}
+int read_scalars(afx_rans* h, const Staging& st, int n, double* v) {   // after the last wait when pinned
+    if (st.status() == hipSuccess) {
+        for (int k = 0; k < n; ++k) v[k] = st.scalars()[k];
+        return AFX_OK;
+    }
+    HIPCHK(hipMemcpyAsync(v, h->sum1.p, (size_t)n * 8, hipMemcpyDeviceToHost, h->stream));
     HIPCHK(hipStreamSynchronize(h->stream));
+    return AFX_OK;
+}
+int norm_of(afx_rans* h, const double* x, int64_t ld, int nrows, double* out) {
+    Staging st;
+    int rc = enqueue_sumsq(h, x, ld, nrows, scalar_slot(h, st));
+    if (rc) return rc;
+    HIPCHK(hipStreamSynchronize(h->stream));
+    double s = 0;
+    if ((rc = read_scalars(h, st, 1, &s))) return rc;
     *out = std::sqrt(s);
     return AFX_OK;
 }
@@ -479,11 +529,7 @@ int upload_operand(afx_rans* h, const double* x, const double* x_nu, const doubl
                                       : "rho nu~ rows only with the Spalart-Allmaras model");
     int rc = upload_aos(h, x, h->ktmp.p);
     if (rc || !x_nu) return rc;
-    std::vector<double> tmp(h->nT);
-    for (int32_t i = 0; i < h->nT; ++i) tmp[i] = x_nu[h->c_new2old[i]];
-    HIPCHK(hipMemcpyAsync(h->ktmp.p + 4 * (size_t)h->nT, tmp.data(), tmp.size() * 8, hipMemcpyHostToDevice, h->stream));
-    HIPCHK(hipStreamSynchronize(h->stream));
-    return AFX_OK;
+    return upload_cells(h, x_nu, h->ktmp.p + 4 * (size_t)h->nT);
 }
 int download_operand(afx_rans* h, double* y, double* y_nu) {
     int rc = download_aos(h, h->kw.p, y);
@@ -1021,6 +1067,7 @@ int create_impl(const Mesh& mesh_in, const afx_gas* g, const afx_opts* o, const 
         HIPCHK_C(h->lsq32.alloc(l32.size())); HIPCHK_C(h->lsq32.upload(l32, s));
         HIPCHK_C(hipStreamSynchronize(s));
     }
+    HIPCHK_C(h->o2n.alloc(nT)); HIPCHK_C(h->o2n.upload(h->c_old2new, s));
     HIPCHK_C(h->c0.alloc(nF)); HIPCHK_C(h->c0.upload(hc0, s));
     HIPCHK_C(h->c1.alloc(nF)); HIPCHK_C(h->c1.upload(hc1, s));
     HIPCHK_C(h->cface.alloc(hcface.size())); HIPCHK_C(h->cface.upload(hcface, s));
@@ -1044,13 +1091,8 @@ int create_impl(const Mesh& mesh_in, const afx_gas* g, const afx_opts* o, const 
     HIPCHK_C(h->flux.alloc((size_t)NV * nF));
     HIPCHK_C(h->flux32.alloc((size_t)NV * nF));
     // ghost limiters are 1 and ghost gradients 0 (solver.h:466-469,519,540)
-    {
-        std::vector<double> ones(nq, 1.0);
-        std::vector<float> ones32(nq, 1.0f);
-        HIPCHK_C(h->lim.upload(ones, s));
-        HIPCHK_C(h->lim32.upload(ones32, s));
-        HIPCHK_C(hipStreamSynchronize(s));
-    }
+    HIPCHK_C(launch_fill(s, h->lim.p, 1.0, (int64_t)nq));
+    HIPCHK_C(launch_fill(s, h->lim32.p, 1.0f, (int64_t)nq));
     // tile tables (only usable when the cell order is the tile order)
     if (opts.renumber) {
         const TileLayout& tl = h->tl;
@@ -1125,7 +1167,7 @@ int create_impl(const Mesh& mesh_in, const afx_gas* g, const afx_opts* o, const 
     }
     h->nblk_red = 1024;
     HIPCHK_C(h->partial.alloc(h->nblk_red));
-    HIPCHK_C(h->sum1.alloc(1));
+    HIPCHK_C(h->sum1.alloc(2));
     HIPCHK_C(h->uni64.alloc(NV_MAX));
     HIPCHK_C(h->uni32.alloc(NV_MAX));
     HIPCHK_C(hipStreamSynchronize(s));
@@ -1344,28 +1386,38 @@ int afx_rans_residual(afx_rans* h, int32_t precision, double* R, double* norm2) 
     if (rc) return rc;
     if (precision != AFX_FP64 && precision != AFX_FP32) return fail(AFX_EARG, "precision must be AFX_FP64 or AFX_FP32");
     if ((rc = enqueue_residual(h, precision))) return rc;
-    if (precision == AFX_FP64) {
-        if (R && (rc = download_aos(h, h->R.p, R))) return rc;
-        if (norm2 && (rc = norm_of(h, h->R.p, h->nT, h->nv, norm2))) return rc;
-    } else if (h->r32_aos) {
-        if (R) {
-            std::vector<float> tmp((size_t)NV * h->nT);
-            HIPCHK(hipMemcpyAsync(tmp.data(), h->R32v.p, tmp.size() * 4, hipMemcpyDeviceToHost, h->stream));
-            HIPCHK(hipStreamSynchronize(h->stream));
-            for (int32_t i = 0; i < h->nT; ++i)
-                for (int k = 0; k < NV; ++k) R[(size_t)NV * h->c_new2old[i] + k] = (double)tmp[(size_t)NV * i + k];
-        }
-        if (norm2) {
-            if ((rc = norm_of32(h, reinterpret_cast<const float*>(h->R32v.p), (int64_t)NV * h->nT, 1, norm2))) return rc;
-            if (h->sa()) {
-                double n5 = 0;
-                if ((rc = norm_of32(h, h->R32n.p, h->nT, 1, &n5))) return rc;
-                *norm2 = std::sqrt(*norm2 * *norm2 + n5 * n5);
+    if (!R && !norm2) return AFX_OK;
+    // norm, then R, and one wait for both
+    Staging st;
+    double* sums = scalar_slot(h, st);
+    int parts = 1;
+    if (norm2) {
+        if (precision == AFX_FP64) {
+            rc = enqueue_sumsq(h, h->R.p, h->nT, h->nv, sums);
+        } else if (h->r32_aos) {
+            rc = enqueue_sumsq(h, reinterpret_cast<const float*>(h->R32v.p), (int64_t)NV * h->nT, 1, sums);
+            if (!rc && h->sa()) {
+                rc = enqueue_sumsq(h, h->R32n.p, h->nT, 1, sums + 1);
+                parts = 2;
             }
+        } else {
+            rc = enqueue_sumsq(h, h->R32.p, h->nT, NV, sums);
         }
+        if (rc) return rc;
+    }
+    if (R) {
+        if (precision == AFX_FP64) rc = fetch_rows(h, st, h->R.p, NV, R);
+        else if (h->r32_aos) rc = fetch_rows(h, st, h->R32v.p, NV, R);
+        else rc = fetch_rows(h, st, h->R32.p, NV, R);
+        if (rc) return rc;
     } else {
-        if (R && (rc = download_aos32(h, h->R32.p, R))) return rc;
-        if (norm2 && (rc = norm_of32(h, h->R32.p, h->nT, NV, norm2))) return rc;
+        HIPCHK(hipStreamSynchronize(h->stream));
+    }
+    if (norm2) {
+        double v[2] = {0, 0};
+        if ((rc = read_scalars(h, st, parts, v))) return rc;
+        const double n0 = std::sqrt(v[0]), n1 = std::sqrt(v[1]);
+        *norm2 = parts == 1 ? n0 : std::sqrt(n0 * n0 + n1 * n1);
     }
     return AFX_OK;
 }
@@ -1902,12 +1954,8 @@ int afx_rans_set_nu(afx_rans* h, const double* nu) {
     if (rc) return rc;
     if (!h->sa()) return fail(AFX_ESTATE, "the solver was not created with the Spalart-Allmaras model");
     if (!nu) return fail(AFX_EARG, "null rho nu~ vector");
-    std::vector<double> tmp(h->nT);
-    for (int32_t i = 0; i < h->nT; ++i) tmp[i] = nu[h->c_new2old[i]];
-    HIPCHK(hipMemcpyAsync(h->q.p + (size_t)4 * h->nT, tmp.data(), tmp.size() * 8, hipMemcpyHostToDevice, h->stream));
-    HIPCHK(hipStreamSynchronize(h->stream));
     h->q32_valid = false;
-    return AFX_OK;
+    return upload_cells(h, nu, h->q.p + (size_t)4 * h->nT);
 }
 
 int afx_rans_get_nu(afx_rans* h, double* nu) {
@@ -1925,11 +1973,7 @@ int afx_rans_nu_residual(afx_rans* h, double* Rnu) {
     if (!Rnu) return fail(AFX_EARG, "null residual vector");
     if (h->last_precision == AFX_FP64) return download_cells(h, h->R.p + (size_t)4 * h->nT, Rnu);
     if (h->last_precision != AFX_FP32) return fail(AFX_ESTATE, "no residual has been evaluated");
-    std::vector<float> tmp(h->nT);
-    HIPCHK(hipMemcpyAsync(tmp.data(), h->R32n.p, tmp.size() * 4, hipMemcpyDeviceToHost, h->stream));
-    HIPCHK(hipStreamSynchronize(h->stream));
-    for (int32_t i = 0; i < h->nT; ++i) Rnu[h->c_new2old[i]] = (double)tmp[i];
-    return AFX_OK;
+    return fetch_rows(h, Staging(), h->R32n.p, 1, Rnu);
 }
 
 int afx_rans_counts(afx_rans* h, int64_t c[5]) {
@@ -2090,14 +2134,7 @@ int afx_rans_adjoint_nu(afx_rans* h, const double* w, const double* w_nu, double
         return fail(AFX_EARG, "rho nu~ seed / output only with the Spalart-Allmaras model");
     if ((rc = adjoint_check(h, true))) return rc;
     if ((rc = upload_aos(h, w, h->a_w.p))) return rc;
-    if (h->sa()) {
-        std::vector<double> tmp(h->nT, 0.0);
-        if (w_nu)
-            for (int32_t i = 0; i < h->nT; ++i) tmp[i] = w_nu[h->c_new2old[i]];
-        HIPCHK(hipMemcpyAsync(h->a_w.p + 4 * (size_t)h->nT, tmp.data(), tmp.size() * 8, hipMemcpyHostToDevice,
-                              h->stream));
-        HIPCHK(hipStreamSynchronize(h->stream));
-    }
+    if (h->sa() && (rc = upload_nu(h, w_nu, h->a_w.p + 4 * (size_t)h->nT))) return rc;
     // wall/slip ghosts as fillRhoRHS sees them (they enter no flux, but the
     // state is then the one the residual reads)
     HIPCHK(launch_set_walls<double>(h->stream, h->w_owner.p, h->w_ghost.p, h->n_walls, h->q.p, h->nT, h->nv));
@@ -2467,13 +2504,7 @@ int afx_rans_tangent(afx_rans* h, const double* v, const double* v_nu, double* j
     const int nv = h->nv;
     const int64_t nT = h->nT;
     if ((rc = upload_aos(h, v, h->tg_v.p))) return rc;
-    if (nv == 5) {
-        std::vector<double> tmp(h->nT, 0.0);
-        if (v_nu)
-            for (int32_t i = 0; i < h->nT; ++i) tmp[i] = v_nu[h->c_new2old[i]];
-        HIPCHK(hipMemcpyAsync(h->tg_v.p + 4 * nT, tmp.data(), tmp.size() * 8, hipMemcpyHostToDevice, s));
-        HIPCHK(hipStreamSynchronize(s));
-    }
+    if (nv == 5 && (rc = upload_nu(h, v_nu, h->tg_v.p + 4 * nT))) return rc;
     if ((rc = enqueue_tangent(h))) return rc;
     if ((rc = download_aos(h, h->tg_out.p, jv))) return rc;
     if (jv_nu && (rc = download_cells(h, h->tg_out.p + 4 * nT, jv_nu))) return rc;

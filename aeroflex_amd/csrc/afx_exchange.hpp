@@ -1,0 +1,60 @@
+// Vectors crossing the C ABI: the reference's cell order and AoS layout on the
+// host side, planes in the device's cell order on the GPU.
+//
+// The permutation runs on the device.  Between the device and the caller's
+// pageable memory the bytes go through pinned staging buffers: vectors of at
+// most kDirectBytes in one go, read or written over PCIe by the layout kernel
+// itself; larger ones in kSlotBytes pieces copied by a few host threads while
+// the next pieces are in flight.
+#pragma once
+#include <cstddef>
+#include <cstdint>
+#include <hip/hip_runtime.h>
+
+namespace afx {
+
+constexpr size_t kSlotBytes = size_t(1) << 20;   // one piece of a large transfer
+constexpr int kSlots = 8;                         // pieces in flight
+constexpr size_t kDirectBytes = 4 * kSlotBytes;   // up to here the kernels access pinned memory themselves
+constexpr int kScalars = 64;                      // doubles for norms and flags behind the pieces
+
+// One pinned staging buffer with its events, on the device that was current
+// when it was taken.  Taken from a process-wide pool and given back by the
+// destructor; a Staging belongs to one call of one thread.
+class Staging {
+public:
+    Staging();
+    ~Staging();
+    Staging(const Staging&) = delete;
+    Staging& operator=(const Staging&) = delete;
+    hipError_t status() const { return err_; }
+    char* piece(int k) const;            // host = device address (unified addressing)
+    double* scalars() const;
+    // caller memory <-> device memory, in pieces; returns once done
+    hipError_t to_device(hipStream_t s, const void* host, void* dev, size_t bytes) const;
+    hipError_t to_host(hipStream_t s, const void* dev, void* host, size_t bytes) const;
+
+private:
+    hipError_t pieces(hipStream_t s, char* host, char* dev, size_t bytes, bool up) const;
+    struct Buf;
+    friend struct StagingPool;
+    Buf* b_ = nullptr;
+    hipError_t err_ = hipSuccess;
+};
+// The pool keeps buffers while any solver handle lives: every handle holds one
+// reference, and the last one to go frees the idle buffers.
+void staging_retain();
+void staging_release();
+
+// device planes <-> rows of nv values in reference order (nv 4: q(4*i+k); 1: one
+// value per cell); old2new: device cell of each reference cell
+hipError_t launch_import_rows(hipStream_t s, const double* rows, const int32_t* old2new, int32_t nT, int nv,
+                              double* planes);
+hipError_t launch_export_rows(hipStream_t s, const double* planes, const int32_t* old2new, int32_t nT, int nv,
+                              double* rows);
+hipError_t launch_export_rows(hipStream_t s, const float* planes, const int32_t* old2new, int32_t nT, int nv,
+                              double* rows);
+hipError_t launch_export_rows(hipStream_t s, const float4* cells, const int32_t* old2new, int32_t nT, int nv,
+                              double* rows);   // nv 4
+
+}  // namespace afx

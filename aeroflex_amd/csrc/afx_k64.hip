@@ -66,6 +66,20 @@ hipError_t launch_copy(hipStream_t s, const double* src, double* dst, int64_t n)
     return hipGetLastError();
 }
 
+template <typename T>
+__global__ void __launch_bounds__(kBlock) k_fill(T* __restrict__ x, T v, int64_t n) {
+    const int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
+    if (i < n) x[i] = v;
+}
+template <typename T>
+hipError_t launch_fill(hipStream_t s, T* x, T v, int64_t n) {
+    if (n <= 0) return hipSuccess;
+    hipLaunchKernelGGL(k_fill<T>, dim3(nblocks(n)), dim3(kBlock), 0, s, x, v, n);
+    return hipGetLastError();
+}
+template hipError_t launch_fill<double>(hipStream_t, double*, double, int64_t);
+template hipError_t launch_fill<float>(hipStream_t, float*, float, int64_t);
+
 // explicitSolver::solve stage update (solver.h:818-821)
 __global__ void __launch_bounds__(kBlock) k_rk_update(const double* __restrict__ q, const double* __restrict__ qW,
                                                       const double* __restrict__ dt, double ai, double relax, int32_t nC,

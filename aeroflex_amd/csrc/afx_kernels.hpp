@@ -201,6 +201,8 @@ hipError_t launch_gather(hipStream_t s, CellsT<T> C, const T* flux, int32_t nF, 
 hipError_t launch_sumsq(hipStream_t s, const double* x, int64_t n, int64_t ld, int nv, double* partial, int nblk);
 hipError_t launch_sumsq_f32(hipStream_t s, const float* x, int64_t n, int64_t ld, int nv, double* partial, int nblk);
 hipError_t launch_final_sum(hipStream_t s, const double* partial, int nblk, double* out);
+template <typename T>
+hipError_t launch_fill(hipStream_t s, T* x, T v, int64_t n);
 hipError_t launch_copy(hipStream_t s, const double* src, double* dst, int64_t n);
 hipError_t launch_rk_update(hipStream_t s, const double* q, const double* qW, const double* dt, double ai, double relax,
                             int32_t nC, int32_t nT, int nv, double* qk);

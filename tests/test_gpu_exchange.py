@@ -1,0 +1,67 @@
+"""Vectors crossing the C ABI (afx_exchange.hip): the device permutation, the
+direct and the pieced transfer on both sides of their limits, and calls from
+several threads at once."""
+import threading
+
+import numpy as np
+import pytest
+
+pytestmark = pytest.mark.gpu
+
+
+def make(ni, nj, renumber, model="inviscid"):
+    from aeroflex_amd import rans
+    m = rans.Mesh.naca_ogrid(ni, nj, r_far=20.0, first_h=2e-3)
+    s = rans.Solver(m, viscosity_model=model, renumber=renumber)
+    far = rans.BoundaryVariables(mach=0.5, angle=0.03)
+    s.set_bcs({"farfield": rans.BoundaryCondition("farfield", far), "wall": rans.BoundaryCondition("slip-wall")})
+    return s
+
+
+# 2 ni nj cells in all: less than a block of the layout kernels, one more and
+# one less than full blocks, the last direct vector (131 072 cells, 4 MB), the
+# first pieced one, a last piece of a few rows, several pieces per worker
+@pytest.mark.parametrize("ni,nj", [(8, 3), (8, 16), (43, 3), (64, 1023), (64, 1024), (64, 1025), (67, 1024),
+                                   (128, 2050)])
+def test_rows_keep_their_cells(ni, nj):
+    s, f = make(ni, nj, True), make(ni, nj, False)   # f: file order on the device
+    rng = np.random.default_rng(ni * nj)
+    s.init()
+    q = s.get_q().reshape(-1, 4)
+    q[:] = q[0] * (1.0 + 0.01 * rng.standard_normal(q.shape))
+    s.set_q(q)
+    f.set_q(q.ravel())
+    assert np.array_equal(s.get_q(), q.ravel())
+    assert np.array_equal(f.get_q(), q.ravel())
+    for a, b in ((s.calc_dt(), f.calc_dt()), (s.fillRhoRHS()[0], f.fillRhoRHS()[0])):
+        # the same operations in the same order per cell: the same bits
+        assert np.array_equal(a[:len(a) - 8 * ni], b[:len(b) - 8 * ni])
+    n64, n32 = s.fillRhoRHS(0)[1], s.fillRhoRHS(1)[1]
+    R64, R32 = s.fillRhoRHS(0)[0], s.fillRhoRHS(1)[0]
+    # norms in another summation order: n eps, below 1e-12 at 1e6 entries
+    assert abs(np.linalg.norm(R64) - n64) <= 1e-12 * n64
+    assert abs(np.linalg.norm(R32) - n32) <= 1e-12 * n32
+    # rows out of place differ by about sqrt(2) |R|; the FP32 form itself by
+    # 6e-8 sum |flux len| / |R|, below 1e-2 even on the cells of many chords
+    # that the coarsest of these grids have
+    assert np.linalg.norm(R32 - R64) <= 0.1 * np.linalg.norm(R64)
+
+
+def test_threads_do_not_mix_their_vectors():
+    solvers = [make(64, 400 + 300 * k, True, "spalart-allmaras") for k in range(4)]
+    bad = []
+
+    def work(k):
+        s, rng = solvers[k], np.random.default_rng(k)
+        for _ in range(6):
+            q, nu = rng.standard_normal(4 * s.n_cells), rng.standard_normal(s.n_cells)
+            s.set_q(q)
+            s.set_nu(nu)
+            if not (np.array_equal(s.get_q(), q) and np.array_equal(s.get_nu(), nu)):
+                bad.append(k)
+    team = [threading.Thread(target=work, args=(k,)) for k in range(4)]
+    for t in team:
+        t.start()
+    for t in team:
+        t.join()
+    assert not bad
