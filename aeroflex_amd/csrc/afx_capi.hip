@@ -145,9 +145,9 @@ struct afx_rans {
     // implicit step: Jacobian blocks, diagonal blocks and their inverses,
     // GMRES work space and state (kg: the GmDev arrays, kflags its flags)
     DBuf<double> Jf, Dblk, Dinv, kV, kw, kz, kr, ktmp, kpart, kg;
-    DBuf<double> ellE, ellD;   // ELL copy of the matrix for the product (launch_assemble_diag)
+    DBuf<double> ellE, ellD;   // block Jacobi: ELL copy of the matrix for the product (launch_assemble_diag)
     DBuf<int32_t> ellN;
-    DBuf<double> dilE, dilD;   // colour-ordered copy for the DILU sweeps (launch_dilu_setup)
+    DBuf<double> dilE, dilT, dilD;   // DILU: colour-ordered copy for sweeps and product (launch_dilu_setup)
     DBuf<int32_t> dilN;
     DBuf<int> kbad, kflags;
     int32_t gm_restart = 30, gm_maxit = 500;
@@ -161,13 +161,18 @@ struct afx_rans {
     int precond = 1;
     DBuf<uint8_t> colour;
     DBuf<int32_t> col_cells, col_pos;   // real cells in colour order, and each cell's position in it
-    DBuf<double> kdil;                   // the DILU sweeps' work vector, by colour position (nv planes of nC)
     std::vector<int32_t> col_off;
     DBuf<double> Dti;
-    GmDev gm_dev() const {
+    ColourOrder colours() const {
+        return ColourOrder{colour.p, col_cells.p, col_pos.p, col_off.data(), (int)col_off.size() - 1};
+    }
+    ColourMatrix colour_matrix() const { return ColourMatrix{dilE.p, dilN.p, dilT.p, dilD.p}; }
+    GmDev gm_dev(int* seen) const {
         const int m = gm_restart;
         double* b = kg.p;
         GmDev G;
+        G.seen = seen;
+        G.sums = kpart.p;
         G.hdr = b;
         G.H = b + 8;
         G.cs = G.H + (size_t)(m + 1) * m;
@@ -191,7 +196,6 @@ struct afx_rans {
     DBuf<Dual1> tg_geo, tg_area, tg_lsq, tg_xc, tg_yc, tg_wd, tg_q, tg_R;
     DBuf<double> tg_v, tg_out;
     int64_t lin_iters = 0;
-    int kblk = 0;
     std::vector<int32_t> t_lg;   // device cell of each local cell (unflagged)
     bool tile64_ok = false, tile32_ok = false;
 
@@ -539,32 +543,39 @@ int download_operand(afx_rans* h, double* y, double* y_nu) {
 
 int ensure_implicit(afx_rans* h) {
     if (h->mf && !h->mfFb.p) HIPCHK(h->mfFb.alloc((size_t)4 * h->nF));
+    if (!h->mf && h->precond == 0 && !h->ellE.p) {   // the product in cell order
+        const size_t nn = (size_t)h->nv * h->nv;
+        HIPCHK(h->ellD.alloc(nn * h->nC));
+        HIPCHK(h->ellN.alloc(4 * (size_t)h->nC));
+        HIPCHK(h->ellE.alloc(4 * nn * h->nC));
+    }
+    if (!h->mf && h->precond == 1 && !h->dilE.p) {   // sweeps and product in colour order
+        const size_t nn = (size_t)h->nv * h->nv;
+        HIPCHK(h->Dti.alloc(nn * h->nC));
+        HIPCHK(h->dilD.alloc(nn * h->nC));
+        HIPCHK(h->dilT.alloc(nn * h->nC));
+        HIPCHK(h->dilN.alloc(4 * (size_t)h->nC));
+        HIPCHK(h->dilE.alloc(4 * nn * h->nC));
+    }
     if (h->Jf.p) return AFX_OK;
     // blocks of nv x nv (five with the Spalart-Allmaras model), vectors of nv planes
     const int nv = h->nv;
     const size_t nn = (size_t)nv * nv;
     const size_t n = (size_t)nv * h->nT;
     const int m = h->gm_restart;
-    h->kblk = 2048;   // at most eight waves per SIMD in the Gram-Schmidt passes
     HIPCHK(h->Jf.alloc(2 * nn * h->nF));
     HIPCHK(h->Dblk.alloc(nn * h->nC));
     HIPCHK(h->Dinv.alloc(nn * h->nC));
-    HIPCHK(h->kV.alloc((size_t)(m + 1) * n));
+    // either order of the process: nv planes of nC, or one row of nv nT
+    HIPCHK(h->kV.alloc(std::max(basis_doubles(h->nC, nv, m), basis_doubles(n, 1, m))));
     HIPCHK(h->kw.alloc(n));
     HIPCHK(h->kz.alloc(n));
     HIPCHK(h->kr.alloc(n));
     HIPCHK(h->ktmp.alloc(n));
-    HIPCHK(h->kpart.alloc((size_t)(m + 2) * h->kblk));
+    HIPCHK(h->kpart.alloc(kGsSums));
     HIPCHK(h->kg.alloc(afx_rans::gm_doubles(m)));
     HIPCHK(h->kflags.alloc(8));
     HIPCHK(h->kbad.alloc(1));
-    HIPCHK(h->Dti.alloc(nn * h->nC));
-    HIPCHK(h->ellE.alloc(4 * nn * h->nC));
-    HIPCHK(h->ellD.alloc(nn * h->nC));
-    HIPCHK(h->ellN.alloc(4 * (size_t)h->nC));
-    HIPCHK(h->dilE.alloc(4 * nn * h->nC));
-    HIPCHK(h->dilD.alloc(nn * h->nC));
-    HIPCHK(h->dilN.alloc(4 * (size_t)h->nC));
     HIPCHK(hipMemsetAsync(h->Jf.p, 0, 2 * nn * h->nF * 8, h->stream));
     HIPCHK(hipMemsetAsync(h->kflags.p, 0, 8 * sizeof(int), h->stream));
     // greedy colouring of the real cells in device order over their
@@ -606,104 +617,131 @@ int ensure_implicit(afx_rans* h) {
         for (int32_t p = 0; p < nC; ++p) where[cells[p]] = p;
         HIPCHK(h->col_pos.alloc(std::max<size_t>(nC, 1)));
         HIPCHK(h->col_pos.upload(where, h->stream));
-        HIPCHK(h->kdil.alloc(std::max<size_t>((size_t)nv * nC, 1)));
         HIPCHK(hipStreamSynchronize(h->stream));
     }
     return AFX_OK;
 }
 
 // Right-preconditioned restarted GMRES (classical Gram-Schmidt applied twice)
-// for LHS x = b; b and x are device vectors of nv planes of nT.  The Arnoldi
-// state stays on the device (GmDev): the steps of a restart cycle are
-// enqueued in chunks, the kernels of a step do nothing once the iteration
-// has converged or broken down, and between chunks the host reads the flags
-// and ends the cycle early once the Arnoldi process is inactive (the steps
-// it skips would do nothing, so the result is the same as enqueueing all m).
-// The first chunk has as many steps as the last converged cycle took, later
-// ones four.  Returns AFX_OK and *converged, or a negative error code.
-int gmres(afx_rans* h, const double* b, double* x, bool* converged) {
-    const int64_t n = (int64_t)h->nv * h->nT;
+// for LHS dq = b; b and dq are device vectors of nv planes of nT, and
+// q += relax dq once converged.  The Arnoldi state stays on the device
+// (GmDev): the steps of a restart cycle are enqueued in chunks, the kernels of
+// a step do nothing once the iteration has converged or broken down, and
+// between chunks the host reads the flags and ends the cycle early once the
+// Arnoldi process is inactive (the steps it skips would do nothing, so the
+// result is the same as enqueueing all m).  The first chunk has as many steps
+// as the last converged cycle took, later ones four.
+// With DILU every vector of the process is held in the colour order of the
+// sweeps (nv planes of nC, real cells only: ghost rows are identity rows with
+// zero right-hand side), so the sweeps, the product and the basis read
+// consecutive addresses and share one copy of the matrix; b enters and dq
+// leaves through the order once per cycle.  Block Jacobi and the matrix-free
+// operator (no preconditioner, solver.h:868) work in cell order.
+// Returns AFX_OK and *converged, or a negative error code.
+int gmres(afx_rans* h, const double* b, double* dq, double relax, bool* converged) {
+    const bool colour = !h->mf && h->precond == 1;
+    const int nv = h->nv;
+    const int64_t n = (int64_t)nv * (colour ? h->nC : h->nT);
     const int m = h->gm_restart;
-    // Gram-Schmidt blocks: about two entries per thread, at most kblk
-    const int nb = (int)std::min<int64_t>(h->kblk, std::max<int64_t>(8, (n + 511) / 512));
     hipStream_t s = h->stream;
     double* V = h->kV.p;
-    double* part = h->kpart.p;
-    const GmDev G = h->gm_dev();
+    Staging st;
+    const bool pinned = st.status() == hipSuccess;
+    volatile int* seen = pinned ? reinterpret_cast<volatile int*>(st.scalars()) : nullptr;
+    const GmDev G = h->gm_dev(const_cast<int*>(seen));
+    const ColourOrder O = h->colours();
+    const ColourMatrix M = h->colour_matrix();
     const int* active = G.flags;
     *converged = false;
-    // the operator and the right preconditioner: the assembled matrix with
-    // block Jacobi or block DILU, or the matrix-free product with none
-    // (solver.h:868)
-    auto apply = [&](const double* in, double* out, const int* act) -> hipError_t {
-        if (h->mf)
-            return launch_mf_apply(s, h->cells64(), h->faces64(), h->q.p, h->dt.p, h->mfFb.p, h->gas64(),
-                                   h->opts.viscosity, in, out, act);
-        return launch_lhs_apply(s, h->nv, h->nC, h->nT, h->ellD.p, h->ellE.p, h->ellN.p, in, out, act);
+    double* x = colour ? h->ktmp.p : dq;   // the solution in the order of the process
+    // column j of the basis from in, w = A M^-1 v_j, and the step
+    auto advance = [&](const double* in, int j, bool show) -> hipError_t {
+        double* vj = h->ktmp.p;   // cell order: column j of the basis by itself
+        int nblk = 0;
+        hipError_t e;
+        if (colour) {
+            e = launch_dilu_apply_next(s, nv, O, M, G, in, V, j, h->kz.p);
+            if (e == hipSuccess)
+                e = launch_colour_apply_dots(s, nv, O, M, G, h->kz.p, h->kw.p, V, j + 1, &nblk);
+        } else {
+            e = launch_next_vector(s, G, in, V, j, vj, n);
+            if (e == hipSuccess && h->mf)
+                e = launch_mf_apply(s, h->cells64(), h->faces64(), h->q.p, h->dt.p, h->mfFb.p, h->gas64(),
+                                    h->opts.viscosity, vj, h->kw.p, active);
+            if (e == hipSuccess && !h->mf)
+                e = launch_block_jacobi(s, nv, h->nC, h->nT, h->Dinv.p, vj, h->kz.p, active);
+            if (e == hipSuccess && !h->mf)
+                e = launch_lhs_apply(s, nv, h->nC, h->nT, h->ellD.p, h->ellE.p, h->ellN.p, h->kz.p, h->kw.p, active);
+            if (e == hipSuccess) e = launch_gs_dots(s, G, V, n, j + 1, h->kw.p, &nblk);
+        }
+        return e == hipSuccess ? launch_gm_step(s, G, colour ? &O : nullptr, nv, V, n, j, show, h->kw.p, nblk) : e;
     };
-    auto precond = [&](const double* in, double* out, const double** res, const int* act) -> hipError_t {
-        if (h->mf) { *res = in; return hipSuccess; }
-        *res = out;
-        if (h->precond == 1)
-            return launch_dilu_apply(s, h->nv, h->nC, h->nT, h->col_cells.p, h->col_pos.p, h->col_off.data(),
-                                     (int)h->col_off.size() - 1, h->dilE.p, h->dilN.p, h->dilD.p, in, out, h->kdil.p,
-                                     act);
-        return launch_block_jacobi(s, h->nv, h->nC, h->nT, h->Dinv.p, in, out, act);
-    };
-    // |r|^2 of the cycle's start vector into hdr[3], then the cycle's set-up
-    auto begin = [&](int first) -> hipError_t {
-        hipError_t e = launch_gs_pass(s, nullptr, n, 0, nullptr, h->kr.p, n, false, part, nb, nullptr);
-        if (e == hipSuccess) e = launch_gm_reduce(s, part, nb, 0, 1, G.hdr + 3, nullptr);
-        if (e == hipSuccess) e = launch_gm_begin(s, G, first);
-        if (e == hipSuccess) e = launch_scale_dev(s, G.hdr + 2, h->kr.p, V, n, active);
-        return e;
-    };
-    const double* pz = nullptr;
-    HIPCHK(hipMemsetAsync(x, 0, n * 8, s));
-    HIPCHK(launch_copy(s, b, h->kr.p, n));
-    HIPCHK(begin(1));
+    // the flags after everything enqueued so far
     int flags[4] = {0, 0, 0, 0};
-    int total_before = 0;
-    while (true) {
+    auto read_flags = [&]() -> int {
+        if (!pinned) HIPCHK(hipMemcpyAsync(flags, G.flags, sizeof(flags), hipMemcpyDeviceToHost, s));
+        HIPCHK(hipStreamSynchronize(s));
+        if (pinned)
+            for (int k = 0; k < 4; ++k) flags[k] = seen[k];
+        return AFX_OK;
+    };
+    if (colour) {
+        HIPCHK(launch_to_colour(s, nv, h->nT, O, b, nullptr, h->kr.p));
+    } else {
+        HIPCHK(hipMemsetAsync(x, 0, n * 8, s));
+        HIPCHK(launch_copy(s, b, h->kr.p, n));
+    }
+    HIPCHK(launch_gm_begin(s, G, h->kr.p, n, 1));
+    int rc, total_before = 0;
+    for (int cycle = 0;; ++cycle) {
         int chunk = std::max(1, std::min<int>(h->gm_chunk, m));
+        bool over = false;   // the flags of the finished cycle are known
         for (int j = 0; j < m; ++j) {
             if (j == chunk) {   // a chunk is enqueued: is the Arnoldi process still active?
-                HIPCHK(hipMemcpyAsync(flags, G.flags, sizeof(flags), hipMemcpyDeviceToHost, s));
-                HIPCHK(hipStreamSynchronize(s));
-                if (!flags[0]) break;
+                if ((rc = read_flags())) return rc;
+                if ((over = !flags[0])) break;
                 chunk += 4;
             }
-            double* vj = V + (size_t)j * n;
-            HIPCHK(precond(vj, h->kz.p, &pz, active));
-            HIPCHK(apply(pz, h->kw.p, active));
-            HIPCHK(launch_gs_pass(s, V, n, j + 1, nullptr, h->kw.p, n, true, part, nb, active));
-            HIPCHK(launch_gm_reduce(s, part, nb, 0, j + 1, G.h1, active));
-            HIPCHK(launch_gs_pass(s, V, n, j + 1, G.h1, h->kw.p, n, true, part, nb, active));
-            HIPCHK(launch_gm_reduce(s, part, nb, 0, j + 1, G.h2, active));
-            HIPCHK(launch_gs_pass(s, V, n, j + 1, G.h2, h->kw.p, n, false, part, nb, active));
-            HIPCHK(launch_gm_reduce(s, part, nb, j + 1, 1, G.hdr + 3, active));
-            HIPCHK(launch_gm_step(s, G, j));
-            if (j + 1 < m) HIPCHK(launch_scale_dev(s, G.hdr + 2, h->kw.p, V + (size_t)(j + 1) * n, n, active));
+            HIPCHK(advance(j == 0 ? h->kr.p : h->kw.p, j, j + 1 == chunk || j + 1 == m));
         }
         // y = H^-1 g, x += M^-1 (V y)
         HIPCHK(launch_gm_solve(s, G));
-        HIPCHK(launch_lincomb_dev(s, V, n, G.flags + 3, G.y, h->ktmp.p, n));
-        HIPCHK(precond(h->ktmp.p, h->kz.p, &pz, nullptr));
-        HIPCHK(launch_axpy(s, 1.0, pz, x, n));
-        HIPCHK(hipMemcpyAsync(flags, G.flags, sizeof(flags), hipMemcpyDeviceToHost, s));
-        HIPCHK(hipStreamSynchronize(s));
+        if (colour) {
+            HIPCHK(launch_dilu_apply_sum(s, nv, O, M, G, V, h->kz.p));
+            HIPCHK(launch_colour_update(s, nv, h->nT, O, cycle == 0, relax, h->kz.p, x, dq, h->q.p, G.flags + 1));
+        } else {
+            HIPCHK(launch_lincomb(s, G, V, h->ktmp.p, n));
+            const double* z = h->ktmp.p;
+            if (!h->mf) {
+                HIPCHK(launch_block_jacobi(s, nv, h->nC, h->nT, h->Dinv.p, h->ktmp.p, h->kz.p));
+                z = h->kz.p;
+            }
+            HIPCHK(launch_axpy(s, 1.0, z, x, n));
+        }
+        if (!over && (rc = read_flags())) return rc;
         h->lin_iters += flags[2] - total_before;
         total_before = flags[2];
         if (flags[1]) {
             h->gm_chunk = std::max(1, flags[3]);
             *converged = true;
+            if (!colour) HIPCHK(launch_axpy(s, relax, dq, h->q.p, n));
             return AFX_OK;
         }
         if (flags[2] >= h->gm_maxit) return AFX_OK;
-        // restart from the true residual
-        HIPCHK(apply(x, h->kw.p, nullptr));
-        HIPCHK(launch_sub(s, b, h->kw.p, h->kr.p, n));
-        HIPCHK(begin(0));   // converged here: the next cycle's kernels do nothing
+        // restart from the true residual; converged here: the next cycle's
+        // kernels do nothing
+        if (colour) {
+            HIPCHK(launch_colour_apply(s, nv, O, M, x, h->kw.p));
+            HIPCHK(launch_to_colour(s, nv, h->nT, O, b, h->kw.p, h->kr.p));
+        } else {
+            if (h->mf)
+                HIPCHK(launch_mf_apply(s, h->cells64(), h->faces64(), h->q.p, h->dt.p, h->mfFb.p, h->gas64(),
+                                       h->opts.viscosity, x, h->kw.p));
+            else
+                HIPCHK(launch_lhs_apply(s, nv, h->nC, h->nT, h->ellD.p, h->ellE.p, h->ellN.p, x, h->kw.p));
+            HIPCHK(launch_sub(s, b, h->kw.p, h->kr.p, n));
+        }
+        HIPCHK(launch_gm_begin(s, G, h->kr.p, n, 0));
     }
 }
 
@@ -1645,11 +1683,10 @@ int afx_rans_implicit_fill(afx_rans* h) {
     }
     HIPCHK(hipMemsetAsync(h->kbad.p, 0, sizeof(int), s));
     HIPCHK(launch_assemble_diag(s, h->nv, h->cells64(), h->faces64(), h->dt.p, h->Jf.p, src, h->Dblk.p, h->Dinv.p,
-                                h->ellE.p, h->ellD.p, h->ellN.p, h->kbad.p));
+                                h->precond == 0 ? h->ellE.p : nullptr, h->ellD.p, h->ellN.p, h->kbad.p));
     if (h->precond == 1)
-        HIPCHK(launch_dilu_setup(s, h->nv, h->cells64(), h->faces64(), h->colour.p, h->col_cells.p, h->col_pos.p,
-                                 h->col_off.data(), (int)h->col_off.size() - 1, h->Dblk.p, h->Jf.p, h->Dti.p,
-                                 h->dilE.p, h->dilN.p, h->dilD.p, h->kbad.p));
+        HIPCHK(launch_dilu_setup(s, h->nv, h->cells64(), h->faces64(), h->colours(), h->Dblk.p, h->Jf.p, h->Dti.p,
+                                 h->colour_matrix(), h->kbad.p));
     HIPCHK(hipMemcpyAsync(&h->lhs_bad, h->kbad.p, sizeof(int), hipMemcpyDeviceToHost, s));
     HIPCHK(hipStreamSynchronize(s));
     h->lhs_ready = true;
@@ -1672,7 +1709,6 @@ int afx_rans_implicit_solve(afx_rans* h, double relaxation, double tol, int32_t 
     if (!h->lhs_ready) return fail(AFX_ESTATE, "call afx_rans_implicit_fill first");
     if (precision != AFX_FP64) return fail(AFX_EUNSUP, "the implicit step uses the FP64 residual");
     hipStream_t s = h->stream;
-    const int64_t n = (int64_t)h->nv * h->nT;
     h->lin_iters = 0;
     auto residual_norm = [&](double* e) -> int {
         // fillRhoRHS starts with calc_dt (solver.h:1081); only the
@@ -1685,12 +1721,9 @@ int afx_rans_implicit_solve(afx_rans* h, double relaxation, double tol, int32_t 
     auto step = [&](bool* ok) -> int {
         if (h->mf)
             HIPCHK(launch_mf_base(s, h->cells64(), h->faces64(), h->q.p, h->gas64(), h->opts.viscosity, h->mfFb.p));
-        int r2 = gmres(h, h->R.p, h->qW.p, ok);
+        int r2 = gmres(h, h->R.p, h->qW.p, relaxation, ok);
         if (r2) return r2;
-        if (*ok) {
-            HIPCHK(launch_axpy(s, relaxation, h->qW.p, h->q.p, n));
-            h->q32_valid = false;
-        }
+        if (*ok) h->q32_valid = false;
         return AFX_OK;
     };
     // Deviation from solver.h:1170-1213: a non-finite residual norm is the
@@ -1728,7 +1761,14 @@ int afx_rans_lhs_apply_nu(afx_rans* h, const double* x, const double* x_nu, doub
     if (!h->lhs_ready) return fail(AFX_ESTATE, "call afx_rans_implicit_fill first");
     if (h->mf) return fail(AFX_ESTATE, "no assembled matrix in matrix-free mode (afx_rans_matrix_free_apply)");
     if ((rc = upload_operand(h, x, x_nu, y_nu))) return rc;
-    HIPCHK(launch_lhs_apply(h->stream, h->nv, h->nC, h->nT, h->ellD.p, h->ellE.p, h->ellN.p, h->ktmp.p, h->kw.p));
+    if (h->precond == 1) {
+        const ColourOrder O = h->colours();
+        HIPCHK(launch_to_colour(h->stream, h->nv, h->nT, O, h->ktmp.p, nullptr, h->kr.p));
+        HIPCHK(launch_colour_apply(h->stream, h->nv, O, h->colour_matrix(), h->kr.p, h->kz.p));
+        HIPCHK(launch_from_colour(h->stream, h->nv, h->nT, O, h->kz.p, h->ktmp.p, h->kw.p));
+    } else {
+        HIPCHK(launch_lhs_apply(h->stream, h->nv, h->nC, h->nT, h->ellD.p, h->ellE.p, h->ellN.p, h->ktmp.p, h->kw.p));
+    }
     return download_operand(h, y, y_nu);
 }
 
@@ -1743,12 +1783,14 @@ int afx_rans_precond_apply_nu(afx_rans* h, const double* x, const double* x_nu, 
     if (!h->lhs_ready) return fail(AFX_ESTATE, "call afx_rans_implicit_fill first");
     if (h->mf) return fail(AFX_ESTATE, "the matrix-free mode has no preconditioner");
     if ((rc = upload_operand(h, x, x_nu, y_nu))) return rc;
-    if (h->precond == 1)
-        HIPCHK(launch_dilu_apply(h->stream, h->nv, h->nC, h->nT, h->col_cells.p, h->col_pos.p, h->col_off.data(),
-                                 (int)h->col_off.size() - 1, h->dilE.p, h->dilN.p, h->dilD.p, h->ktmp.p, h->kw.p,
-                                 h->kdil.p));
-    else
+    if (h->precond == 1) {
+        const ColourOrder O = h->colours();
+        HIPCHK(launch_to_colour(h->stream, h->nv, h->nT, O, h->ktmp.p, nullptr, h->kr.p));
+        HIPCHK(launch_dilu_apply(h->stream, h->nv, O, h->colour_matrix(), h->kr.p, h->kz.p));
+        HIPCHK(launch_from_colour(h->stream, h->nv, h->nT, O, h->kz.p, h->ktmp.p, h->kw.p));
+    } else {
         HIPCHK(launch_block_jacobi(h->stream, h->nv, h->nC, h->nT, h->Dinv.p, h->ktmp.p, h->kw.p));
+    }
     return download_operand(h, y, y_nu);
 }
 

@@ -317,3 +317,65 @@ def test_matrix_free_mode_switches():
     s.set_matrix_free(False)
     s.fill()
     assert np.array_equal(s.lhs_apply(x), y0)
+
+
+# cells in all: rows of the blocks split over threads everywhere; whole in the
+# product only; whole in the large colours too.  At 1e-10 the basis passes every
+# column count at which the passes change variant.
+@pytest.mark.parametrize("model", ["inviscid", "spalart-allmaras"])
+@pytest.mark.parametrize("ni,nj", [(61, 40), (128, 129), (250, 143)])
+def test_colour_order_solve_at_the_variants_edges(ni, nj, model):
+    """The product in colour order equals the one in cell order (block Jacobi's)
+    bit for bit, and the update of a DILU solve satisfies the stopping rule on
+    it: GMRES estimates |A dq - R| <= tol |R|; the update's own rounding adds
+    eps |A| |q| / |R|, bounded by the second term."""
+    from aeroflex_amd import rans
+    sa = model == "spalart-allmaras"
+    m = rans.Mesh.jittered(ni, nj, first_h=2e-3, seed=3, quad_frac=0.3)
+    s = rans.Solver(m, gas=rans.Gas(mu_L=1e-6 if sa else 1e-5), viscosity_model=model)
+    far = rans.BoundaryVariables(mach=0.5, angle=0.03)
+    s.set_bcs({"farfield": rans.BoundaryCondition("farfield", far),
+               "wall": rans.BoundaryCondition("wall" if sa else "slip-wall")})
+    s.init()
+    s.refill_bcs()
+    s.set_cfl(5.0)
+    rng = np.random.default_rng(ni)
+    n, nr = s.n_cells, s.n_real
+    q0 = s.get_q()
+    q0[:4 * nr] *= 1.0 + 1e-3 * rng.standard_normal(4 * nr)
+    nu0 = s.get_nu() if sa else None
+    s.set_q(q0)
+    x, xn = rng.standard_normal(4 * n), rng.standard_normal(n)
+    x[4 * nr:] = 0.0
+    xn[nr:] = 0.0
+
+    def apply(v, vn):
+        out = s.lhs_apply(v, vn) if sa else (s.lhs_apply(v),)
+        return np.concatenate(out)
+    s.set_preconditioner("block-jacobi")
+    s.fill()
+    by_cell = apply(x, xn)
+    s.set_preconditioner("dilu")
+    s.fill()
+    assert s.compute() == 0
+    assert np.array_equal(apply(x, xn), by_cell)
+    R = s.fillRhoRHS()[0]
+    R = np.concatenate([R, s.nu_residual()]) if sa else R
+    tol = 1e-10
+    s.set_linear_solver(30, tol, 500)
+    assert s.solve(relaxation=1.0, tol=0.0, rhs_iterations=0) >= 0
+    its = s.linear_iterations()
+    dq = s.get_q() - q0
+    dn = s.get_nu() - nu0 if sa else None
+    dq[4 * nr:] = 0.0
+    if sa:
+        dn[nr:] = 0.0
+    left = apply(dq, dn)
+    keep = np.ones(len(left), bool)
+    keep[4 * nr:4 * n] = False
+    if sa:
+        keep[4 * n + nr:] = False
+    size = np.linalg.norm(apply(np.abs(q0) * (np.arange(4 * n) < 4 * nr), nu0 * (np.arange(n) < nr) if sa else None))
+    bound = tol * np.linalg.norm(R) + 4 * np.finfo(float).eps * 100 * size
+    assert np.linalg.norm((left - R)[keep]) <= bound
+    assert its > 8
