@@ -97,7 +97,7 @@ struct afx_rans {
     DBuf<uint32_t> cface;
 
     // state and work arrays
-    DBuf<double> q, qk, qW, dt, gx, gy, lim, R, flux;
+    DBuf<double> q, qk, qk2, qW, dt, gx, gy, lim, R, flux;   // qk, qk2: stage states
     DBuf<float> q32, gx32, gy32, lim32, R32, flux32;
     DBuf<double> partial, sum1, uni64, wall_d, states;
     DBuf<double> sa_wd;   // the Spalart-Allmaras model's wall distance (compute_wall_distance)
@@ -1562,12 +1562,46 @@ int afx_rans_explicit_residual(afx_rans* h, const double* qk, double* qW) {
 }  // extern "C"
 
 namespace {
+bool fused64(const afx_rans* h) { return h->opts.fused != 0 && h->tile64_ok; }
+
+// explicitSolver::solve (solver.h:802-828) in the tile kernel, from qin to qout
+// (they may be the same): dt from qin, gradients from qin (A3; from the stage
+// state with the SA model), limiters and fluxes from the stage states, which
+// alternate between two buffers.  keep as for explicit_step64; last_R: where
+// the last stage's undivided residual goes (nullable).
+int explicit_step_tiles(afx_rans* h, const double* qin, double* qout, double relax, double* const* keep,
+                        double* last_R) {
+    static const double alpha[3] = {0.25, 0.5, 1.};
+    hipStream_t s = h->stream;
+    const int64_t nq = (int64_t)h->nv * h->nT;
+    if (!h->qk2.p) HIPCHK(h->qk2.alloc((size_t)NV_MAX * h->nT));
+    double* a = keep ? keep[3] : h->qk2.p;
+    double* b = keep ? keep[4] : h->qk.p;
+    // the last stage writes beside its input and, when viscous fluxes read qin
+    // of neighbouring cells, beside qin
+    const bool beside = qout == qin && h->opts.viscosity == 1;
+    double* last = beside ? h->qk2.p : qout;
+    const double* from[3] = {qin, a, b};
+    double* to[3] = {a, b, last};
+    for (int st = 0; st < 3; ++st) {
+        double* W = keep ? keep[st] : st == 2 ? h->qW.p : nullptr;
+        const StageT<double> stage{qin,     to[st],  W,      st == 2 ? last_R : nullptr, h->dt.p, h->gx.p,
+                                   h->gy.p, h->cfl,  alpha[st], relax,   h->needs_gradients() ? 1 : 0};
+        HIPCHK(launch_stage_tile(s, h->tiles<double>(h->t_geo64.p), from[st], h->nT, h->nC, h->area.p, h->lsq.p,
+                                 h->xc.p, h->yc.p, h->sa_wd.p, h->gas64(), h->opts.gradient, h->so(),
+                                 h->opts.limiter_k, h->opts.viscosity, stage, st == 0));
+    }
+    if (last != qout) HIPCHK(launch_copy(s, last, qout, nq));
+    return AFX_OK;
+}
+
 // explicitSolver::solve (solver.h:802-828) for four variables, from qin to
 // qout (they may alias): dt from qin, stage states qk, gradients from qin
 // (A3), limiters and fluxes from qk, qk = qin + qW dt alpha_s relax.  With
 // keep non-null the stage residuals go to keep[0..2] and the stage states
 // qk_1, qk_2 to keep[3], keep[4] (for the reverse sweep).
 int explicit_step64(afx_rans* h, const double* qin, double* qout, double relax, double* const* keep) {
+    if (fused64(h)) return explicit_step_tiles(h, qin, qout, relax, keep, nullptr);
     static const double alpha[3] = {0.25, 0.5, 1.};
     hipStream_t s = h->stream;
     const int64_t nq = (int64_t)NV * h->nT;
@@ -1603,24 +1637,11 @@ int afx_rans_explicit_step(afx_rans* h, double relaxation, double* err) {
         // explicitSolver::solve (solver.h:802-828) with the five-variable
         // fused residual: gradients and limiters from the stage state
         if (!h->tile64_ok) return fail(AFX_EUNSUP, "the Spalart-Allmaras residual needs the fused tile kernels");
-        static const double alpha5[3] = {0.25, 0.5, 1.};
-        hipStream_t s = h->stream;
-        const int64_t nq = (int64_t)h->nv * h->nT;
-        HIPCHK(launch_dt<double>(s, h->cells64(), h->faces64(), h->q.p, h->gas64(), h->cfl, h->dt.p, 1));
-        HIPCHK(launch_copy(s, h->q.p, h->qk.p, nq));
-        for (double ai : alpha5) {
-            HIPCHK(launch_residual_tile<double>(s, h->tiles<double>(h->t_geo64.p), h->qk.p, h->nT, h->nC, h->area.p,
-                                                h->lsq.p, h->xc.p, h->yc.p, h->sa_wd.p, h->gas64(), h->opts.gradient,
-                                                h->so(), h->opts.limiter_k, h->opts.viscosity, h->R.p,
-                                                h->qk.p));
-            HIPCHK(launch_rk_update_area(s, h->q.p, h->R.p, h->area.p, h->dt.p, ai * relaxation, h->nC, h->nT, h->nv,
-                                         h->qk.p, h->qW.p));
-        }
-        HIPCHK(launch_copy(s, h->qk.p, h->q.p, nq));
+        if ((rc = explicit_step_tiles(h, h->q.p, h->q.p, relaxation, nullptr, h->R.p))) return rc;
         h->q32_valid = false;
         h->last_precision = AFX_FP64;
         if (err) return norm_of(h, h->qW.p, h->nT, h->nv, err);
-        HIPCHK(hipStreamSynchronize(s));
+        HIPCHK(hipStreamSynchronize(h->stream));
         return AFX_OK;
     }
     if ((rc = explicit_step64(h, h->q.p, h->q.p, relaxation, nullptr))) return rc;

@@ -366,15 +366,19 @@ __device__ __forceinline__ T sa_cell_source(const GasT<T>& g, const T* q, const 
 // (owner state on boundary faces); the cell's viscous radius is the sum of
 // coef len^2 / A and enters with weight 4.  q: planes of nT cells.
 template <typename T>
+__device__ __forceinline__ T sa_viscous_radius(const GasT<T>& g, T rho, T nuf) {
+    const T mut = nuf * sa_fv1<T>(ddiv<T>(nuf, g.mu));
+    const T kmax = g.gamma > T(4.0 / 3.0) ? g.gamma : T(4.0 / 3.0);
+    return ddiv<T>(kmax * (ddiv<T>(g.mu, g.PrL) + ddiv<T>(mut, g.PrT)), rho);
+}
+template <typename T>
 __device__ __forceinline__ T sa_viscous_radius(const GasT<T>& g, const T* q, size_t nT, int o, int n, bool internal) {
     T rho = q[o], nuf = q[4 * nT + o];
     if (internal) {
         rho = T(0.5) * (rho + q[n]);
         nuf = T(0.5) * (nuf + q[4 * nT + n]);
     }
-    const T mut = nuf * sa_fv1<T>(ddiv<T>(nuf, g.mu));
-    const T kmax = g.gamma > T(4.0 / 3.0) ? g.gamma : T(4.0 / 3.0);
-    return ddiv<T>(kmax * (ddiv<T>(g.mu, g.PrL) + ddiv<T>(mut, g.PrT)), rho);
+    return sa_viscous_radius<T>(g, rho, nuf);
 }
 
 // ---------------------------------------------------------------- kernels --
@@ -638,18 +642,65 @@ __global__ void __launch_bounds__(kBlock) k_gather(CellsT<T> C, const T* __restr
 
 
 
+// what the tile kernel makes of the residual: R, or the update of an explicit
+// stage (StageT): the first one, which also forms the local time step and
+// leaves the gradients of its state, and the later ones, which with four
+// variables read those gradients (A3) instead of forming their own
+enum TileMode { TILE_RESIDUAL = 0, TILE_FIRST = 1, TILE_LATER = 2 };
+
+// local time step of solver.h:308-356 (and the SA model's viscous radius) of
+// cell c of the tile from the staged states, as k_dt forms it
+template <typename T, int NV, bool BND>
+__device__ __forceinline__ T tile_time_step(const TilesT<T>& S, const GasT<T>& g, const T* sq, int LM, int fo,
+                                            uint64_t sw, T area, T cfl) {
+    const int64_t NF = S.nFtot;
+    const T gm1 = g.gamma - T(1);
+    T sum = T(0), sv = T(0);
+    auto speed = [&](int c, T nx, T ny) {
+        const T q0 = sq[c], q1 = sq[LM + c], q2 = sq[2 * LM + c], q3 = sq[3 * LM + c];
+        const T V = ddiv<T>(q1 * nx + q2 * ny, q0);
+        const T p = gm1 * (q3 - ddiv<T>(T(0.5), q0) * (q1 * q1 + q2 * q2));
+        return dsqrt<T>(ddiv<T>(p * g.gamma, q0)) + dabs<T>(V);
+    };
+    for (int s = 0; s < 4; ++s) {
+        const uint32_t e = (uint32_t)(sw >> (16 * s)) & 0xFFFFu;
+        if (e == 0xFFFFu) break;
+        const int f = fo + (int)(e & 0x7FFFu);
+        const uint32_t fc = S.fcell[f];
+        const int o = (int)(fc & 0xFFFFu), n = (int)(fc >> 16);
+        const bool internal = !BND || S.fkind[f] == K_INTERNAL;
+        const T nx = S.geo[f], ny = S.geo[NF + f], L = S.geo[2 * NF + f];
+        T eig = speed(o, nx, ny);
+        if (internal) {
+            const T r = speed(n, nx, ny);
+            eig = (eig < r) ? r : eig;
+        }
+        sum += eig * L;
+        if constexpr (NV == 5) {
+            T rho = sq[o], nuf = sq[4 * LM + o];
+            if (internal) {
+                rho = T(0.5) * (rho + sq[n]);
+                nuf = T(0.5) * (nuf + sq[4 * LM + n]);
+            }
+            sv += sa_viscous_radius<T>(g, rho, nuf) * L * L;
+        }
+    }
+    return NV == 5 ? ddiv<T>(cfl * area, sum + T(4) * ddiv<T>(sv, area)) : ddiv<T>(cfl * area, sum);
+}
+
 // BND: the tile's face list holds boundary faces; without, every face is
 // taken as interior at compile time (no kind tests, no boundary states, no
 // ghost writes) - the same operations on the same values, so the same bits
-template <typename T, int NV, bool BND>
+template <typename T, int NV, bool BND, int MODE = TILE_RESIDUAL>
 __device__ __forceinline__ void residual_tile_body(const TilesT<T>& S, const T* __restrict__ q, int32_t nT, int32_t nC,
                                                    const T* __restrict__ area, const T* __restrict__ lsq,
                                                    const T* __restrict__ xc, const T* __restrict__ yc,
                                                    const T* __restrict__ wd, const GasT<T>& g, int gg,
                                                    int second_order, T limiter_k, int viscous,
                                                    T* __restrict__ R, T* __restrict__ qghost, const int t,
-                                                   unsigned char* smem_raw) {
+                                                   unsigned char* smem_raw, const StageT<T>& st = StageT<T>{}) {
     constexpr bool SA = (NV == 5);
+    constexpr bool STORED = MODE == TILE_LATER && !SA;   // gradients of the first stage's state
     const int c0g = S.cell0[t], nTt = S.cell0[t + 1] - c0g;
     const int lo = S.loff[t], nL = S.loff[t + 1] - lo;
     const int nG = S.ng[t];
@@ -680,7 +731,9 @@ __device__ __forceinline__ void residual_tile_body(const TilesT<T>& S, const T* 
         T sx[NV], sy[NV];
         for (int k = 0; k < NV; ++k) { sx[k] = T(0); sy[k] = T(0); }
         const int gc = Lg[c];
-        if (gg) {
+        if constexpr (STORED) {
+            for (int k = 0; k < NV; ++k) { sx[k] = st.gx[(size_t)k * nT + gc]; sy[k] = st.gy[(size_t)k * nT + gc]; }
+        } else if (gg) {
             for (int s = 0; s < 4; ++s) {
                 const uint32_t e = (uint32_t)(sw >> (16 * s)) & 0xFFFFu;
                 if (e == 0xFFFFu) break;
@@ -745,6 +798,13 @@ __device__ __forceinline__ void residual_tile_body(const TilesT<T>& S, const T* 
             }
         }
         for (int k = 0; k < NV; ++k) { sgx[k * GM + c] = sx[k]; sgy[k * GM + c] = sy[k]; }
+        if constexpr (MODE == TILE_FIRST && !SA) {
+            if (c < nTt)
+                for (int k = 0; k < NV; ++k) {
+                    st.gx[(size_t)k * nT + gc] = sx[k];
+                    st.gy[(size_t)k * nT + gc] = sy[k];
+                }
+        }
         if (second_order) {
             T qmin[NV], qmax[NV];
             for (int k = 0; k < NV; ++k) { qmin[k] = qc[k]; qmax[k] = qc[k]; }
@@ -819,7 +879,9 @@ __device__ __forceinline__ void residual_tile_body(const TilesT<T>& S, const T* 
             const T l = dsqrt<T>(t0 * t0 + t1 * t1);
             t0 = ddiv<T>(t0, l); t1 = ddiv<T>(t1, l);
             for (int k = 0; k < NV; ++k) {
-                const T dir = SA ? ddiv<T>(sq[k * LM + n] - sq[k * LM + o], l) : ddiv<T>(sq[k * LM + o] - sq[k * LM + n], l);
+                T dq = SA ? sq[k * LM + n] - sq[k * LM + o] : sq[k * LM + o] - sq[k * LM + n];
+                if constexpr (STORED) dq = st.q0[(size_t)k * nT + go_] - st.q0[(size_t)k * nT + gn_];
+                const T dir = ddiv<T>(dq, l);
                 const T gxb = (sgx[k * GM + o] + sgx[k * GM + n]) * T(0.5);
                 const T gyb = (sgy[k * GM + o] + sgy[k * GM + n]) * T(0.5);
                 const T dot = gxb * t0 + gyb * t1;
@@ -840,6 +902,7 @@ __device__ __forceinline__ void residual_tile_body(const TilesT<T>& S, const T* 
     __syncthreads();
 
     // 4. signed sums in reference face order; one coalesced write per cell
+    T* const ghosts = MODE == TILE_RESIDUAL ? qghost : st.next;
     for (int c = threadIdx.x; c < nTt; c += blockDim.x) {
         const uint64_t sw = S.slots[go + c];
         Acc<T> acc[NV];
@@ -849,20 +912,46 @@ __device__ __forceinline__ void residual_tile_body(const TilesT<T>& S, const T* 
             const int fl = (int)(e & 0x7FFFu);
             if (e >> 15) for (int k = 0; k < NV; ++k) acc[k].add(sfl[k * FM + fl]);
             else for (int k = 0; k < NV; ++k) acc[k].sub(sfl[k * FM + fl]);
-            if (BND && qghost) {
+            if (BND && ghosts) {
                 const int kind = S.fkind[fo + fl];
+                const int n = (int)(S.fcell[fo + fl] >> 16);
                 if (kind == K_WALL || kind == K_SLIP) {
-                    const int gh = -1 - Lg[(int)(S.fcell[fo + fl] >> 16)];
-                    for (int k = 0; k < NV; ++k) qghost[(size_t)k * nT + gh] = sq[k * LM + c];
+                    const size_t gh = (size_t)(-1 - Lg[n]);
+                    const bool copy = MODE == TILE_RESIDUAL || SA || st.walls != 0;
+                    for (int k = 0; k < NV; ++k)
+                        ghosts[(size_t)k * nT + gh] = copy ? sq[k * LM + c] : q[(size_t)k * nT + gh];
+                } else if (MODE != TILE_RESIDUAL && kind != K_INTERNAL) {
+                    for (int k = 0; k < NV; ++k) ghosts[(size_t)k * nT + Lg[n]] = sq[k * LM + n];
                 }
             }
         }
-        for (int k = 0; k < 4; ++k) R[(size_t)k * nT + c0g + c] = acc[k].value();
+        const int gc = c0g + c;
+        T sum[NV];
+        for (int k = 0; k < NV; ++k) sum[k] = acc[k].value();
         if constexpr (SA) {
             T qs[NV], gxs[NV], gys[NV];
             for (int k = 0; k < NV; ++k) { qs[k] = sq[k * LM + c]; gxs[k] = sgx[k * GM + c]; gys[k] = sgy[k * GM + c]; }
-            const int gc = c0g + c;
-            R[(size_t)4 * nT + gc] = acc[4].value() + area[gc] * sa_cell_source<T>(g, qs, gxs, gys, wd[gc]);
+            sum[4] = sum[4] + area[gc] * sa_cell_source<T>(g, qs, gxs, gys, wd[gc]);
+        }
+        if constexpr (MODE == TILE_RESIDUAL) {
+            for (int k = 0; k < NV; ++k) R[(size_t)k * nT + gc] = sum[k];
+        } else {
+            const T A = area[gc];
+            T dt;
+            if constexpr (MODE == TILE_FIRST) {
+                dt = tile_time_step<T, NV, BND>(S, g, sq, LM, fo, sw, A, st.cfl);
+                st.dt[gc] = dt;
+            } else {
+                dt = st.dt[gc];
+            }
+            for (int k = 0; k < NV; ++k) {
+                const size_t i = (size_t)k * nT + gc;
+                if (st.R) st.R[i] = sum[k];
+                // solver.h:818-821, and with SA the operation order of its own step
+                const T w = SA ? sum[k] * (T(1.0) / A) : ddiv<T>(sum[k], A);
+                if (st.W) st.W[i] = w;
+                st.next[i] = SA ? st.q0[i] + w * dt * (st.alpha * st.relax) : st.q0[i] + w * dt * st.alpha * st.relax;
+            }
         }
     }
 }
@@ -883,6 +972,31 @@ __global__ void __launch_bounds__(kBlock) k_residual_tile(TilesT<T> S, const T* 
     else
         residual_tile_body<T, NV, true>(S, q, nT, nC, area, lsq, xc, yc, wd, g, gg, second_order, limiter_k, viscous, R,
                                         qghost, t, smem_raw);
+}
+
+// One explicit stage of every tile.  In place of the time step, gradient,
+// limiter, flux, sum, update and ghost kernels of a stage (22 launches per
+// step with four variables) it is one launch whose intermediate values stay in
+// LDS, and the gradients, which A3 takes from the step's start, are formed once
+// per step.  Bound by the latency of one tile's FP64 chain on small meshes and
+// by FP64 issue on large ones.  A step of a 16k-cell inviscid mesh with its
+// norm went from 109 to 93 us, six SA steps of 250k cells with their transfers
+// from 3.18 to 2.94 ms.
+template <typename T, int NV, int MODE>
+__global__ void __launch_bounds__(kBlock) k_stage_tile(TilesT<T> S, const T* __restrict__ q, int32_t nT, int32_t nC,
+                                                       const T* __restrict__ area, const T* __restrict__ lsq,
+                                                       const T* __restrict__ xc, const T* __restrict__ yc,
+                                                       const T* __restrict__ wd, GasT<T> g, int gg, int second_order,
+                                                       T limiter_k, int viscous, StageT<T> st) {
+    extern __shared__ unsigned char smem_raw[];
+    const int t = xcd_tile(blockIdx.x, gridDim.x);
+    if (t >= S.ntiles) return;
+    if (S.nbf && S.nbf[t] == 0)
+        residual_tile_body<T, NV, false, MODE>(S, q, nT, nC, area, lsq, xc, yc, wd, g, gg, second_order, limiter_k,
+                                               viscous, nullptr, nullptr, t, smem_raw, st);
+    else
+        residual_tile_body<T, NV, true, MODE>(S, q, nT, nC, area, lsq, xc, yc, wd, g, gg, second_order, limiter_k,
+                                              viscous, nullptr, nullptr, t, smem_raw, st);
 }
 
 // ---------------------------------------------------------------------------

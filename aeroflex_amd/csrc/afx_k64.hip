@@ -6,6 +6,19 @@
 namespace afx {
 AFX_INSTANTIATE_LAUNCHERS(double)
 
+hipError_t launch_stage_tile(hipStream_t s, TilesT<double> S, const double* q, int32_t nT, int32_t nC,
+                             const double* area, const double* lsq, const double* xc, const double* yc,
+                             const double* wd, GasT<double> g, int gg, int so, double lk, int viscous,
+                             const StageT<double>& st, bool first) {
+    const int nb = ((S.ntiles + 7) / 8) * 8, nv = viscous == 2 ? 5 : 4;
+    const size_t lds = tile_lds_bytes<double>(S.lmax, S.gmax, S.ftmax, nv);
+    auto stage = nv == 5 ? (first ? k_stage_tile<double, 5, TILE_FIRST> : k_stage_tile<double, 5, TILE_LATER>)
+                         : (first ? k_stage_tile<double, 4, TILE_FIRST> : k_stage_tile<double, 4, TILE_LATER>);
+    hipLaunchKernelGGL(stage, dim3(nb), dim3(kBlock), lds, s, S, q, nT, nC, area, lsq, xc, yc, wd, g, gg, so, lk,
+                       viscous, st);
+    return hipGetLastError();
+}
+
 // sum of squares over nv rows of length n (row stride ld); one partial per block
 template <typename T>
 __global__ void __launch_bounds__(kBlock) k_sumsq(const T* __restrict__ x, int64_t n, int64_t ld, int nv,
@@ -94,30 +107,6 @@ __global__ void __launch_bounds__(kBlock) k_rk_update(const double* __restrict__
 hipError_t launch_rk_update(hipStream_t s, const double* q, const double* qW, const double* dt, double ai, double relax,
                             int32_t nC, int32_t nT, int nv, double* qk) {
     hipLaunchKernelGGL(k_rk_update, dim3(nblocks(nC)), dim3(kBlock), 0, s, q, qW, dt, ai, relax, nC, nT, nv, qk);
-    return hipGetLastError();
-}
-
-// explicit stage update from an undivided residual (R / A as qW of
-// solver.h:790-792), for the Spalart-Allmaras explicit step
-__global__ void __launch_bounds__(kBlock) k_rk_update_area(const double* __restrict__ q, const double* __restrict__ R,
-                                                           const double* __restrict__ area,
-                                                           const double* __restrict__ dt, double coef, int32_t nC,
-                                                           int32_t nT, int nv, double* __restrict__ qk,
-                                                           double* __restrict__ qW) {
-    int c = blockIdx.x * blockDim.x + threadIdx.x;
-    if (c >= nC) return;
-    const double ia = 1.0 / area[c];
-    for (int k = 0; k < nv; ++k) {
-        size_t i = (size_t)k * nT + c;
-        const double w = R[i] * ia;
-        qW[i] = w;
-        qk[i] = q[i] + w * dt[c] * coef;
-    }
-}
-hipError_t launch_rk_update_area(hipStream_t s, const double* q, const double* R, const double* area, const double* dt,
-                                 double coef, int32_t nC, int32_t nT, int nv, double* qk, double* qW) {
-    hipLaunchKernelGGL(k_rk_update_area, dim3(nblocks(nC)), dim3(kBlock), 0, s, q, R, area, dt, coef, nC, nT, nv, qk,
-                       qW);
     return hipGetLastError();
 }
 

@@ -85,6 +85,31 @@ hipError_t launch_residual_tile(hipStream_t s, TilesT<T> S, const T* q, int32_t 
                                 const T* lsq, const T* xc, const T* yc, const T* wd, GasT<T> g, int gg,
                                 int second_order, T limiter_k, int viscous, T* R, T* qghost);
 
+// One explicit stage (explicitSolver::solve, solver.h:802-828) in the tile
+// kernel instead of the residual alone: next = q0 + W dt alpha relax of the
+// real cells, W = R / A, and the ghosts of next: wall and slip ghosts take
+// their owner's state of this stage (set_walls_from_internal; with walls = 0,
+// the first-order inviscid step, they keep theirs), farfield ghosts keep theirs.  next must not be the state the stage reads; it may be q0 from
+// the second stage on, unless the model is laminar (viscous fluxes read q0 of
+// the neighbours).
+template <typename T>
+struct StageT {
+    const T* q0;
+    T* next;
+    T* W;         // nullable
+    T* R;         // nullable: the undivided residual
+    T* dt;        // local time step, written by the first stage
+    T* gx;        // four variables: the gradients of q0 (A3), written by the
+    T* gy;        // first stage and read by the later ones
+    T cfl, alpha, relax;
+    int walls;
+};
+// first: the stage state is q0 itself
+hipError_t launch_stage_tile(hipStream_t s, TilesT<double> S, const double* q, int32_t nT, int32_t nC,
+                             const double* area, const double* lsq, const double* xc, const double* yc,
+                             const double* wd, GasT<double> g, int gg, int second_order, double limiter_k, int viscous,
+                             const StageT<double>& st, bool first);
+
 // FP32 throughput form of the same (afx_k32.hip): cell states, gradients,
 // limiters, fluxes and residuals are float4 per cell / face (rho, rho u,
 // rho v, rho E); per tile face two float4 (nx, ny, len, g) and (d0x, d0y,
@@ -163,9 +188,6 @@ inline size_t tile_lds_bytes_f32(const TilesF32& S, int nv, bool dt) {
 hipError_t launch_residual_tile_f32_batch(hipStream_t s, const TileArgsF32* members, const int2* items, int32_t nitems,
                                           size_t lds, int viscous, int gg, int second_order);
 
-// SA explicit step of one solver: qk = q + R / A dt coef (real cells, nv planes), qW = R / A
-hipError_t launch_rk_update_area(hipStream_t s, const double* q, const double* R, const double* area, const double* dt,
-                                 double coef, int32_t nC, int32_t nT, int nv, double* qk, double* qW);
 hipError_t launch_to_f32x4(hipStream_t s, const double* src, int32_t nT, float4* dst);
 
 // ---- launchers (instantiated for double in afx_k64.hip, float in afx_k32.hip)
