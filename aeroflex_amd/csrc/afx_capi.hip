@@ -541,6 +541,92 @@ int download_operand(afx_rans* h, double* y, double* y_nu) {
     return download_cells(h, h->kw.p + 4 * (size_t)h->nT, y_nu);
 }
 
+// A colouring of the cells (at most four neighbours each, -1: none) with few
+// colours: every colour beyond the first costs a GMRES step two more launches,
+// however few cells it has, while the number of steps hardly depends on the
+// colouring (30 for a 16k-cell grid at CFL 40 with two, three or four).
+// Breadth first over the whole mesh, each cell the lowest free colour: two
+// colours where the cells' graph has two (a grid of split quadrilaterals), three
+// and a last handful of cells elsewhere.  Those are then freed by Kempe chains:
+// a cell whose neighbours use every lower colour takes colour a once the
+// (a, b) chains of its neighbours of colour a are flipped, which is possible
+// where none of them reaches a neighbour of colour b.  Chains of more than
+// kChain cells are left alone, so the work is linear in the mesh.
+std::vector<uint8_t> colour_cells(const std::vector<int32_t>& nbr, int32_t nC, int* ncolours) {
+    constexpr uint8_t none = 0xFF;
+    constexpr size_t kChain = 16;
+    std::vector<uint8_t> col(nC, none);
+    std::vector<int32_t> queue;
+    queue.reserve(nC);
+    std::vector<char> seen(nC, 0);
+    size_t count[5] = {0, 0, 0, 0, 0};   // at most four neighbours: at most five colours
+    for (int32_t s = 0; s < nC; ++s) {
+        if (seen[s]) continue;
+        seen[s] = 1;
+        size_t head = queue.size();
+        queue.push_back(s);
+        while (head < queue.size()) {
+            const int32_t i = queue[head++];
+            unsigned used = 0;
+            for (int k = 0; k < 4; ++k) {
+                const int32_t j = nbr[4 * (size_t)i + k];
+                if (j < 0) continue;
+                if (col[j] != none) used |= 1u << col[j];
+                if (!seen[j]) { seen[j] = 1; queue.push_back(j); }
+            }
+            int c = 0;
+            while (used & (1u << c)) ++c;
+            col[i] = (uint8_t)c;
+            ++count[c];
+        }
+    }
+    int n = 0;
+    while (n < 5 && count[n]) ++n;
+    // free the last colour while it holds less than a tenth of the cells
+    std::vector<int32_t> chain;
+    auto has = [&](int32_t j) { return std::find(chain.begin(), chain.end(), j) != chain.end(); };
+    while (n > 2 && count[n - 1] * 10 < (size_t)nC) {
+        const int top = n - 1;
+        size_t left = 0;
+        for (int32_t v = 0; v < nC; ++v) {
+            if (col[v] != top) continue;
+            const int32_t* nv = &nbr[4 * (size_t)v];
+            bool freed = false;
+            for (int a = 0; a < top && !freed; ++a)
+                for (int b = 0; b < top && !freed; ++b) {
+                    if (a == b) continue;
+                    chain.clear();
+                    for (int k = 0; k < 4; ++k)
+                        if (nv[k] >= 0 && col[nv[k]] == a && !has(nv[k])) chain.push_back(nv[k]);
+                    bool ok = true;
+                    for (size_t q = 0; q < chain.size() && ok; ++q)
+                        for (int k = 0; k < 4 && ok; ++k) {
+                            const int32_t w = nbr[4 * (size_t)chain[q] + k];
+                            if (w < 0 || w == v || (col[w] != a && col[w] != b) || has(w)) continue;
+                            if (col[w] == b && (w == nv[0] || w == nv[1] || w == nv[2] || w == nv[3])) ok = false;
+                            else chain.push_back(w);
+                            if (chain.size() > kChain) ok = false;
+                        }
+                    if (!ok) continue;
+                    for (int32_t u : chain) {
+                        --count[col[u]];
+                        col[u] = (uint8_t)(col[u] == a ? b : a);
+                        ++count[col[u]];
+                    }
+                    --count[top];
+                    ++count[a];
+                    col[v] = (uint8_t)a;
+                    freed = true;
+                }
+            left += !freed;
+        }
+        if (left) break;
+        --n;
+    }
+    *ncolours = n;
+    return col;
+}
+
 int ensure_implicit(afx_rans* h) {
     if (h->mf && !h->mfFb.p) HIPCHK(h->mfFb.alloc((size_t)4 * h->nF));
     if (!h->mf && h->precond == 0 && !h->ellE.p) {   // the product in cell order
@@ -578,8 +664,7 @@ int ensure_implicit(afx_rans* h) {
     HIPCHK(h->kbad.alloc(1));
     HIPCHK(hipMemsetAsync(h->Jf.p, 0, 2 * nn * h->nF * 8, h->stream));
     HIPCHK(hipMemsetAsync(h->kflags.p, 0, 8 * sizeof(int), h->stream));
-    // greedy colouring of the real cells in device order over their
-    // real-cell face neighbours (at most four), for the DILU sweeps
+    // colouring of the real cells, for the DILU sweeps
     {
         const int32_t nC = h->nC;
         std::vector<uint32_t> cf((size_t)4 * nC);
@@ -588,22 +673,17 @@ int ensure_implicit(afx_rans* h) {
         HIPCHK(hipMemcpyAsync(c0.data(), h->c0.p, c0.size() * 4, hipMemcpyDeviceToHost, h->stream));
         HIPCHK(hipMemcpyAsync(c1.data(), h->c1.p, c1.size() * 4, hipMemcpyDeviceToHost, h->stream));
         HIPCHK(hipStreamSynchronize(h->stream));
-        std::vector<uint8_t> col(nC, 0xFF);
-        int ncol = 0;
-        for (int32_t i = 0; i < nC; ++i) {
-            unsigned used = 0;
+        std::vector<int32_t> nbr((size_t)4 * nC, -1);
+        for (int32_t i = 0; i < nC; ++i)
             for (int sl = 0; sl < 4; ++sl) {
                 const uint32_t e = cf[(size_t)sl * nC + i];
                 if (e == 0xFFFFFFFFu) break;
                 const int32_t f = (int32_t)(e & 0x7FFFFFFFu);
                 const int32_t j = (e >> 31) ? c0[f] : c1[f];
-                if (j < nC && col[j] != 0xFF) used |= 1u << col[j];
+                if (j < nC) nbr[4 * (size_t)i + sl] = j;
             }
-            int c = 0;
-            while (used & (1u << c)) ++c;   // at most 4 neighbours: c <= 4
-            col[i] = (uint8_t)c;
-            ncol = std::max(ncol, c + 1);
-        }
+        int ncol = 0;
+        const std::vector<uint8_t> col = colour_cells(nbr, nC, &ncol);
         h->col_off.assign(ncol + 1, 0);
         for (int32_t i = 0; i < nC; ++i) h->col_off[col[i] + 1]++;
         for (int c = 0; c < ncol; ++c) h->col_off[c + 1] += h->col_off[c];
@@ -951,6 +1031,14 @@ int afx_rans_create_like(const afx_rans* base, const afx_gas* g, afx_rans** out)
 }
 
 namespace {
+// Residuals (FP64 / FP32, us) with tiles of 192 to 224 and of 128 cells: 4k cells
+// inviscid 26.1 / 8.7 and 15.7 / 5.9, SA 31.7 / 10.6 and 21.7 / 7.9; 16k SA 29.9
+// / 10.0 and 18.9 / 7.2; 60k SA 38.6 / 12.1 and 28.2 / 9.2; 115k SA 51.0 / 13.0
+// and 43.4 / 11.5; a batched step of eight members 60 and 54 (16k), 81 and 88
+// (29k), 148 and 135 (60k), 218 and 231 (115k).  At 2M cells the FP64 form is
+// alike at 128 and 160 and the FP32 form 7 % faster at 192 to 200.
+constexpr int32_t kSmallMesh = 131072;
+
 int create_impl(const Mesh& mesh_in, const afx_gas* g, const afx_opts* o, const afx_rans* like, afx_rans** out) {
     afx_opts opts;
     afx_default_opts(&opts);
@@ -993,8 +1081,10 @@ int create_impl(const Mesh& mesh_in, const afx_gas* g, const afx_opts* o, const 
         if (opts.renumber) seeds = rcm_order(m);
         else { seeds.resize(nC); std::iota(seeds.begin(), seeds.end(), 0u); }
         // automatic size: the largest tile (from 256 cells down) whose FP64
-        // working set fits the 64 KiB of LDS one workgroup may use
-        int32_t target = opts.tile_cells > 0 ? opts.tile_cells : 256;
+        // working set fits the 64 KiB of LDS one workgroup may use; 128 cells
+        // below kSmallMesh, where larger tiles leave compute units idle and
+        // give each thread of a tile two cells and faces in turn
+        int32_t target = opts.tile_cells > 0 ? opts.tile_cells : nC < kSmallMesh ? 128 : 256;
         try {
             h->tl = build_tiles(m, seeds, target);
             while (opts.tile_cells <= 0 && target > 64 &&
@@ -1097,23 +1187,18 @@ int create_impl(const Mesh& mesh_in, const afx_gas* g, const afx_opts* o, const 
     HIPCHK_C(h->fxf32.alloc(nF)); HIPCHK_C(h->fxf32.upload(to_device_order_faces<float>(h, m.edgesCentersX), s));
     HIPCHK_C(h->fyf32.alloc(nF)); HIPCHK_C(h->fyf32.upload(to_device_order_faces<float>(h, m.edgesCentersY), s));
     HIPCHK_C(h->fgw.alloc(nF)); HIPCHK_C(h->fgw.upload(hgw, s));
-    {
-        std::vector<float> g32(hgw.begin(), hgw.end());
-        HIPCHK_C(h->fgw32.alloc(nF)); HIPCHK_C(h->fgw32.upload(g32, s));
-        std::vector<float> l32(hlsq.begin(), hlsq.end());
-        HIPCHK_C(h->lsq.alloc(hlsq.size())); HIPCHK_C(h->lsq.upload(hlsq, s));
-        HIPCHK_C(h->lsq32.alloc(l32.size())); HIPCHK_C(h->lsq32.upload(l32, s));
-        HIPCHK_C(hipStreamSynchronize(s));
-    }
+    // (the vectors uploaded from here on live until the wait at the end)
+    std::vector<float> g32(hgw.begin(), hgw.end());
+    HIPCHK_C(h->fgw32.alloc(nF)); HIPCHK_C(h->fgw32.upload(g32, s));
+    std::vector<float> l32(hlsq.begin(), hlsq.end());
+    HIPCHK_C(h->lsq.alloc(hlsq.size())); HIPCHK_C(h->lsq.upload(hlsq, s));
+    HIPCHK_C(h->lsq32.alloc(l32.size())); HIPCHK_C(h->lsq32.upload(l32, s));
     HIPCHK_C(h->o2n.alloc(nT)); HIPCHK_C(h->o2n.upload(h->c_old2new, s));
     HIPCHK_C(h->c0.alloc(nF)); HIPCHK_C(h->c0.upload(hc0, s));
     HIPCHK_C(h->c1.alloc(nF)); HIPCHK_C(h->c1.upload(hc1, s));
     HIPCHK_C(h->cface.alloc(hcface.size())); HIPCHK_C(h->cface.upload(hcface, s));
-    {
-        std::vector<int8_t> kind(nF, K_INTERNAL);
-        HIPCHK_C(h->fkind.alloc(nF)); HIPCHK_C(h->fkind.upload(kind, s));
-        HIPCHK_C(hipStreamSynchronize(s));
-    }
+    static_assert(K_INTERNAL == 0, "interior faces are the zero kind");
+    HIPCHK_C(h->fkind.alloc(nF)); HIPCHK_C(hipMemsetAsync(h->fkind.p, 0, std::max(nF, 1), s));
     // state arrays (NV_MAX planes; the fifth holds rho nu~ with the SA model)
     const size_t nq = (size_t)NV_MAX * nT;
     for (DBuf<double>* b : {&h->q, &h->qk, &h->qW, &h->gx, &h->gy, &h->lim, &h->R}) {
@@ -1132,14 +1217,20 @@ int create_impl(const Mesh& mesh_in, const afx_gas* g, const afx_opts* o, const 
     HIPCHK_C(launch_fill(s, h->lim.p, 1.0, (int64_t)nq));
     HIPCHK_C(launch_fill(s, h->lim32.p, 1.0f, (int64_t)nq));
     // tile tables (only usable when the cell order is the tile order)
+    std::vector<int32_t> lg;
+    std::vector<float> ia, a15, geo32;
+    std::vector<double> geo;
+    std::vector<float4> g4;
+    std::vector<uint32_t> fck;
     if (opts.renumber) {
         const TileLayout& tl = h->tl;
-        std::vector<int32_t> lg(tl.L_ref.size());
+        lg.resize(tl.L_ref.size());
         for (size_t i = 0; i < lg.size(); ++i) lg[i] = h->c_old2new[tl.L_ref[i]];
         h->t_lg = lg;
         {
             // FP32 form: 1/A and A^1.5 per cell (K3a = K^3 A^1.5, solver.h:551-552)
-            std::vector<float> ia(nT), a15(nT);
+            ia.resize(nT);
+            a15.resize(nT);
             for (int32_t i = 0; i < nT; ++i) {
                 double A = m.cellsAreas[h->c_new2old[i]];
                 ia[i] = (float)(1.0 / A);
@@ -1147,11 +1238,10 @@ int create_impl(const Mesh& mesh_in, const afx_gas* g, const afx_opts* o, const 
             }
             HIPCHK_C(h->iarea32.alloc(nT)); HIPCHK_C(h->iarea32.upload(ia, s));
             HIPCHK_C(h->a15_32.alloc(nT)); HIPCHK_C(h->a15_32.upload(a15, s));
-            HIPCHK_C(hipStreamSynchronize(s));
         }
         const size_t nft = tl.fref.size();
-        std::vector<double> geo(8 * nft);
-        std::vector<float> geo32(8 * nft);
+        geo.resize(8 * nft);
+        geo32.resize(8 * nft);
         for (size_t i = 0; i < nft; ++i) {
             int32_t f = tl.fref[i];
             uint32_t a = m.edgesCells[2 * (size_t)f], b = m.edgesCells[2 * (size_t)f + 1];
@@ -1179,8 +1269,8 @@ int create_impl(const Mesh& mesh_in, const afx_gas* g, const afx_opts* o, const 
         HIPCHK_C(h->t_geo64.alloc(geo.size())); HIPCHK_C(h->t_geo64.upload(geo, s));
         HIPCHK_C(h->t_geo32.alloc(geo32.size())); HIPCHK_C(h->t_geo32.upload(geo32, s));
         {
-            std::vector<float4> g4(2 * nft);
-            std::vector<uint32_t> fck(nft);
+            g4.resize(2 * nft);
+            fck.resize(nft);
             for (size_t i = 0; i < nft; ++i) {
                 g4[2 * i] = make_float4(geo32[i], geo32[nft + i], geo32[2 * nft + i], geo32[3 * nft + i]);
                 g4[2 * i + 1] = make_float4(geo32[4 * nft + i], geo32[5 * nft + i], geo32[6 * nft + i], geo32[7 * nft + i]);
@@ -1197,9 +1287,7 @@ int create_impl(const Mesh& mesh_in, const afx_gas* g, const afx_opts* o, const 
                 HIPCHK_C(h->R32n.alloc(nT)); HIPCHK_C(hipMemsetAsync(h->R32n.p, 0, (size_t)nT * 4, s));
                 HIPCHK_C(h->sa_ad32.alloc(nT)); HIPCHK_C(hipMemsetAsync(h->sa_ad32.p, 0, (size_t)nT * 8, s));
             }
-            HIPCHK_C(hipStreamSynchronize(s));
         }
-        HIPCHK_C(hipStreamSynchronize(s));
         h->tile64_ok = tile_lds_bytes<double>(tl.lmax, tl.gmax, tl.ftmax, h->nv) <= 65536;
         h->tile32_ok = tile_lds_bytes<float>(tl.lmax, tl.gmax, tl.ftmax, h->nv) <= 65536;
     }
