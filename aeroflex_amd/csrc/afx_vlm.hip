@@ -8,7 +8,7 @@
 //     segments per ring (potential.cpp:36-58, solver.cpp:139-254);
 //   - FP32 LU with partial pivoting: a cooperative panel kernel (rows of the
 //     panel in LDS, pivot keys exchanged between workgroups), row
-//     interchanges, a wavefront triangular solve for the block row and the
+//     interchanges with a wavefront triangular solve for the block row, and the
 //     trailing update as a hand-written FP32 GEMM on the matrix cores
 //     (k_gemm_sub_f32, v_mfma_f32_32x32x2f32);
 //   - FP64 iterative refinement on the FP64 matrix with the FP32 factor as
@@ -38,81 +38,94 @@ namespace {
     } while (0)
 
 constexpr int LU_NB = 128;          // panel width = trailing-update depth = solve block
-constexpr int PANEL_R = 120;        // panel rows per workgroup held in LDS (120 x 128 FP32 = 60 KiB)
-constexpr int MAX_PANEL_WG = 512;   // -> n <= 61440
+constexpr int PANEL_R = 256;        // panel rows per workgroup held in LDS (256 x 128 FP32 = 128 of 160 KiB)
+constexpr int MAX_PANEL_WG = 240;   // one to a compute unit, -> n <= 61440
+constexpr int SUB = 16;             // columns of a sub-panel
+constexpr int KEY_STRIDE = 256;     // words of a key buffer: MAX_PANEL_WG in whole wavefronts
 constexpr unsigned SPIN_LIMIT = 1u << 21;
 constexpr double FOUR_PI = 12.566370614359172;
 
 // ------------------------------------------------- panel pivot exchange --
-// Candidate key of one workgroup for one column: |a| bits (31) | row (17) |
-// sequence (16).  The sequence is the 1-based column of the whole matrix, so
-// a key left from an earlier column (or an earlier factorisation: the keys
-// are cleared before each one) never matches.  Row 0x1ffff: no candidate.
+// Candidate of one workgroup for one column as one ordered key: |a| bits (31) |
+// 0x1ffff - row (17) | sequence (16), so the largest key is the largest |a| and,
+// among equals, the lowest row.  The sequence is the 1-based column of the whole
+// matrix: a key left from an earlier column (or an earlier factorisation: the
+// words are cleared before each one) never matches.  Row 0x1ffff: no candidate.
 constexpr unsigned NO_ROW = 0x1ffffu;
 __device__ inline unsigned long long make_key(float absval, unsigned row, unsigned seq) {
     const unsigned long long ab = (unsigned long long)(__float_as_uint(absval) & 0x7fffffffu);
-    return (ab << 33) | ((unsigned long long)(row & NO_ROW) << 16) | (unsigned long long)(seq & 0xffffu);
+    return (ab << 33) | ((unsigned long long)(NO_ROW - row) << 16) | (unsigned long long)(seq & 0xffffu);
 }
+__device__ inline int key_row(unsigned long long k) { return (int)(NO_ROW - ((unsigned)(k >> 16) & NO_ROW)); }
 
-__device__ inline void argmax_combine(float& v, int& i, float ov, int oi) {
-    if (ov > v || (ov == v && oi < i)) { v = ov; i = oi; }
-}
-
-// (|a|, row) as one ordered 64-bit key: larger |a| first, then the lower
-// row; |a| < 0 (no candidate) maps to 0.  |a| >= 0 (or +inf) orders as its bits.
-__device__ inline unsigned long long argmax_key(float v, int i) {
-    return v < 0.f ? 0ull : ((unsigned long long)__float_as_uint(v) << 32) | (unsigned long long)(0xFFFFFFFFu - (unsigned)i);
-}
-__device__ inline void argmax_unkey(unsigned long long k, float& v, int& i) {
-    v = k ? __uint_as_float((unsigned)(k >> 32)) : -1.f;
-    i = k ? (int)(0xFFFFFFFFu - (unsigned)(k & 0xFFFFFFFFull)) : INT_MAX;
-}
-// one step of a wavefront max of 64-bit keys through DPP lane moves
+// maximum of a 32-bit unsigned over the wavefront's 64 lanes, through DPP lane
+// moves: pairs and quads (quad_perm), half rows and rows (mirrors), then rows 1
+// and 3 from lane 15 of the row below (row_bcast15) and rows 2 and 3 from lane 31
+// (row_bcast31); lane 63 then holds it
 template <int CTRL, int ROW_MASK>
-__device__ inline unsigned long long dpp_max_step(unsigned long long k) {
-    const int lo = (int)(unsigned)k, hi = (int)(unsigned)(k >> 32);
-    const int olo = __builtin_amdgcn_update_dpp(lo, lo, CTRL, ROW_MASK, 0xF, false);
-    const int ohi = __builtin_amdgcn_update_dpp(hi, hi, CTRL, ROW_MASK, 0xF, false);
-    const unsigned long long o = ((unsigned long long)(unsigned)ohi << 32) | (unsigned long long)(unsigned)olo;
-    return o > k ? o : k;
+__device__ inline unsigned dpp_max_step(unsigned k) {
+    return max(k, (unsigned)__builtin_amdgcn_update_dpp((int)k, (int)k, CTRL, ROW_MASK, 0xF, false));
 }
-// maximum over the wavefront's 64 lanes, returned in every lane: pairs and
-// quads (quad_perm), half rows and rows (mirrors), then rows 1 and 3 from
-// lane 15 of the row below (row_bcast15) and rows 2 and 3 from lane 31
-// (row_bcast31); lane 63 then holds the maximum
-__device__ inline unsigned long long wave_max_key(unsigned long long k) {
+__device__ inline unsigned wave_max(unsigned k) {
     k = dpp_max_step<0xB1, 0xF>(k);    // quad_perm [1,0,3,2]
     k = dpp_max_step<0x4E, 0xF>(k);    // quad_perm [2,3,0,1]
     k = dpp_max_step<0x141, 0xF>(k);   // row_half_mirror
     k = dpp_max_step<0x140, 0xF>(k);   // row_mirror
     k = dpp_max_step<0x142, 0xA>(k);   // row_bcast15
     k = dpp_max_step<0x143, 0xC>(k);   // row_bcast31
-    const unsigned lo = (unsigned)__builtin_amdgcn_readlane((int)(unsigned)k, 63);
-    const unsigned hi = (unsigned)__builtin_amdgcn_readlane((int)(unsigned)(k >> 32), 63);
-    return ((unsigned long long)hi << 32) | lo;
+    return (unsigned)__builtin_amdgcn_readlane((int)k, 63);
 }
-__device__ inline void wave_argmax(float& v, int& i) { argmax_unkey(wave_max_key(argmax_key(v, i)), v, i); }
+// the lane holding the largest (hi, lo), 0 <= lo; -1 where every hi is zero.
+// The low words are compared only among lanes that share the largest high word.
+__device__ inline int wave_winner(unsigned hi, unsigned lo) {
+    const unsigned top = wave_max(hi);
+    unsigned long long who = __ballot(hi == top);
+    if (__builtin_expect((who & (who - 1ull)) != 0ull, 0)) {
+        if (top == 0u) return -1;
+        const unsigned low = hi == top ? lo : 0u;
+        const unsigned most = wave_max(low);
+        who = __ballot(hi == top && low == most);
+    }
+    return __ffsll(who) - 1;
+}
 
 // --------------------------------------------------- panel factorisation --
-// Unblocked LU with partial pivoting of the m x nbc panel whose top-left
-// entry is A(j0, j0) (column-major, leading dimension lda).  Workgroup w holds
-// panel rows [w R, w R + R) of all nbc columns in LDS.  Per column every
-// workgroup posts its largest |a| (ties: lowest row) as one 64-bit key after
-// the row's values (and the owner of the diagonal row posts that row), then
-// polls the keys of all workgroups: once every key carries this column's
-// sequence, all workgroups know the same pivot without any counter, read the
-// pivot row, perform the interchange on the rows they own, scale their part
-// of the column and update their part of the panel.  The update is ordered so
-// that the next column's key leaves early: column j + 1 is updated first, its
-// candidate found, the two rows to be posted (candidate and diagonal) finish
-// step j, the key is posted, and only then does the rest of the rank-1 update
-// run, while the other workgroups' keys are in flight.  Every element still
-// takes the same operations as in the plain right-looking order.  Keys and
-// rows alternate between two buffers, so posting for column j + 1 cannot
-// overwrite what a slower workgroup still reads for column j (it cannot post
+// LU with partial pivoting of the m x nbc panel whose top-left entry is
+// A(j0, j0) (column-major, leading dimension lda).  Workgroup w holds the panel
+// rows [w R, w R + R) of all nbc columns in LDS, one row per thread, and no row
+// moves before the end: a thread knows its row's position, which the
+// interchanges change, and writes it there.
+//
+// The panel advances in sub-panels of SUB columns, whose entries a thread keeps
+// in registers (the current column in a[0]).  Per column every wave leaves its
+// candidate (key and SUB values) in LDS; wave 0 posts the workgroup's best as
+// value | sequence words and its key, polls the keys of all workgroups and then
+// reads the winner's values: no counter and no fence, since each word carries its
+// sequence.  Only one wave polls: with all four, and every candidate's values in
+// the same round trip, the requests to those few lines took longer than the
+// second trip (690 us a panel of 16 384 rows).  Meanwhile the owner of the last
+// pivot row publishes the rest of it (L to the left inside the sub-panel, the
+// columns to the right as they stand).  After SUB columns every workgroup reads
+// those rows, solves for their U (the substitution is repeated in every
+// workgroup: a column per thread) and updates its own rows of the remaining
+// columns, four rows per lane and a quarter of the columns per wave.  Every
+// element takes the operations of the plain right-looking order.
+//
+// Words alternate between two buffers, so posting for column j + 1 cannot
+// overwrite what a slower workgroup still reads for column j: it cannot post
 // j + 2 before every workgroup has posted j + 1, which each does only after
-// reading column j's pivot row).  Every wait is bounded: a workgroup that
-// polls longer than SPIN_LIMIT raises `abort` and every workgroup returns.
+// reading column j's words; the published rows alternate by sub-panel alike.
+// With one workgroup (m <= R) nothing is exchanged.  Every wait is bounded: a
+// wave that polls longer than SPIN_LIMIT raises `abort` and every workgroup
+// returns.
+//
+// Bound by the latency of that exchange (a word takes about 0.55 us from one
+// compute unit to another) and, with one workgroup, by the column's chain of
+// maximum, LDS exchange, division and update.  Keys go to a mailbox of each
+// reader: polled by all, one row of keys cost 4.4 us a column at 64 workgroups
+// where this costs 2.8.  A panel of 256, 2 048 and 16 384 rows takes 140, 320
+// and 370 us; with a row's 128 columns exchanged and updated per column, 120
+// rows to a workgroup, it took 590, 560 and 690.
 __device__ inline unsigned long long tagged(unsigned seq, float v) {
     return ((unsigned long long)seq << 32) | (unsigned long long)__float_as_uint(v);
 }
@@ -128,196 +141,278 @@ __device__ inline bool wait_tagged(const unsigned long long* p, unsigned seq, fl
     return true;
 }
 
-// the workgroup's candidate (largest |a|, lowest row) from one (|a|, row) per
-// thread; leaves it in rv[0], ri[0] and returns its workgroup-local row, or -1
-__device__ inline int block_candidate(float best, int bi, float* rv, int* ri, int* s_lrow, int rbase) {
-    const int t = threadIdx.x;
-    wave_argmax(best, bi);
-    if ((t & 63) == 0) { rv[t >> 6] = best; ri[t >> 6] = bi; }
-    __syncthreads();
-    if (t == 0) {
-        for (int q = 1; q < 4; ++q) argmax_combine(rv[0], ri[0], rv[q], ri[q]);
-        *s_lrow = ri[0] != INT_MAX ? ri[0] - rbase : -1;
-    }
-    __syncthreads();
-    return *s_lrow;
-}
-
-__global__ __launch_bounds__(256) void k_panel_lu(float* __restrict__ A, int lda, int m, int nbc, int j0,
-                                                  int* __restrict__ ipiv, unsigned long long* keys,
-                                                  unsigned long long* __restrict__ s_vals,
-                                                  unsigned long long* __restrict__ s_diag,
-                                                  unsigned* abort_flag, int* __restrict__ info) {
-    __shared__ float slab[LU_NB * PANEL_R];   // panel column c at slab[c * PANEL_R]
-    __shared__ float urow[LU_NB];
-    __shared__ float rv[4];
-    __shared__ int ri[4];
-    __shared__ int s_lrow, s_win;
-    const int t = threadIdx.x, w = blockIdx.x, nwg = gridDim.x;
+__global__ __launch_bounds__(256, 1) void k_panel_lu(float* __restrict__ A, int lda, int m, int nbc, int j0,
+                                                     int* __restrict__ ipiv, int* __restrict__ src,
+                                                     int* __restrict__ dst, unsigned long long* keys,
+                                                     unsigned long long* vals, unsigned long long* prow,
+                                                     unsigned* abort_flag, int* __restrict__ info) {
+    __shared__ float4 slab4[LU_NB * PANEL_R / 4];     // panel column c at slab[c * PANEL_R]
+    __shared__ float4 U4[(LU_NB - SUB) * SUB / 4];    // U of the sub-panel's rows, column by column
+    __shared__ float4 Ls4[SUB * SUB / 4];             // L of the sub-panel's rows
+    __shared__ float4 cand4[2][4][SUB / 4];           // the waves' candidates
+    __shared__ float4 urow4[2][SUB / 4];              // the pivot row
+    __shared__ unsigned long long wk[2][4], s_win[2];
+    __shared__ int lrow[SUB];                         // the sub-panel's pivot rows in this workgroup
+    __shared__ int s_fail;
+    float* slab = reinterpret_cast<float*>(slab4);
+    float* Ls = reinterpret_cast<float*>(Ls4);
+    const int t = threadIdx.x, lane = t & 63, w = blockIdx.x, nwg = gridDim.x;
+    const int wv = __builtin_amdgcn_readfirstlane(t >> 6);
     const int rbase = w * PANEL_R;
     const int rows = min(PANEL_R, m - rbase);
     float* P = A + (size_t)j0 * lda + j0;
 
-    for (int idx = t; idx < nbc * PANEL_R; idx += 256) {
-        const int c = idx / PANEL_R, r = idx - c * PANEL_R;
-        slab[idx] = r < rows ? P[(size_t)c * lda + rbase + r] : 0.f;
-    }
-    __syncthreads();
-
-    // column j's candidate row (local row lrow, or none) and, from the
-    // workgroup holding panel row j, the diagonal row, as value | sequence
-    // words (a reader checks each word's sequence, so no fence orders them
-    // before the key), then the key
-    auto post = [&](int j, int lrow) {
-        const int par = j & 1;
-        const unsigned seq = (unsigned)(j0 + j + 1);
-        if (lrow >= 0)
-            for (int c = t; c < nbc; c += 256)
-                __hip_atomic_store(&s_vals[((size_t)par * MAX_PANEL_WG + w) * LU_NB + c],
-                                   tagged(seq, slab[c * PANEL_R + lrow]), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-        if (w == j / PANEL_R)
-            for (int c = t; c < nbc; c += 256)
-                __hip_atomic_store(&s_diag[par * LU_NB + c], tagged(seq, slab[c * PANEL_R + (j - rbase)]),
-                                   __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-        if (t == 0) {
-            const unsigned long long key =
-                lrow >= 0 ? make_key(rv[0], (unsigned)ri[0], seq) : make_key(0.f, NO_ROW, seq);
-            __hip_atomic_store(&keys[par * MAX_PANEL_WG + w], key, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-        }
-    };
-    // |a| of a candidate entry; a NaN is taken as the largest
-    auto mag = [](float a) { const float v = fabsf(a); return v == v ? v : INFINITY; };
-
     {
-        const bool live = t < rows;
-        post(0, block_candidate(live ? mag(slab[t]) : -1.f, live ? rbase + t : INT_MAX, rv, ri, &s_lrow, rbase));
+        const float* mine = P + rbase + min(t, rows - 1);
+#pragma unroll 1
+        for (int c = 0; c < LU_NB; c += 32) {
+            float v[32];
+#pragma unroll
+            for (int i = 0; i < 32; ++i) v[i] = mine[(size_t)min(c + i, nbc - 1) * lda];
+#pragma unroll
+            for (int i = 0; i < 32; ++i) slab[(c + i) * PANEL_R + t] = (t < rows && c + i < nbc) ? v[i] : 0.f;
+        }
     }
+    if (t == 0) s_fail = 0;
+    __syncthreads();
+    int pos = t < rows ? rbase + t : -1;   // the row's position in the panel, -1: none
 
-    for (int j = 0; j < nbc; ++j) {
-        const int par = j & 1;
-        const unsigned seq = (unsigned)(j0 + j + 1);
-
-        // gather: every key of this column's sequence
-        float best = -1.f;
-        int bi = INT_MAX;
-        unsigned spins = 0;
-        for (;;) {
-            int ok = 1;
-            best = -1.f;
-            bi = INT_MAX;
-            for (int q = t; q < nwg; q += 256) {
-                const unsigned long long k =
-                    __hip_atomic_load(&keys[par * MAX_PANEL_WG + q], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-                if ((unsigned)(k & 0xffffu) != (seq & 0xffffu)) {
-                    ok = 0;
-                } else {
-                    const unsigned row = (unsigned)(k >> 16) & NO_ROW;
-                    if (row != NO_ROW) argmax_combine(best, bi, __uint_as_float((unsigned)(k >> 33)), (int)row);
+    for (int c0 = 0;; c0 += SUB) {
+        const int sw = min(SUB, nbc - c0), sub = (c0 / SUB) & 1;
+        unsigned long long* rest = prow + (size_t)sub * SUB * LU_NB;
+        auto publish = [&](int jj, int i) {   // row jj of the sub-panel, from its first column on
+            if (i >= 0 && i < nbc - c0)
+                __hip_atomic_store(&rest[jj * LU_NB + i],
+                                   tagged((unsigned)(j0 + c0 + jj + 1), slab[(c0 + i) * PANEL_R + lrow[jj]]),
+                                   __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+        };
+        float a[SUB];   // (columns past the last are zero in the slab)
+#pragma unroll
+        for (int i = 0; i < SUB; ++i) a[i] = slab[(c0 + i) * PANEL_R + t];
+        bool won = false;
+        for (int jj = 0; jj < sw; ++jj) {
+            const int j = c0 + jj, par = j & 1;
+            const unsigned seq = (unsigned)(j0 + j + 1);
+            // the wave's candidate: largest |a|, a NaN taken as the largest
+            // number; rows already chosen offer none
+            const float fa = fabsf(a[0]);
+            const unsigned mag = __float_as_uint(fa == fa ? fa : INFINITY);
+            const int best = wave_winner(pos >= j ? mag + 1u : 0u, NO_ROW - (unsigned)pos);
+            if (lane == max(best, 0)) {
+                wk[par][wv] = best < 0 ? 0ull : make_key(__uint_as_float(mag), (unsigned)pos, seq);
+#pragma unroll
+                for (int i = 0; i < SUB / 4; ++i)
+                    cand4[par][wv][i] = make_float4(a[4 * i], a[4 * i + 1], a[4 * i + 2], a[4 * i + 3]);
+            }
+            __syncthreads();
+            const unsigned long long k0 = wk[par][0], k1 = wk[par][1], k2 = wk[par][2], k3 = wk[par][3];
+            const unsigned long long k01 = k0 > k1 ? k0 : k1, k23 = k2 > k3 ? k2 : k3;
+            const int m01 = k0 > k1 ? 0 : 1, m23 = k2 > k3 ? 2 : 3;
+            const unsigned long long mine = k01 > k23 ? k01 : k23;
+            const int mw = k01 > k23 ? m01 : m23;
+            unsigned long long win = mine;
+            const float4* ur = cand4[par][mw];
+            int fail = 0;
+            if (nwg > 1) {
+                if (wv == 0) {
+                    unsigned long long* kbox = keys + par * KEY_STRIDE;   // reader q's at 2 q KEY_STRIDE
+                    unsigned long long* vbox = vals + par * SUB;          // workgroup q's at 2 q SUB
+                    const unsigned long long post = mine != 0ull ? mine : make_key(0.f, NO_ROW, seq);
+                    for (int q = lane; q < nwg; q += 64)
+                        __hip_atomic_store(&kbox[2 * q * KEY_STRIDE + w], post, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+                    kbox += 2 * w * KEY_STRIDE;
+                    if (lane < SUB)
+                        __hip_atomic_store(&vbox[2 * w * SUB + lane], tagged(seq, reinterpret_cast<const float*>(ur)[lane]),
+                                           __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+                    constexpr int SLOTS = KEY_STRIDE / 64;
+                    unsigned long long kk = 0ull;
+                    int kq = 0;
+                    unsigned spins = 0;
+                    bool late = false;
+                    for (;;) {
+                        bool ok = true;
+                        kk = 0ull;
+#pragma unroll
+                        for (int sl = 0; sl < SLOTS; ++sl) {
+                            if (sl * 64 >= nwg) break;
+                            const int q = sl * 64 + lane;   // (past nwg: words of earlier, taller panels)
+                            unsigned long long k =
+                                __hip_atomic_load(&kbox[q], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+                            ok = ok && (q >= nwg || (unsigned)(k & 0xffffu) == (seq & 0xffffu));
+                            k = q < nwg ? k : 0ull;
+                            kq = k > kk ? q : kq;
+                            kk = k > kk ? k : kk;
+                        }
+                        if (__all(ok)) break;
+                        if (++spins > SPIN_LIMIT ||
+                            ((spins & 63u) == 0u &&
+                             __hip_atomic_load(abort_flag, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) != 0u)) {
+                            late = true;
+                            break;
+                        }
+                    }
+                    if (!late) {
+                        // (every key ends in the sequence: the high words
+                        // hold |a| and the top of the row, never all zero
+                        // while a live row is left)
+                        const int wl = max(0, wave_winner((unsigned)(kk >> 32), (unsigned)kk));
+                        const int wq = __builtin_amdgcn_readlane(kq, wl);
+                        const unsigned lo = (unsigned)__builtin_amdgcn_readlane((int)(unsigned)kk, wl);
+                        const unsigned hi = (unsigned)__builtin_amdgcn_readlane((int)(unsigned)(kk >> 32), wl);
+                        float f = 0.f;
+                        if (lane < SUB) late = !wait_tagged(&vbox[2 * wq * SUB + lane], seq, f);
+                        if (lane < SUB) reinterpret_cast<float*>(urow4[par])[lane] = f;
+                        if (lane == 0) s_win[par] = ((unsigned long long)hi << 32) | lo;
+                    }
+                    if (__any(late)) {
+                        if (lane == 0) {
+                            s_fail = 1;
+                            __hip_atomic_store(abort_flag, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+                        }
+                    }
+                } else if (won) {
+                    publish(jj - 1, t - 64);
+                }
+                __syncthreads();
+                win = s_win[par];
+                ur = urow4[par];
+                fail = s_fail;
+            }
+            float u[SUB];
+#pragma unroll
+            for (int i = 0; i < SUB / 4; ++i) {
+                const float4 v = ur[i];
+                u[4 * i] = v.x; u[4 * i + 1] = v.y; u[4 * i + 2] = v.z; u[4 * i + 3] = v.w;
+            }
+            if (fail) return;
+            won = win == mine;
+            const int p = key_row(win);   // panel-relative pivot position, >= j
+            if (won && pos == p) {
+                lrow[jj] = t;
+                ipiv[j0 + j] = j0 + p;
+            }
+            pos = pos == j ? p : pos == p ? j : pos;
+            const bool upd = __builtin_amdgcn_readfirstlane((int)(__float_as_uint(u[0]) << 1)) != 0;
+            if (__builtin_expect(upd, 1)) {
+                if (pos > j) {
+                    const float l = a[0] / u[0];
+                    slab[j * PANEL_R + t] = l;
+#pragma unroll
+                    for (int i = 0; i + 1 < SUB; ++i) a[i] = a[i + 1] - l * u[i + 1];
+                    a[SUB - 1] = 0.f;
+                }
+            } else {   // a zero pivot leaves the column, whose entries are all zero, alone
+                if (w == 0 && t == 0 && *info == 0) *info = j0 + j + 1;
+                if (pos > j) {
+                    slab[j * PANEL_R + t] = a[0];
+#pragma unroll
+                    for (int i = 0; i + 1 < SUB; ++i) a[i] = a[i + 1];
+                    a[SUB - 1] = 0.f;
                 }
             }
-            if (__syncthreads_and(ok)) break;
-            const int ab = __hip_atomic_load(abort_flag, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) != 0u;
-            if (__syncthreads_or(ab || ++spins > SPIN_LIMIT)) {
-                if (t == 0) __hip_atomic_store(abort_flag, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-                return;
+        }
+        const int rem = nbc - c0 - SUB;
+        __syncthreads();   // lrow and L of the last columns
+        if (nwg > 1 && rem > 0 && won) publish(SUB - 1, t);
+        if (pos >= c0 && pos < c0 + sw) {   // the sub-panel's part of U, as the row stood when it was chosen
+            const int k = pos - c0;
+#pragma unroll
+            for (int i = 0; i < SUB; ++i)
+                if (k + i < sw) slab[(pos + i) * PANEL_R + t] = a[i];
+        }
+        if (rem <= 0) break;
+        // the pivot rows: L of the sub-panel, and the columns right of it
+        float v[SUB];
+        bool ok = true;
+        {
+            const int k = t / SUB, i = t % SUB;
+            float l = 0.f;
+            if (i < k) {
+                if (nwg == 1) l = slab[(c0 + i) * PANEL_R + lrow[k]];
+                else ok = wait_tagged(&rest[k * LU_NB + i], (unsigned)(j0 + c0 + k + 1), l);
             }
-            __builtin_amdgcn_s_sleep(1);
+            Ls[t] = l;
         }
-        wave_argmax(best, bi);
-        if ((t & 63) == 0) { rv[t >> 6] = best; ri[t >> 6] = bi; }
-        __syncthreads();
-        if (t == 0) {
-            for (int q = 1; q < 4; ++q) argmax_combine(rv[0], ri[0], rv[q], ri[q]);
-            s_win = ri[0] == INT_MAX ? j : ri[0];   // every posted row is valid; keep j otherwise
-        }
-        __syncthreads();
-        const int p = s_win;                 // panel-relative pivot row, >= j
-        const int pw = p / PANEL_R, jw = j / PANEL_R;
-        int late = 0;
-        for (int c = t; c < nbc; c += 256) {
-            float v;
-            late |= !wait_tagged(&s_vals[((size_t)par * MAX_PANEL_WG + pw) * LU_NB + c], seq, v);
-            urow[c] = v;
-        }
-        if (w == 0 && t == 0) ipiv[j0 + j] = j0 + p;
-        if (p != j && w == pw)
-            for (int c = t; c < nbc; c += 256) {
-                float v;
-                late |= !wait_tagged(&s_diag[par * LU_NB + c], seq, v);
-                slab[c * PANEL_R + (p - rbase)] = v;
+        if (t < rem) {
+            if (nwg == 1) {
+#pragma unroll
+                for (int k = 0; k < SUB; ++k) v[k] = slab[(c0 + SUB + t) * PANEL_R + lrow[k]];
+            } else {
+                unsigned long long x[SUB];   // all at once; the last few may not be there yet
+#pragma unroll
+                for (int k = 0; k < SUB; ++k)
+                    x[k] = __hip_atomic_load(&rest[k * LU_NB + SUB + t], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+#pragma unroll
+                for (int k = 0; k < SUB; ++k) {
+                    const unsigned seq = (unsigned)(j0 + c0 + k + 1);
+                    v[k] = __uint_as_float((unsigned)x[k]);
+                    if ((unsigned)(x[k] >> 32) != seq) ok = wait_tagged(&rest[k * LU_NB + SUB + t], seq, v[k]) && ok;
+                }
             }
-        if (__syncthreads_or(late)) {
-            if (t == 0) __hip_atomic_store(abort_flag, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-            return;
         }
-        if (p != j && w == jw)
-            for (int c = t; c < nbc; c += 256) slab[c * PANEL_R + (j - rbase)] = urow[c];
+        if (!ok) {
+            s_fail = 1;
+            __hip_atomic_store(abort_flag, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+        }
         __syncthreads();
-        const float piv = urow[j];
-        const bool upd = piv != 0.f;
-        if (!upd && w == 0 && t == 0 && *info == 0) *info = j0 + j + 1;
-        const bool below = t < rows && rbase + t > j;   // rows that step j updates
-        if (j + 1 == nbc) {
-            if (upd && below) slab[j * PANEL_R + t] /= piv;
-            break;
-        }
-        // one thread per row: scale column j, update column j + 1, and offer
-        // the result as column j + 1's candidate
-        float c1 = -1.f;
-        if (below) {
-            float a1 = slab[(j + 1) * PANEL_R + t];
-            if (upd) {
-                const float l = slab[j * PANEL_R + t] / piv;
-                slab[j * PANEL_R + t] = l;
-                a1 -= l * urow[j + 1];
-                slab[(j + 1) * PANEL_R + t] = a1;
+        if (s_fail) return;
+        if (t < rem) {
+#pragma unroll
+            for (int k = 1; k < SUB; ++k)
+#pragma unroll
+                for (int i = 0; i < k; ++i) v[k] -= Ls[k * SUB + i] * v[i];
+#pragma unroll
+            for (int k = 0; k < SUB / 4; ++k) {
+                const float4 x = make_float4(v[4 * k], v[4 * k + 1], v[4 * k + 2], v[4 * k + 3]);
+                U4[t * (SUB / 4) + k] = x;
+                // every workgroup has read its rows of A by now
+                if (w == 0) *reinterpret_cast<float4*>(P + (size_t)(c0 + SUB + t) * lda + c0 + 4 * k) = x;
             }
-            c1 = mag(a1);
         }
-        const int lrow1 = block_candidate(c1, below ? rbase + t : INT_MAX, rv, ri, &s_lrow, rbase);
-        // the rows posted for column j + 1 finish step j first
-        const int drow1 = w == (j + 1) / PANEL_R ? j + 1 - rbase : -1;
-        if (upd)
-            for (int c = j + 2 + t; c < nbc; c += 256) {
-                if (lrow1 >= 0) slab[c * PANEL_R + lrow1] -= slab[j * PANEL_R + lrow1] * urow[c];
-                if (drow1 >= 0 && drow1 != lrow1) slab[c * PANEL_R + drow1] -= slab[j * PANEL_R + drow1] * urow[c];
-            }
         __syncthreads();
-        post(j + 1, lrow1);
-        // the rest of the rank-1 update: two threads per row, the multiplier
-        // in a register and the pivot row broadcast from LDS, columns interleaved
-        if (upd && t < 2 * PANEL_R) {
-            const int r = t < PANEL_R ? t : t - PANEL_R, h2 = t < PANEL_R ? 0 : 1;
-            if (r < rows && rbase + r > j && r != lrow1 && r != drow1) {
-                const float l = slab[j * PANEL_R + r];
+        // rows that are pivots by now take part: what becomes of their remaining
+        // entries is not read again
+        {
+            float4 l[SUB];
+#pragma unroll
+            for (int k = 0; k < SUB; ++k) l[k] = slab4[(c0 + k) * (PANEL_R / 4) + lane];
 #pragma unroll 4
-                for (int c = j + 2 + h2; c < nbc; c += 2) slab[c * PANEL_R + r] -= l * urow[c];
+            for (int c = wv; c < rem; c += 4) {
+                float4 x = slab4[(c0 + SUB + c) * (PANEL_R / 4) + lane];
+                float uc[SUB];
+#pragma unroll
+                for (int k = 0; k < SUB / 4; ++k) {
+                    const float4 y = U4[c * (SUB / 4) + k];
+                    uc[4 * k] = y.x; uc[4 * k + 1] = y.y; uc[4 * k + 2] = y.z; uc[4 * k + 3] = y.w;
+                }
+#pragma unroll
+                for (int k = 0; k < SUB; ++k) {
+                    x.x -= l[k].x * uc[k];
+                    x.y -= l[k].y * uc[k];
+                    x.z -= l[k].z * uc[k];
+                    x.w -= l[k].w * uc[k];
+                }
+                slab4[(c0 + SUB + c) * (PANEL_R / 4) + lane] = x;
             }
         }
         __syncthreads();
     }
-    __syncthreads();
-
-    for (int idx = t; idx < nbc * PANEL_R; idx += 256) {
-        const int c = idx / PANEL_R, r = idx - c * PANEL_R;
-        if (r < rows) P[(size_t)c * lda + rbase + r] = slab[idx];
-    }
-}
-
-// row interchanges of the panel [j0, j0 + nbc) applied to the columns
-// [cbeg, cend) (LAPACK slaswp), one thread per column
-__global__ __launch_bounds__(256) void k_laswp(float* __restrict__ A, int lda, int cbeg, int cend, int j0, int nbc,
-                                               const int* __restrict__ ipiv) {
-    const int col = cbeg + blockIdx.x * 256 + threadIdx.x;
-    if (col >= cend) return;
-    float* cp = A + (size_t)col * lda;
-    for (int k = 0; k < nbc; ++k) {
-        const int p = ipiv[j0 + k];
-        if (p != j0 + k) {
-            const float a = cp[j0 + k];
-            cp[j0 + k] = cp[p];
-            cp[p] = a;
+    // a pivot row's columns right of its sub-panel were written as U above
+    if (pos >= 0) {
+        const int end = pos < nbc ? min(nbc, (pos / SUB + 1) * SUB) : nbc;
+#pragma unroll 1
+        for (int c = 0; c < LU_NB; c += SUB) {
+            float v[SUB];
+#pragma unroll
+            for (int i = 0; i < SUB; ++i) v[i] = slab[(c + i) * PANEL_R + t];
+#pragma unroll
+            for (int i = 0; i < SUB; ++i)
+                if (c + i < end) P[(size_t)(c + i) * lda + pos] = v[i];
         }
+        // the interchanges as a whole: which row each of the panel's first nbc
+        // positions takes, and where the rows that were there go
+        if (pos < nbc) src[j0 + pos] = rbase + t;
+        if (rbase + t < nbc) dst[j0 + rbase + t] = pos;
     }
 }
 
@@ -325,55 +420,79 @@ __device__ inline float readlane_f(float v, int lane) {
     return __int_as_float(__builtin_amdgcn_readlane(__float_as_int(v), lane));
 }
 
-// A(j0:j0+nbc, cbeg:cend) <- L11^-1 A(j0:j0+nbc, cbeg:cend), L11 unit lower
-// (strsm L,L,N,U).  Each wavefront solves TRSM_CPW columns together, two rows
-// per lane, L11 in LDS: the columns' substitution chains are independent, so
-// interleaving them inside the k loop hides the latency of each step
-// (readlane of x_k after its last update) behind the other columns' work.
-constexpr int TRSM_CPW = 8;   // columns per wavefront
-__global__ __launch_bounds__(256) void k_trsm_llnu(float* __restrict__ A, int lda, int cbeg, int cend, int j0,
-                                                   int nbc) {
-    __shared__ float Ls[LU_NB * LU_NB];
+// The row interchanges of the panel [j0, j0 + nbc) applied to the columns
+// [cbeg, cend), and with SOLVE (nbc = 128) the block row solved at once:
+// A(j0:j0+128, cbeg:cend) <- L11^-1 of it, L11 unit lower.  A wavefront takes CPW
+// columns, two of the panel's rows per lane: it gathers the rows that come to the
+// top, solves, and stores them and the rows that they displace (all reads of a
+// column precede its writes, and the column belongs to this wave).  The columns'
+// substitution chains are independent, so CPW of them hide the latency of each
+// step (readlane of x_k after its last update); two are enough where the
+// columns are few and every wave runs at once.  Without SOLVE `extra` is one more
+// column (the permutation, as bits).  Interchanges column by column in their own
+// kernel, a chain of 128 dependent loads, took 9 to 110 us a panel, and the
+// solve with its L11 staged by single words 45.
+template <int CPW, bool SOLVE>
+__global__ __launch_bounds__(256) void k_swap_solve(float* __restrict__ A, int lda, int cbeg, int cend, int j0,
+                                                    int nbc, const int* __restrict__ src,
+                                                    const int* __restrict__ dst, float* __restrict__ extra) {
+    __shared__ float4 Ls4[SOLVE ? LU_NB * LU_NB / 4 : 1];   // column k at Ls[k * LU_NB], zero on and above the diagonal
+    const float* Ls = reinterpret_cast<const float*>(Ls4);
     const int t = threadIdx.x, lane = t & 63, wv = t >> 6;
-    for (int idx = t; idx < nbc * nbc; idx += 256) {
-        const int k = idx / nbc, r = idx - k * nbc;
-        Ls[k * LU_NB + r] = A[(size_t)(j0 + k) * lda + j0 + r];
-    }
-    __syncthreads();
-    const int c0 = cbeg + (blockIdx.x * 4 + wv) * TRSM_CPW;
-    float b0[TRSM_CPW], b1[TRSM_CPW];
+    if (SOLVE) {
 #pragma unroll
-    for (int q = 0; q < TRSM_CPW; ++q) {
-        const float* cp = A + (size_t)(c0 + q) * lda + j0;
-        const bool live = c0 + q < cend;
-        b0[q] = live && lane < nbc ? cp[lane] : 0.f;
-        b1[q] = live && lane + 64 < nbc ? cp[lane + 64] : 0.f;
+        for (int q = 0; q < LU_NB * LU_NB / 4 / 256; ++q) {
+            const int idx = q * 256 + t, k = idx / (LU_NB / 4), r = (idx % (LU_NB / 4)) * 4;
+            float4 v = *reinterpret_cast<const float4*>(A + (size_t)(j0 + k) * lda + j0 + r);
+            v.x = r > k ? v.x : 0.f;
+            v.y = r + 1 > k ? v.y : 0.f;
+            v.z = r + 2 > k ? v.z : 0.f;
+            v.w = r + 3 > k ? v.w : 0.f;
+            Ls4[idx] = v;
+        }
+        __syncthreads();
     }
-    for (int k = 0; k < nbc; ++k) {
-        // only rows r > k (and r < nbc) take -L(r, k) x_k
-        const bool u0 = lane > k && lane < nbc, u1 = lane + 64 > k && lane + 64 < nbc;
-        const float l0 = Ls[k * LU_NB + lane], l1 = Ls[k * LU_NB + lane + 64];
-        if (k < 64) {
+    const int c0 = cbeg + (blockIdx.x * 4 + wv) * CPW, ncol = cend + (extra ? 1 : 0) - c0;
+    if (ncol <= 0) return;
+    const bool in0 = lane < nbc, in1 = lane + 64 < nbc;
+    const int s0 = in0 ? src[j0 + lane] : 0, s1 = in1 ? src[j0 + lane + 64] : 0;
+    const int d0 = in0 ? dst[j0 + lane] : 0, d1 = in1 ? dst[j0 + lane + 64] : 0;
+    float b0[CPW], b1[CPW], o0[CPW], o1[CPW];
 #pragma unroll
-            for (int q = 0; q < TRSM_CPW; ++q) {
+    for (int q = 0; q < CPW; ++q) {
+        const float* cp = c0 + q < cend ? A + (size_t)(c0 + q) * lda + j0 : extra + j0;
+        const bool live = q < ncol;
+        b0[q] = live && in0 ? cp[s0] : 0.f;
+        b1[q] = live && in1 ? cp[s1] : 0.f;
+        o0[q] = live && d0 >= nbc ? cp[lane] : 0.f;
+        o1[q] = live && d1 >= nbc ? cp[lane + 64] : 0.f;
+    }
+    if (SOLVE) {
+#pragma unroll 2
+        for (int k = 0; k < 64; ++k) {
+            const float l0 = Ls[k * LU_NB + lane], l1 = Ls[k * LU_NB + lane + 64];
+#pragma unroll
+            for (int q = 0; q < CPW; ++q) {
                 const float xk = readlane_f(b0[q], k);
-                b0[q] = u0 ? b0[q] - l0 * xk : b0[q];
-                b1[q] = u1 ? b1[q] - l1 * xk : b1[q];
+                b0[q] -= l0 * xk;
+                b1[q] -= l1 * xk;
             }
-        } else {
+        }
+#pragma unroll 2
+        for (int k = 64; k < LU_NB; ++k) {
+            const float l1 = Ls[k * LU_NB + lane + 64];
 #pragma unroll
-            for (int q = 0; q < TRSM_CPW; ++q) {
-                const float xk = readlane_f(b1[q], k - 64);
-                b1[q] = u1 ? b1[q] - l1 * xk : b1[q];
-            }
+            for (int q = 0; q < CPW; ++q) b1[q] -= l1 * readlane_f(b1[q], k - 64);
         }
     }
 #pragma unroll
-    for (int q = 0; q < TRSM_CPW; ++q) {
-        if (c0 + q >= cend) break;
-        float* cp = A + (size_t)(c0 + q) * lda + j0;
-        if (lane < nbc) cp[lane] = b0[q];
-        if (lane + 64 < nbc) cp[lane + 64] = b1[q];
+    for (int q = 0; q < CPW; ++q) {
+        if (q >= ncol) break;
+        float* cp = c0 + q < cend ? A + (size_t)(c0 + q) * lda + j0 : extra + j0;
+        if (in0 && (SOLVE || s0 != lane)) cp[lane] = b0[q];
+        if (in1 && (SOLVE || s1 != lane + 64)) cp[lane + 64] = b1[q];
+        if (d0 >= nbc) cp[d0] = o0[q];
+        if (d1 >= nbc) cp[d1] = o1[q];
     }
 }
 
@@ -402,50 +521,92 @@ __global__ void k_gather_perm(const double* __restrict__ r, const int* __restric
     if (i < n) y[i] = (float)r[perm[i]];
 }
 
-// Inverse of every 128 x 128 diagonal block of the factor, computed in
-// place in LDS column by column (LAPACK strti2): unit lower L -> L^-1 and
-// upper U -> U^-1, blocks past n padded with the identity.  One workgroup per
-// block; the triangular solves apply these with a matrix-vector product
-// instead of a 128-step substitution.
-template <bool LOWER>
-__global__ __launch_bounds__(128) void k_tri_inv(const float* __restrict__ A, int lda, int n,
-                                                 float* __restrict__ Tinv) {
-    __shared__ float X[LU_NB * LU_NB];   // column k at X[k * LU_NB]
-    const int i = threadIdx.x, b0 = blockIdx.x * LU_NB, nb = min(LU_NB, n - b0);
-    for (int k = 0; k < LU_NB; ++k) {
-        float v = (k == i) ? 1.f : 0.f;
-        if (k < nb && i < nb) {
-            const bool keep = LOWER ? (i > k) : (i <= k);
-            v = keep ? A[(size_t)(b0 + k) * lda + b0 + i] : ((k == i) ? 1.f : 0.f);
+// Inverses of the 128 x 128 diagonal blocks of the factor, unit lower L
+// (blockIdx.y = 0) and upper U (1, as the lower U^T), blocks past n padded with
+// the identity; the triangular solves apply these with a matrix-vector product
+// instead of a 128-step substitution.  One workgroup per block, in LDS: the eight
+// 16 x 16 diagonal blocks by substitution, a column per thread, then doubled:
+// the inverse of [A 0; C B] has -B^-1 (C A^-1) below the diagonal, two products
+// in which each of the 256 threads forms S / 16 rows of four columns.  Column by
+// column with two barriers each it took 190 us for L and 350 us for U.
+constexpr int INV_LD = LU_NB + 4;
+template <int S>
+__device__ inline void inv_double(float (*X)[INV_LD], float* W, int t) {
+    constexpr int TR = S / 16;
+    const int p = t / (4 * S), q = t % (4 * S), cg = (q % (S / 4)) * 4, rg = (q / (S / 4)) * TR;
+    const int o = 2 * S * p;
+    float* Wp = W + p * S * S;
+    float s[TR][4];
+    auto product = [&](auto left, auto right) {
+#pragma unroll
+        for (int i = 0; i < TR; ++i)
+#pragma unroll
+            for (int c = 0; c < 4; ++c) s[i][c] = 0.f;
+#pragma unroll 4
+        for (int k = 0; k < S; ++k) {
+            const float4 m = *reinterpret_cast<const float4*>(right(k));
+#pragma unroll
+            for (int i = 0; i < TR; ++i) {
+                const float l = left(rg + i, k);
+                s[i][0] += l * m.x;
+                s[i][1] += l * m.y;
+                s[i][2] += l * m.z;
+                s[i][3] += l * m.w;
+            }
         }
-        X[k * LU_NB + i] = v;
+    };
+    product([&](int r, int k) { return X[o + S + r][o + k]; }, [&](int k) { return &X[o + k][o + cg]; });
+#pragma unroll
+    for (int i = 0; i < TR; ++i)
+        *reinterpret_cast<float4*>(&Wp[(rg + i) * S + cg]) = make_float4(s[i][0], s[i][1], s[i][2], s[i][3]);
+    __syncthreads();
+    product([&](int r, int k) { return X[o + S + r][o + S + k]; }, [&](int k) { return &Wp[k * S + cg]; });
+#pragma unroll
+    for (int i = 0; i < TR; ++i)
+        *reinterpret_cast<float4*>(&X[o + S + rg + i][o + cg]) = make_float4(-s[i][0], -s[i][1], -s[i][2], -s[i][3]);
+    __syncthreads();
+}
+
+__global__ __launch_bounds__(256) void k_tri_inv(const float* __restrict__ A, int lda, int n, float* __restrict__ Linv,
+                                                 float* __restrict__ Uinv) {
+    __shared__ alignas(16) float X[LU_NB][INV_LD];   // row r of the lower triangle
+    __shared__ alignas(16) float W[64 * 64];
+    const int t = threadIdx.x, b0 = blockIdx.x * LU_NB, nb = min(LU_NB, n - b0);
+    const bool upper = blockIdx.y == 1;
+#pragma unroll 16
+    for (int q = 0; q < LU_NB * LU_NB / 256; ++q) {
+        const int idx = q * 256 + t, k = idx / LU_NB, i = idx % LU_NB;   // row i, column k of the factor
+        float v = k == i ? 1.f : 0.f;
+        if (k < nb && i < nb && (upper ? i <= k : i > k)) v = A[(size_t)(b0 + k) * lda + b0 + i];
+        if (upper) X[k][i] = v;
+        else X[i][k] = v;
     }
     __syncthreads();
-    if (LOWER) {
-        for (int j = LU_NB - 2; j >= 0; --j) {
-            float s = 0.f;
-            if (i > j) {
-                s = X[j * LU_NB + i];
-                for (int k = j + 1; k < i; ++k) s += X[k * LU_NB + i] * X[j * LU_NB + k];
-            }
-            __syncthreads();
-            if (i > j) X[j * LU_NB + i] = -s;
-            __syncthreads();
-        }
-    } else {
-        for (int j = 0; j < LU_NB; ++j) {
-            const float d = 1.f / X[j * LU_NB + j];
-            float s = 0.f;
-            if (i < j)
-                for (int k = i; k < j; ++k) s += X[k * LU_NB + i] * X[j * LU_NB + k];
-            __syncthreads();
-            if (i < j) X[j * LU_NB + i] = -d * s;
-            if (i == j) X[j * LU_NB + j] = d;
-            __syncthreads();
+    float x[16];
+    const int o = (t / 16) * 16, c = t % 16;
+    if (t < LU_NB) {
+#pragma unroll
+        for (int r = 0; r < 16; ++r) {
+            float v = r == c ? 1.f : 0.f;
+#pragma unroll
+            for (int k = 0; k < r; ++k) v -= X[o + r][o + k] * x[k];
+            x[r] = upper ? v * (1.f / X[o + r][o + r]) : v;
         }
     }
-    float* out = Tinv + (size_t)blockIdx.x * LU_NB * LU_NB;
-    for (int k = 0; k < LU_NB; ++k) out[k * LU_NB + i] = X[k * LU_NB + i];
+    __syncthreads();
+    if (t < LU_NB)
+#pragma unroll
+        for (int r = 0; r < 16; ++r) X[o + r][o + c] = x[r];
+    __syncthreads();
+    inv_double<16>(X, W, t);
+    inv_double<32>(X, W, t);
+    inv_double<64>(X, W, t);
+    float* out = (upper ? Uinv : Linv) + (size_t)blockIdx.x * LU_NB * LU_NB;
+#pragma unroll 8
+    for (int q = 0; q < LU_NB * LU_NB / 256; ++q) {
+        const int idx = q * 256 + t, k = idx / LU_NB, i = idx % LU_NB;
+        out[idx] = upper ? X[k][i] : X[i][k];
+    }
 }
 
 // Blocked triangular solve in one launch (y <- L^-1 y or U^-1 y in place).
@@ -826,6 +987,8 @@ __global__ void k_forces_stations(const double* __restrict__ corner, const doubl
 // MFMAs.  Operand layout of the 32x32x2 instruction: lane l supplies
 // A[l % 32][l / 32] and B[l / 32][l % 32] of the 32 x 2 and 2 x 32 slices;
 // accumulator element v of lane l is C[8 (v / 4) + 4 (l / 32) + v % 4][l % 32].
+// The product is formed transposed (B's columns as the instruction's rows), so
+// that a store of one element by 32 lanes is 32 consecutive rows of a column.
 // Blocks map to tiles XCD-aware (consecutive tiles of one XCD share A rows).
 constexpr int GM_TM = 128, GM_TN = 128, GM_TK = 16;
 constexpr int GM_LDB = GM_TN + 4;
@@ -855,21 +1018,12 @@ __global__ void __launch_bounds__(256) k_gemm_sub_f32(const float* __restrict__ 
     float ra[8], rb[8];
     auto load = [&](int kb) {
         const int ka = kb + a_k, kbb = kb + b_k;
-        if (full && kb + GM_TK <= k) {
-            const float4* pa = reinterpret_cast<const float4*>(A + (size_t)ka * ld + row0 + a_r);
-            const float4 a0 = pa[0], a1 = pa[1];
-            ra[0] = a0.x; ra[1] = a0.y; ra[2] = a0.z; ra[3] = a0.w; ra[4] = a1.x; ra[5] = a1.y; ra[6] = a1.z; ra[7] = a1.w;
-            const float4* pb = reinterpret_cast<const float4*>(B + (size_t)(col0 + b_c) * ld + kbb);
-            const float4 b0 = pb[0], b1 = pb[1];
-            rb[0] = b0.x; rb[1] = b0.y; rb[2] = b0.z; rb[3] = b0.w; rb[4] = b1.x; rb[5] = b1.y; rb[6] = b1.z; rb[7] = b1.w;
-        } else {
-            for (int i = 0; i < 8; ++i) {
-                const int r = row0 + a_r + i;
-                ra[i] = (r < m && ka < k) ? A[(size_t)ka * ld + r] : 0.f;
-                const int c = col0 + b_c, kk = kbb + i;
-                rb[i] = (c < n && kk < k) ? B[(size_t)c * ld + kk] : 0.f;
-            }
-        }
+        const float4* pa = reinterpret_cast<const float4*>(A + (size_t)ka * ld + row0 + a_r);
+        const float4 a0 = pa[0], a1 = pa[1];
+        ra[0] = a0.x; ra[1] = a0.y; ra[2] = a0.z; ra[3] = a0.w; ra[4] = a1.x; ra[5] = a1.y; ra[6] = a1.z; ra[7] = a1.w;
+        const float4* pb = reinterpret_cast<const float4*>(B + (size_t)min(col0 + b_c, n - 1) * ld + kbb);
+        const float4 b0 = pb[0], b1 = pb[1];
+        rb[0] = b0.x; rb[1] = b0.y; rb[2] = b0.z; rb[3] = b0.w; rb[4] = b1.x; rb[5] = b1.y; rb[6] = b1.z; rb[7] = b1.w;
     };
     auto store = [&](int buf) {
         float4* da = reinterpret_cast<float4*>(&As[buf][a_k][a_r]);
@@ -893,10 +1047,10 @@ __global__ void __launch_bounds__(256) k_gemm_sub_f32(const float* __restrict__ 
         for (int kk = 0; kk < GM_TK; kk += 2) {
             const float a0 = As[buf][kk + lk][wm + lr], a1 = As[buf][kk + lk][wm + 32 + lr];
             const float b0 = Bs[buf][kk + lk][wn + lr], b1 = Bs[buf][kk + lk][wn + 32 + lr];
-            acc[0][0] = __builtin_amdgcn_mfma_f32_32x32x2f32(a0, b0, acc[0][0], 0, 0, 0);
-            acc[0][1] = __builtin_amdgcn_mfma_f32_32x32x2f32(a0, b1, acc[0][1], 0, 0, 0);
-            acc[1][0] = __builtin_amdgcn_mfma_f32_32x32x2f32(a1, b0, acc[1][0], 0, 0, 0);
-            acc[1][1] = __builtin_amdgcn_mfma_f32_32x32x2f32(a1, b1, acc[1][1], 0, 0, 0);
+            acc[0][0] = __builtin_amdgcn_mfma_f32_32x32x2f32(b0, a0, acc[0][0], 0, 0, 0);
+            acc[0][1] = __builtin_amdgcn_mfma_f32_32x32x2f32(b1, a0, acc[0][1], 0, 0, 0);
+            acc[1][0] = __builtin_amdgcn_mfma_f32_32x32x2f32(b0, a1, acc[1][0], 0, 0, 0);
+            acc[1][1] = __builtin_amdgcn_mfma_f32_32x32x2f32(b1, a1, acc[1][1], 0, 0, 0);
         }
         if (c + 1 < nk) {
             store(buf ^ 1);   // the other buffer: its last readers finished before the previous barrier
@@ -904,22 +1058,23 @@ __global__ void __launch_bounds__(256) k_gemm_sub_f32(const float* __restrict__ 
         __syncthreads();
     }
     // C -= acc
+#pragma unroll
     for (int i = 0; i < 2; ++i)
+#pragma unroll
         for (int j = 0; j < 2; ++j) {
-            const int col = col0 + wn + j * 32 + lr;
-            for (int g = 0; g < 4; ++g) {
-                const int row = row0 + wm + i * 32 + 8 * g + 4 * lk;   // rows row .. row + 3
-                if (full) {
-                    float4* pc = reinterpret_cast<float4*>(C + (size_t)col * ld + row);
-                    float4 cv = *pc;
-                    cv.x -= acc[i][j][4 * g + 0];
-                    cv.y -= acc[i][j][4 * g + 1];
-                    cv.z -= acc[i][j][4 * g + 2];
-                    cv.w -= acc[i][j][4 * g + 3];
-                    *pc = cv;
-                } else if (col < n) {
-                    for (int v = 0; v < 4; ++v)
-                        if (row + v < m) C[(size_t)col * ld + row + v] -= acc[i][j][4 * g + v];
+            const int row = row0 + wm + i * 32 + lr, cb = col0 + wn + j * 32 + 4 * lk;
+            float* pc = C + (size_t)cb * ld + row;
+            if (full) {
+                float cv[16];
+#pragma unroll
+                for (int v = 0; v < 16; ++v) cv[v] = pc[(size_t)(8 * (v / 4) + v % 4) * ld];
+#pragma unroll
+                for (int v = 0; v < 16; ++v) pc[(size_t)(8 * (v / 4) + v % 4) * ld] = cv[v] - acc[i][j][v];
+            } else {
+#pragma unroll
+                for (int v = 0; v < 16; ++v) {
+                    const int dc = 8 * (v / 4) + v % 4;
+                    if (row < m && cb + dc < n) pc[(size_t)dc * ld] -= acc[i][j][v];
                 }
             }
         }
@@ -933,14 +1088,15 @@ hipError_t launch_gemm_sub_f32(hipStream_t s, const float* A, const float* B, fl
     return hipGetLastError();
 }
 
-__global__ void k_panel_reset(unsigned long long* keys, unsigned long long* s_vals, unsigned long long* s_diag,
-                              unsigned* abort_flag, unsigned* trsv_abort, int* info) {
+__global__ void k_panel_reset(unsigned long long* keys, unsigned long long* vals, unsigned long long* prow, int* perm,
+                              int n, int nwg, unsigned* abort_flag, unsigned* trsv_abort, int* info) {
     const int stride = gridDim.x * blockDim.x, i0 = blockIdx.x * blockDim.x + threadIdx.x;
-    for (int q = i0; q < 2 * MAX_PANEL_WG; q += stride) keys[q] = 0ull;
-    // the row words carry the column sequence j0 + j + 1, which repeats from one
-    // factorisation to the next: clear them with the keys
-    for (int q = i0; q < 2 * MAX_PANEL_WG * LU_NB; q += stride) s_vals[q] = 0ull;
-    for (int q = i0; q < 2 * LU_NB; q += stride) s_diag[q] = 0ull;
+    // the words carry the column sequence j0 + j + 1, which repeats from one
+    // factorisation to the next
+    for (int q = i0; q < 2 * KEY_STRIDE * nwg; q += stride) keys[q] = 0ull;
+    for (int q = i0; q < 2 * SUB * nwg; q += stride) vals[q] = 0ull;
+    for (int q = i0; q < 2 * SUB * LU_NB; q += stride) prow[q] = 0ull;
+    for (int q = i0; q < n; q += stride) perm[q] = q;
     if (i0 == 0) {
         *abort_flag = 0u;
         *trsv_abort = 0u;   // a new factorisation also re-arms the triangular solves
@@ -962,16 +1118,17 @@ struct afx_dense {
     // look-ahead of the factorisation: the update of the columns past the
     // next panel runs on s2 while s factors that panel
     hipStream_t s2 = nullptr;
-    hipEvent_t ev_panel = nullptr, ev_far = nullptr;
+    hipEvent_t ev_panel = nullptr, ev_near = nullptr, ev_far = nullptr;
     double* A64 = nullptr;     // row-major n x n
     float* A32 = nullptr;      // column-major lda x n, LU in place
-    int* ipiv = nullptr;
+    int* ipiv = nullptr;       // followed by src and dst
     int* perm = nullptr;
     double *b = nullptr, *x = nullptr, *r = nullptr, *rowabs = nullptr, *norms = nullptr;
     float* y = nullptr;
-    unsigned long long* keys = nullptr;
-    unsigned long long* s_vals = nullptr;   // candidate rows, value | column sequence
-    unsigned long long* s_diag = nullptr;
+    int *src = nullptr, *dst = nullptr;   // every panel's interchanges as a whole (k_panel_lu)
+    unsigned long long* keys = nullptr;   // candidates of the panel's workgroups, followed by vals and prow
+    unsigned long long* vals = nullptr;   // and their values, value | column sequence
+    unsigned long long* prow = nullptr;   // pivot rows of a sub-panel, value | column sequence
     unsigned* pabort = nullptr;
     int* info = nullptr;
     float *Linv = nullptr, *Uinv = nullptr;   // inverses of the 128 x 128 diagonal blocks
@@ -983,11 +1140,12 @@ struct afx_dense {
     bool factored = false;
     ~afx_dense() {
         for (void* p : {(void*)A64, (void*)A32, (void*)ipiv, (void*)perm, (void*)b, (void*)x, (void*)r,
-                        (void*)rowabs, (void*)norms, (void*)y, (void*)keys, (void*)s_vals,
-                        (void*)s_diag, (void*)pabort, (void*)info, (void*)Linv, (void*)Uinv, (void*)tk,
+                        (void*)rowabs, (void*)norms, (void*)y, (void*)keys,
+                        (void*)pabort, (void*)info, (void*)Linv, (void*)Uinv, (void*)tk,
                         (void*)yx, (void*)abort})
             if (p) (void)hipFree(p);
         if (ev_panel) (void)hipEventDestroy(ev_panel);
+        if (ev_near) (void)hipEventDestroy(ev_near);
         if (ev_far) (void)hipEventDestroy(ev_far);
         if (s) (void)hipStreamDestroy(s);
         if (s2) (void)hipStreamDestroy(s2);
@@ -1010,11 +1168,14 @@ int dense_init(afx_dense* h, int n) {
     VCHK(hipStreamCreateWithFlags(&h->s, hipStreamNonBlocking));
     VCHK(hipStreamCreateWithFlags(&h->s2, hipStreamNonBlocking));
     VCHK(hipEventCreateWithFlags(&h->ev_panel, hipEventDisableTiming));
+    VCHK(hipEventCreateWithFlags(&h->ev_near, hipEventDisableTiming));
     VCHK(hipEventCreateWithFlags(&h->ev_far, hipEventDisableTiming));
     const size_t nn = (size_t)n;
     VCHK(dalloc(&h->A64, nn * nn));
-    VCHK(dalloc(&h->A32, (size_t)h->lda * nn));
-    VCHK(dalloc(&h->ipiv, nn));
+    VCHK(dalloc(&h->A32, (size_t)h->lda * nn + LU_NB));   // (the update reads whole tiles of rows)
+    VCHK(dalloc(&h->ipiv, 3 * nn));
+    h->src = h->ipiv + nn;
+    h->dst = h->src + nn;
     VCHK(dalloc(&h->perm, nn));
     VCHK(dalloc(&h->b, nn));
     VCHK(dalloc(&h->x, nn));
@@ -1022,9 +1183,10 @@ int dense_init(afx_dense* h, int n) {
     VCHK(dalloc(&h->rowabs, nn));
     VCHK(dalloc(&h->norms, 4));
     VCHK(dalloc(&h->y, nn));
-    VCHK(dalloc(&h->keys, 2 * MAX_PANEL_WG));
-    VCHK(dalloc(&h->s_vals, (size_t)2 * MAX_PANEL_WG * LU_NB));
-    VCHK(dalloc(&h->s_diag, 2 * LU_NB));
+    const size_t nwg = (nn + PANEL_R - 1) / PANEL_R;
+    VCHK(dalloc(&h->keys, 2 * nwg * KEY_STRIDE + 2 * nwg * SUB + 2 * SUB * LU_NB));
+    h->vals = h->keys + 2 * nwg * KEY_STRIDE;
+    h->prow = h->vals + 2 * nwg * SUB;
     VCHK(dalloc(&h->pabort, 1));
     VCHK(dalloc(&h->info, 1));
     h->nblk = (n + LU_NB - 1) / LU_NB;
@@ -1047,76 +1209,76 @@ int dense_factor(afx_dense* h, int32_t* info_out) {
     dim3 tg((n + 63) / 64, (n + 63) / 64);
     k_to_cm32<<<tg, 256, 0, s>>>(h->A64, n, h->A32, lda);
     VCHK(hipGetLastError());
-    k_panel_reset<<<64, 256, 0, s>>>(h->keys, h->s_vals, h->s_diag, h->pabort, h->abort, h->info);
+    k_panel_reset<<<64, 256, 0, s>>>(h->keys, h->vals, h->prow, h->perm, n, (n + PANEL_R - 1) / PANEL_R, h->pabort, h->abort, h->info);
     VCHK(hipGetLastError());
     // Right-looking blocked LU with a look-ahead of one panel.  After panel
-    // k (columns [j0, c1)) is factored on s, s2 swaps the rows of the columns
-    // left of it and past the next panel ([0, j0) and [c2, n)) and applies
-    // step k's update to [c2, n), while s applies it to the next panel's
-    // columns [c1, c2) alone and factors that panel.  s waits for the far
-    // update of step k - 1 before its own update of step k, since that one
-    // brought [c1, c2) up to step k - 1; the column sets the two streams touch
-    // at the same time are disjoint.
+    // k (columns [j0, c1)) is factored on s, s2 interchanges the rows of the
+    // columns past the next panel ([c2, n)), solves their block row and applies
+    // step k's update, while s does the same for the next panel's columns
+    // [c1, c2) alone and factors that panel.  s waits for the far update of
+    // step k - 1 before its own of step k, since that one brought [c1, c2) up to
+    // step k - 1; the column sets the two streams touch at the same time are
+    // disjoint.  The far product is held back until the near one is done and
+    // behind the interchanges of the columns left of the panel (and of the
+    // permutation), so that the next panel's workgroups, which need a compute
+    // unit's LDS each, find their places before it fills the chip: behind it a
+    // panel of 64 workgroups waited out all of the product (1300 us for one of
+    // 560).
     float* A = h->A32;
     for (int j0 = 0; j0 < n; j0 += LU_NB) {
         const int nbc = std::min(LU_NB, n - j0);
         const int m = n - j0;
         const int nwg = (m + PANEL_R - 1) / PANEL_R;
-        int ldai = lda, mi = m, nbci = nbc, j0i = j0;
-        void* args[] = {&A, &ldai, &mi, &nbci, &j0i, &h->ipiv, &h->keys, &h->s_vals, &h->s_diag, &h->pabort,
-                        &h->info};
-        VCHK(hipLaunchCooperativeKernel((const void*)k_panel_lu, dim3(nwg), dim3(256), args, 0, s));
-        VCHK(hipEventRecord(h->ev_panel, s));
+        if (nwg == 1) {   // waits for no other workgroup: needs no cooperative launch
+            k_panel_lu<<<1, 256, 0, s>>>(A, lda, m, nbc, j0, h->ipiv, h->src, h->dst, h->keys, h->vals, h->prow,
+                                         h->pabort, h->info);
+            VCHK(hipGetLastError());
+        } else {
+            int ldai = lda, mi = m, nbci = nbc, j0i = j0;
+            void* args[] = {&A,       &ldai,    &mi,      &nbci,    &j0i,       &h->ipiv, &h->src,
+                            &h->dst,  &h->keys, &h->vals, &h->prow, &h->pabort, &h->info};
+            VCHK(hipLaunchCooperativeKernel((const void*)k_panel_lu, dim3(nwg), dim3(256), args, 0, s));
+        }
         const int c1 = j0 + nbc, c2 = std::min(n, c1 + LU_NB), rest = n - c1;
         const float* A21 = A + (size_t)j0 * lda + c1;
-        auto update = [&](hipStream_t st, int cb, int ce) -> int {
-            k_laswp<<<(ce - cb + 255) / 256, 256, 0, st>>>(A, lda, cb, ce, j0, nbc, h->ipiv);
-            k_trsm_llnu<<<(ce - cb + 4 * TRSM_CPW - 1) / (4 * TRSM_CPW), 256, 0, st>>>(A, lda, cb, ce, j0, nbc);
-            VCHK(hipGetLastError());
-            VCHK(launch_gemm_sub_f32(st, A21, A + (size_t)cb * lda + j0, A + (size_t)cb * lda + c1, lda, rest, ce - cb,
-                                     nbc));
-            return AFX_OK;
-        };
+        VCHK(hipEventRecord(h->ev_panel, s));
         VCHK(hipStreamWaitEvent(h->s2, h->ev_panel, 0));
-        if (j0 > 0) {
-            k_laswp<<<(j0 + 255) / 256, 256, 0, h->s2>>>(A, lda, 0, j0, j0, nbc, h->ipiv);
-            VCHK(hipGetLastError());
-        }
         if (c2 < n) {
-            const int rc = update(h->s2, c2, n);
-            if (rc != AFX_OK) return rc;
+            constexpr int CPW = 8;
+            k_swap_solve<CPW, true><<<(n - c2 + 4 * CPW - 1) / (4 * CPW), 256, 0, h->s2>>>(A, lda, c2, n, j0, nbc, h->src,
+                                                                                        h->dst, nullptr);
+            VCHK(hipGetLastError());
         }
         if (c1 < n) {
+            constexpr int CPW = 2;
             if (j0 > 0) VCHK(hipStreamWaitEvent(s, h->ev_far, 0));   // step k - 1 on [c1, c2)
-            const int rc = update(s, c1, c2);
-            if (rc != AFX_OK) return rc;
+            k_swap_solve<CPW, true><<<(c2 - c1 + 4 * CPW - 1) / (4 * CPW), 256, 0, s>>>(A, lda, c1, c2, j0, nbc, h->src,
+                                                                                     h->dst, nullptr);
+            VCHK(hipGetLastError());
+            VCHK(launch_gemm_sub_f32(s, A21, A + (size_t)c1 * lda + j0, A + (size_t)c1 * lda + c1, lda, rest, c2 - c1,
+                                     nbc));
+        }
+        VCHK(hipEventRecord(h->ev_near, s));
+        VCHK(hipStreamWaitEvent(h->s2, h->ev_near, 0));
+        k_swap_solve<1, false><<<(j0 + 1 + 3) / 4, 256, 0, h->s2>>>(A, lda, 0, j0, j0, nbc, h->src, h->dst,
+                                                                    reinterpret_cast<float*>(h->perm));
+        VCHK(hipGetLastError());
+        if (c2 < n) {
+            VCHK(launch_gemm_sub_f32(h->s2, A21, A + (size_t)c2 * lda + j0, A + (size_t)c2 * lda + c1, lda, rest, n - c2,
+                                     nbc));
         }
         VCHK(hipEventRecord(h->ev_far, h->s2));
     }
+    k_tri_inv<<<dim3(h->nblk, 2), 256, 0, s>>>(h->A32, lda, n, h->Linv, h->Uinv);
+    VCHK(hipGetLastError());
+    VCHK(hipEventRecord(h->ev_far, h->s2));
     VCHK(hipStreamWaitEvent(s, h->ev_far, 0));
     unsigned aborted = 0;
     int info = 0;
     VCHK(hipMemcpyAsync(&aborted, h->pabort, sizeof(unsigned), hipMemcpyDeviceToHost, s));
     VCHK(hipMemcpyAsync(&info, h->info, sizeof(int), hipMemcpyDeviceToHost, s));
-    std::vector<int> ipiv(n);
-    VCHK(hipMemcpyAsync(ipiv.data(), h->ipiv, n * sizeof(int), hipMemcpyDeviceToHost, s));
     VCHK(hipStreamSynchronize(s));
     if (aborted) return api_fail(AFX_EHIP, "LU panel: pivot exchange timed out (workgroups not co-resident)");
-    // P b = b[perm]: the interchanges applied in order to the identity
-    std::vector<int> perm(n);
-    for (int i = 0; i < n; ++i) perm[i] = i;
-    for (int k = 0; k < n; ++k) {
-        const int p = ipiv[k];
-        if (p < k || p >= n) return api_fail(AFX_EHIP, "LU panel produced an invalid pivot");
-        std::swap(perm[k], perm[p]);
-    }
-    VCHK(hipMemcpyAsync(h->perm, perm.data(), n * sizeof(int), hipMemcpyHostToDevice, s));
-    if (!info) {
-        k_tri_inv<true><<<h->nblk, LU_NB, 0, s>>>(h->A32, lda, n, h->Linv);
-        k_tri_inv<false><<<h->nblk, LU_NB, 0, s>>>(h->A32, lda, n, h->Uinv);
-        VCHK(hipGetLastError());
-    }
-    VCHK(hipStreamSynchronize(s));
     if (info_out) *info_out = info;
     h->factored = info == 0;
     if (info) return api_fail(AFX_EARG, "matrix is singular in FP32: zero pivot at column " + std::to_string(info - 1));

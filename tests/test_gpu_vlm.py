@@ -73,6 +73,43 @@ def test_lu_factor_backward_error_and_pivoting(vlm, n):
     assert piv[0] == np.argmax(np.abs(A32[:, 0]))  # first pivot is the column maximum
 
 
+# one row group and more, sub-panels of 16 columns whole and ragged, a row group
+# of one row, a last panel of one column; entries of few values, so that the
+# largest is tied within and across row groups
+@pytest.mark.parametrize("n", [15, 16, 17, 33, 127, 255, 256, 257, 385, 513, 600, 1025])
+@pytest.mark.parametrize("ties", [False, True])
+def test_first_panel_takes_the_plain_right_looking_steps(vlm, n, ties):
+    rng = np.random.default_rng(n)
+    A = rng.integers(-3, 4, size=(n, n)).astype(float) if ties else rng.normal(size=(n, n))
+    A[np.arange(n), np.arange(n)] += 0.5 if ties else 0.0
+    d = vlm.Dense(n)
+    d.set(A)
+    try:
+        d.factor()
+    except vlm.VlmError:
+        assert ties   # small integer matrices can be singular
+    lu, piv = d.lu()
+    nb = min(n, 128)
+    P = A[:, :nb].astype(np.float32)
+    want = np.zeros(nb, int)
+    for j in range(nb):
+        p = j + int(np.argmax(np.abs(P[j:, j])))   # the lowest of equal rows
+        want[j] = p
+        P[[j, p]] = P[[p, j]]
+        if P[j, j] != 0.0:
+            P[j + 1:, j] /= P[j, j]
+            # one rounding per element, as the fused multiply-add
+            P[j + 1:, j + 1:] = (P[j + 1:, j + 1:].astype(float)
+                                 - np.outer(P[j + 1:, j].astype(float), P[j, j + 1:].astype(float))).astype(np.float32)
+    assert np.array_equal(piv[:nb], want)
+    # later panels only interchange the rows below these columns' first nb
+    assert np.array_equal(lu[:nb, :nb], P[:nb])
+    perm = np.arange(n)
+    for k in range(nb, n):
+        perm[[k, piv[k]]] = perm[[piv[k], k]]
+    assert np.array_equal(lu[nb:, :nb], P[perm[nb:]])
+
+
 @pytest.mark.parametrize("n,cond", [(300, 1e2), (700, 1e6), (1537, 1e3)])
 def test_refined_solve_matches_fp64(vlm, n, cond):
     print(f"[vlm] refine n={n} cond={cond:g}", flush=True)
