@@ -514,12 +514,13 @@ __global__ __launch_bounds__(256) void k_to_cm32(const double* __restrict__ A64,
 }
 
 // ------------------------------------------------- triangular solves ----
-// y = (float) r[perm]  (P applied to the FP64 residual)
-__global__ void k_gather_perm(const double* __restrict__ r, const int* __restrict__ perm, float* __restrict__ y,
-                              int n) {
-    const int i = blockIdx.x * blockDim.x + threadIdx.x;
-    if (i < n) y[i] = (float)r[perm[i]];
-}
+// State of a refined solve, kept on the device so that its steps can be queued
+// without waiting for each: the kernels of a step return at once when done.
+struct SolveState {
+    double anorm, prev, contraction, backward;
+    int it, converged, done;
+    unsigned aborted;
+};
 
 // Inverses of the 128 x 128 diagonal blocks of the factor, unit lower L
 // (blockIdx.y = 0) and upper U (1, as the lower U^T), blocks past n padded with
@@ -609,44 +610,74 @@ __global__ __launch_bounds__(256) void k_tri_inv(const float* __restrict__ A, in
     }
 }
 
-// Blocked triangular solve in one launch (y <- L^-1 y or U^-1 y in place).
-// Each workgroup takes a ticket; ticket t owns block row t (forward) or
-// nblk - 1 - t (backward), so a workgroup only waits on blocks owned by
-// workgroups that started before it.  It accumulates T(b, c) x_c over the
-// blocks c it depends on (the block of T is loaded before the wait), applies
-// the inverse of its diagonal block and publishes x_b.  Publication is one
-// 64-bit word per element, the value in the low half and the call's epoch in
-// the high half: a consumer thread polls the element it needs, so the value
-// arrives with its own flag in a single round trip (no separate flag, fence
-// or reload).  Every wait is bounded (abort flag, the grid still drains).
+// Blocked triangular solve in one launch: forward y <- L^-1 P r (r in FP64,
+// rounded to FP32), backward x += U^-1 y (x in FP64).  Each workgroup takes a
+// ticket; ticket t owns block row t (forward) or nblk - 1 - t (backward), so a
+// workgroup only waits on blocks owned by workgroups that started before it.  It
+// accumulates T(b, c) x_c over the blocks c it depends on, applies the inverse of
+// its diagonal block and publishes x_b.  Publication is one 64-bit word per
+// element, the value in the low half and the call's epoch in the high half: a
+// consumer thread polls the element it needs, so the value arrives with its own
+// flag in a single round trip (no separate flag, fence or reload).  Every wait is
+// bounded (abort flag, the grid still drains).
+//
+// Bound by the chain of blocks: a message between compute units and two
+// products of a 128 x 128 block per link.  A row of the block is shared by four
+// threads, 32 columns each in two sums, and the next block's columns are
+// loaded before the wait for this one's x: at order 1 280 and 16 384 the forward
+// solve takes 11 and 198 us; two threads per row, one sum and each block's loads
+// exposed took 32 and 420.
+constexpr int TRSV_G = 4, TRSV_K = LU_NB / TRSV_G;   // threads of a row, columns of a thread
 template <bool LOWER>
-__global__ __launch_bounds__(256) void k_trsv(const float* __restrict__ A, int lda, const float* __restrict__ Tinv,
-                                              float* __restrict__ y, int n, int nblk, unsigned* ticket,
-                                              unsigned base, unsigned long long* yx, unsigned epoch,
-                                              unsigned* abort_flag) {
-    __shared__ float xs[LU_NB];
-    __shared__ float part[2][LU_NB];
+__global__ __launch_bounds__(LU_NB * TRSV_G) void k_trsv(const float* __restrict__ A, int lda,
+                                                         const float* __restrict__ Tinv, const double* __restrict__ r64,
+                                                         const int* __restrict__ perm, float* __restrict__ y,
+                                                         double* __restrict__ x64, int n, int nblk, unsigned* ticket,
+                                                         unsigned base, unsigned long long* yx, unsigned epoch,
+                                                         unsigned* abort_flag, const SolveState* __restrict__ st) {
+    __shared__ float4 xs4[2][LU_NB / 4];
+    __shared__ float part[TRSV_G][LU_NB];
     __shared__ int s_b;
-    const int t = threadIdx.x, r = t & (LU_NB - 1), half = t >> 7;
+    const int t = threadIdx.x, r = t & (LU_NB - 1), g = t >> 7;
     if (t == 0) s_b = (int)(atomicAdd(ticket, 1u) - base);
+    if (st->done) return;
     __syncthreads();
     const int b = LOWER ? s_b : nblk - 1 - s_b;
-    const int b0 = b * LU_NB, nb = min(LU_NB, n - b0);
-    float tinv[LU_NB / 2];
-    const float* Tb = Tinv + (size_t)b * LU_NB * LU_NB;
-#pragma unroll
-    for (int q = 0; q < LU_NB / 2; ++q) tinv[q] = Tb[(2 * q + half) * LU_NB + r];
-    float acc = 0.f;
+    const int b0 = b * LU_NB, nb = min(LU_NB, n - b0), k0 = g * TRSV_K;
+    const float* Ar = A + b0 + min(r, nb - 1);
     const int ndep = LOWER ? b : nblk - 1 - b;
-    for (int d = 0; d < ndep; ++d) {
-        const int c = LOWER ? d : nblk - 1 - d;
-        const int c0 = c * LU_NB, nc = min(LU_NB, n - c0);
-        float a[LU_NB / 2];
+    // columns past n (in the last block alone) are read as the last, times zero
+    auto load = [&](int d, float* a) {
+        const int c0 = (LOWER ? d : nblk - 1 - d) * LU_NB, last = n - 1 - c0;
 #pragma unroll
-        for (int q = 0; q < LU_NB / 2; ++q) {
-            const int k = 2 * q + half;
-            a[q] = (k < nc && r < nb) ? A[(size_t)(c0 + k) * lda + b0 + r] : 0.f;
+        for (int q = 0; q < TRSV_K; ++q) a[q] = Ar[(size_t)(c0 + min(k0 + q, last)) * lda];
+    };
+    float a[TRSV_K], next[TRSV_K], tinv[TRSV_K];
+    if (ndep > 0) load(0, next);
+    const float* Tb = Tinv + (size_t)b * LU_NB * LU_NB + k0 * LU_NB + r;
+#pragma unroll
+    for (int q = 0; q < TRSV_K; ++q) tinv[q] = Tb[q * LU_NB];
+    float rhs = 0.f;
+    if (t < nb) rhs = LOWER ? (float)r64[perm[b0 + t]] : y[b0 + t];
+    auto dot = [&](const float* m, const float4* x) {
+        float s0 = 0.f, s1 = 0.f;
+#pragma unroll
+        for (int q = 0; q < TRSV_K / 4; ++q) {
+            const float4 v = x[k0 / 4 + q];
+            s0 += m[4 * q] * v.x;
+            s1 += m[4 * q + 1] * v.y;
+            s0 += m[4 * q + 2] * v.z;
+            s1 += m[4 * q + 3] * v.w;
         }
+        return s0 + s1;
+    };
+    float acc = 0.f;
+    for (int d = 0; d < ndep; ++d) {
+        const int c0 = (LOWER ? d : nblk - 1 - d) * LU_NB, nc = min(LU_NB, n - c0);
+#pragma unroll
+        for (int q = 0; q < TRSV_K; ++q) a[q] = next[q];
+        if (d + 1 < ndep) load(d + 1, next);
+        float* xs = reinterpret_cast<float*>(xs4[d & 1]);   // (its last readers passed the barrier of d - 1)
         if (t < LU_NB) {
             float v = 0.f;
             if (t < nc) {
@@ -655,7 +686,7 @@ __global__ __launch_bounds__(256) void k_trsv(const float* __restrict__ A, int l
                 while (true) {
                     w = __hip_atomic_load(&yx[c0 + t], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
                     if ((unsigned)(w >> 32) == epoch) break;
-                    if ((spins & 31u) == 0u &&
+                    if ((spins & 31u) == 31u &&
                         __hip_atomic_load(abort_flag, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) != 0u)
                         break;
                     if (++spins > SPIN_LIMIT) {
@@ -669,38 +700,30 @@ __global__ __launch_bounds__(256) void k_trsv(const float* __restrict__ A, int l
             xs[t] = v;
         }
         __syncthreads();
-#pragma unroll
-        for (int q = 0; q < LU_NB / 2; ++q) acc += a[q] * xs[2 * q + half];
-        __syncthreads();
+        acc += dot(a, xs4[d & 1]);
     }
-    part[half][r] = acc;
+    part[g][r] = acc;
     __syncthreads();
-    if (t < LU_NB) xs[t] = t < nb ? y[b0 + t] - (part[0][t] + part[1][t]) : 0.f;
+    if (t < LU_NB)
+        reinterpret_cast<float*>(xs4[0])[t] = t < nb ? rhs - ((part[0][t] + part[1][t]) + (part[2][t] + part[3][t])) : 0.f;
     __syncthreads();
-    float s = 0.f;
-#pragma unroll
-    for (int q = 0; q < LU_NB / 2; ++q) s += tinv[q] * xs[2 * q + half];
-    part[half][r] = s;
+    part[g][r] = dot(tinv, xs4[0]);
     __syncthreads();
     if (t < nb) {
-        const float xv = part[0][t] + part[1][t];
-        y[b0 + t] = xv;
+        const float xv = (part[0][t] + part[1][t]) + (part[2][t] + part[3][t]);
         __hip_atomic_store(&yx[b0 + t], ((unsigned long long)epoch << 32) | (unsigned long long)__float_as_uint(xv),
                            __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+        if (LOWER) y[b0 + t] = xv;
+        else x64[b0 + t] += (double)xv;
     }
-}
-
-// x += (double) y
-__global__ void k_add_f32(double* __restrict__ x, const float* __restrict__ y, int n) {
-    const int i = blockIdx.x * blockDim.x + threadIdx.x;
-    if (i < n) x[i] += (double)y[i];
 }
 
 // ------------------------------------------------------ FP64 residual ----
 constexpr int RES_ROWS = 4;   // matrix rows per wavefront (x is read once per 4 rows)
 __global__ __launch_bounds__(256) void k_resid64(const double* __restrict__ A, int n, const double* __restrict__ x,
                                                  const double* __restrict__ b, double* __restrict__ r,
-                                                 double* __restrict__ rowabs) {
+                                                 double* __restrict__ rowabs, const SolveState* __restrict__ st) {
+    if (st && st->done) return;
     const int lane = threadIdx.x & 63, wv = threadIdx.x >> 6;
     const int row0 = (blockIdx.x * 4 + wv) * RES_ROWS;
     if (row0 >= n) return;
@@ -753,11 +776,15 @@ __global__ __launch_bounds__(256) void k_resid64(const double* __restrict__ A, i
     }
 }
 
-// out = {max|r|, max|x|, max|b|, max rowabs}: one workgroup
-__global__ __launch_bounds__(1024) void k_norms(const double* __restrict__ r, const double* __restrict__ x,
-                                                const double* __restrict__ b, const double* __restrict__ rowabs,
-                                                int n, double* __restrict__ out) {
+// The end of a refinement step, one workgroup: the normwise backward error
+// |r| / (|A| |x| + |b|) (|A| from rowabs when given) and whether to go on.
+__global__ __launch_bounds__(1024) void k_refine_check(const double* __restrict__ r, const double* __restrict__ x,
+                                                       const double* __restrict__ b,
+                                                       const double* __restrict__ rowabs, int n, int it, double tol,
+                                                       int max_iter, const unsigned* __restrict__ abort_flag,
+                                                       SolveState* __restrict__ st) {
     __shared__ double red[4][16];
+    if (it > 0 && st->done) return;
     double m[4] = {0.0, 0.0, 0.0, 0.0};
     for (int i = threadIdx.x; i < n; i += 1024) {
         m[0] = fmax(m[0], fabs(r[i]));
@@ -770,11 +797,22 @@ __global__ __launch_bounds__(1024) void k_norms(const double* __restrict__ r, co
     const int lane = threadIdx.x & 63, wv = threadIdx.x >> 6;
     if (lane == 0) for (int q = 0; q < 4; ++q) red[q][wv] = m[q];
     __syncthreads();
-    if (threadIdx.x < 4) {
+    if (threadIdx.x != 0) return;
+    for (int q = 0; q < 4; ++q) {
         double v = 0.0;
-        for (int k = 0; k < 16; ++k) v = fmax(v, red[threadIdx.x][k]);
-        out[threadIdx.x] = v;
+        for (int k = 0; k < 16; ++k) v = fmax(v, red[q][k]);
+        m[q] = v;
     }
+    const double anorm = rowabs ? m[3] : st->anorm, denom = anorm * m[1] + m[2];
+    const double be = denom > 0.0 ? m[0] / denom : 0.0;
+    st->anorm = anorm;
+    st->backward = be;
+    st->contraction = it > 0 && st->prev > 0.0 ? m[0] / st->prev : it > 0 ? st->contraction : 0.0;
+    st->prev = m[0];
+    st->it = it;
+    st->aborted = *abort_flag;
+    st->converged = be <= tol;
+    st->done = st->aborted != 0u || !isfinite(be) || be <= tol || it >= max_iter;
 }
 
 // ---------------------------------------------------------- VLM kernels --
@@ -1123,27 +1161,34 @@ struct afx_dense {
     float* A32 = nullptr;      // column-major lda x n, LU in place
     int* ipiv = nullptr;       // followed by src and dst
     int* perm = nullptr;
-    double *b = nullptr, *x = nullptr, *r = nullptr, *rowabs = nullptr, *norms = nullptr;
+    double *b = nullptr, *x = nullptr, *r = nullptr, *rowabs = nullptr;
     float* y = nullptr;
     int *src = nullptr, *dst = nullptr;   // every panel's interchanges as a whole (k_panel_lu)
     unsigned long long* keys = nullptr;   // candidates of the panel's workgroups, followed by vals and prow
     unsigned long long* vals = nullptr;   // and their values, value | column sequence
     unsigned long long* prow = nullptr;   // pivot rows of a sub-panel, value | column sequence
     unsigned* pabort = nullptr;
-    int* info = nullptr;
+    int* info = nullptr;   // followed by pabort
     float *Linv = nullptr, *Uinv = nullptr;   // inverses of the 128 x 128 diagonal blocks
     unsigned *tk = nullptr, *abort = nullptr;   // triangular-solve tickets and abort flag
     unsigned long long* yx = nullptr;            // published solution elements: value | epoch << 32
     unsigned tk_base = 0, epoch = 0;
     int nblk = 0;
-    double anorm = -1.0;       // |A|inf of the current FP64 matrix (-1: not yet known)
+    bool anorm_known = false;   // state->anorm is |A|inf of the current FP64 matrix
+    SolveState* state = nullptr;
+    struct Results {            // pinned: what factor and solve read back
+        SolveState solve;
+        int info;
+        unsigned aborted;
+    }* host = nullptr;
     bool factored = false;
     ~afx_dense() {
         for (void* p : {(void*)A64, (void*)A32, (void*)ipiv, (void*)perm, (void*)b, (void*)x, (void*)r,
-                        (void*)rowabs, (void*)norms, (void*)y, (void*)keys,
-                        (void*)pabort, (void*)info, (void*)Linv, (void*)Uinv, (void*)tk,
+                        (void*)rowabs, (void*)state, (void*)y, (void*)keys,
+                        (void*)info, (void*)Linv, (void*)Uinv, (void*)tk,
                         (void*)yx, (void*)abort})
             if (p) (void)hipFree(p);
+        if (host) (void)hipHostFree(host);
         if (ev_panel) (void)hipEventDestroy(ev_panel);
         if (ev_near) (void)hipEventDestroy(ev_near);
         if (ev_far) (void)hipEventDestroy(ev_far);
@@ -1181,14 +1226,15 @@ int dense_init(afx_dense* h, int n) {
     VCHK(dalloc(&h->x, nn));
     VCHK(dalloc(&h->r, nn));
     VCHK(dalloc(&h->rowabs, nn));
-    VCHK(dalloc(&h->norms, 4));
+    VCHK(dalloc(&h->state, 1));
+    VCHK(hipHostMalloc((void**)&h->host, sizeof(afx_dense::Results), hipHostMallocDefault));
     VCHK(dalloc(&h->y, nn));
     const size_t nwg = (nn + PANEL_R - 1) / PANEL_R;
     VCHK(dalloc(&h->keys, 2 * nwg * KEY_STRIDE + 2 * nwg * SUB + 2 * SUB * LU_NB));
     h->vals = h->keys + 2 * nwg * KEY_STRIDE;
     h->prow = h->vals + 2 * nwg * SUB;
-    VCHK(dalloc(&h->pabort, 1));
-    VCHK(dalloc(&h->info, 1));
+    VCHK(dalloc(&h->info, 2));
+    h->pabort = reinterpret_cast<unsigned*>(h->info + 1);
     h->nblk = (n + LU_NB - 1) / LU_NB;
     VCHK(dalloc(&h->Linv, (size_t)h->nblk * LU_NB * LU_NB));
     VCHK(dalloc(&h->Uinv, (size_t)h->nblk * LU_NB * LU_NB));
@@ -1273,80 +1319,67 @@ int dense_factor(afx_dense* h, int32_t* info_out) {
     VCHK(hipGetLastError());
     VCHK(hipEventRecord(h->ev_far, h->s2));
     VCHK(hipStreamWaitEvent(s, h->ev_far, 0));
-    unsigned aborted = 0;
-    int info = 0;
-    VCHK(hipMemcpyAsync(&aborted, h->pabort, sizeof(unsigned), hipMemcpyDeviceToHost, s));
-    VCHK(hipMemcpyAsync(&info, h->info, sizeof(int), hipMemcpyDeviceToHost, s));
+    VCHK(hipMemcpyAsync(&h->host->info, h->info, 2 * sizeof(int), hipMemcpyDeviceToHost, s));
     VCHK(hipStreamSynchronize(s));
-    if (aborted) return api_fail(AFX_EHIP, "LU panel: pivot exchange timed out (workgroups not co-resident)");
+    const int info = h->host->info;
+    if (h->host->aborted) return api_fail(AFX_EHIP, "LU panel: pivot exchange timed out (workgroups not co-resident)");
     if (info_out) *info_out = info;
     h->factored = info == 0;
     if (info) return api_fail(AFX_EARG, "matrix is singular in FP32: zero pivot at column " + std::to_string(info - 1));
     return AFX_OK;
 }
 
-// y <- U^-1 L^-1 y (y already permuted): one launch per triangle
-int dense_lu_solve(afx_dense* h) {
-    hipStream_t s = h->s;
-    const int nb = h->nblk;
-    k_trsv<true><<<nb, 256, 0, s>>>(h->A32, h->lda, h->Linv, h->y, h->n, nb, h->tk, h->tk_base, h->yx,
-                                    ++h->epoch, h->abort);
-    h->tk_base += (unsigned)nb;
-    k_trsv<false><<<nb, 256, 0, s>>>(h->A32, h->lda, h->Uinv, h->y, h->n, nb, h->tk, h->tk_base, h->yx,
-                                     ++h->epoch, h->abort);
-    h->tk_base += (unsigned)nb;
-    VCHK(hipGetLastError());
-    return AFX_OK;
-}
-
 // FP64 iterative refinement: x = 0 (or the caller's x when warm); repeat r = b - A x (FP64), stop when the
-// normwise backward error |r| / (|A| |x| + |b|) <= tol, else x += LU^-1 P r.
+// normwise backward error |r| / (|A| |x| + |b|) <= tol, else x += U^-1 L^-1 P r.  The decisions are taken on
+// the device (SolveState) and steps are queued two at a time: a wait after each, with its copies back, took
+// a third of a solve of order 1 280, and a step that turns out not to be needed costs its four launches.
 int dense_solve_dev(afx_dense* h, const double* b_dev, double* x_dev, double tol, int max_iter, bool warm,
                     afx_solve_info* info) {
     if (!h->factored) return api_fail(AFX_ESTATE, "no factorisation: call factor first");
-    const int n = h->n;
+    const int n = h->n, nb = h->nblk;
     hipStream_t s = h->s;
     if (tol <= 0.0) tol = std::sqrt((double)n) * 1.1102230246251565e-16;
     if (max_iter <= 0) max_iter = 30;
     if (!warm) VCHK(hipMemsetAsync(x_dev, 0, n * sizeof(double), s));
-    afx_solve_info inf{};
-    double prev = -1.0;
-    const int tb = 256;
-    for (int it = 0;; ++it) {
-        const bool need_norm = h->anorm < 0.0;
-        k_resid64<<<(n + 4 * RES_ROWS - 1) / (4 * RES_ROWS), 256, 0, s>>>(h->A64, n, x_dev, b_dev, h->r,
-                                                                         need_norm ? h->rowabs : nullptr);
-        k_norms<<<1, 1024, 0, s>>>(h->r, x_dev, b_dev, need_norm ? h->rowabs : nullptr, n, h->norms);
-        VCHK(hipGetLastError());
-        double nrm[4];
-        unsigned aborted = 0;
-        VCHK(hipMemcpyAsync(nrm, h->norms, sizeof(nrm), hipMemcpyDeviceToHost, s));
-        VCHK(hipMemcpyAsync(&aborted, h->abort, sizeof(unsigned), hipMemcpyDeviceToHost, s));
-        VCHK(hipStreamSynchronize(s));
-        if (aborted) {
-            // the timed-out launch left the solution words incomplete: the
-            // factorisation is discarded, and the next factor call clears the
-            // flag (k_panel_reset)
-            h->factored = false;
-            return api_fail(AFX_EHIP, "triangular solve: a block wait timed out (factor again before solving)");
+    const bool need_norm = !h->anorm_known;
+    auto evaluate = [&](int it) {
+        double* rowabs = it == 0 && need_norm ? h->rowabs : nullptr;
+        k_resid64<<<(n + 4 * RES_ROWS - 1) / (4 * RES_ROWS), 256, 0, s>>>(h->A64, n, x_dev, b_dev, h->r, rowabs,
+                                                                         it > 0 ? h->state : nullptr);
+        k_refine_check<<<1, 1024, 0, s>>>(h->r, x_dev, b_dev, rowabs, n, it, tol, max_iter, h->abort, h->state);
+    };
+    evaluate(0);
+    SolveState& st = h->host->solve;
+    for (int it = 0;;) {
+        for (int q = 0; q < 2 && it < max_iter; ++q) {
+            k_trsv<true><<<nb, LU_NB * TRSV_G, 0, s>>>(h->A32, h->lda, h->Linv, h->r, h->perm, h->y, nullptr, n, nb, h->tk,
+                                                      h->tk_base, h->yx, ++h->epoch, h->abort, h->state);
+            h->tk_base += (unsigned)nb;
+            k_trsv<false><<<nb, LU_NB * TRSV_G, 0, s>>>(h->A32, h->lda, h->Uinv, nullptr, nullptr, h->y, x_dev, n, nb, h->tk,
+                                                       h->tk_base, h->yx, ++h->epoch, h->abort, h->state);
+            h->tk_base += (unsigned)nb;
+            evaluate(++it);
         }
-        if (need_norm) h->anorm = nrm[3];
-        const double denom = h->anorm * nrm[1] + nrm[2];
-        inf.backward_error = denom > 0.0 ? nrm[0] / denom : 0.0;
-        if (prev > 0.0) inf.contraction = nrm[0] / prev;
-        prev = nrm[0];
-        inf.iterations = it;
-        if (!std::isfinite(inf.backward_error)) break;
-        if (inf.backward_error <= tol) { inf.converged = 1; break; }
-        if (it >= max_iter) break;
-        k_gather_perm<<<(n + tb - 1) / tb, tb, 0, s>>>(h->r, h->perm, h->y, n);
         VCHK(hipGetLastError());
-        int rc = dense_lu_solve(h);
-        if (rc) return rc;
-        k_add_f32<<<(n + tb - 1) / tb, tb, 0, s>>>(x_dev, h->y, n);
-        VCHK(hipGetLastError());
+        VCHK(hipMemcpyAsync(&st, h->state, sizeof(st), hipMemcpyDeviceToHost, s));
+        VCHK(hipStreamSynchronize(s));
+        if (st.done) break;
     }
-    if (info) *info = inf;
+    if (st.aborted) {
+        // the timed-out launch left the solution words incomplete: the
+        // factorisation is discarded, and the next factor call clears the
+        // flag (k_panel_reset)
+        h->factored = false;
+        return api_fail(AFX_EHIP, "triangular solve: a block wait timed out (factor again before solving)");
+    }
+    h->anorm_known = true;
+    if (info) {
+        *info = afx_solve_info{};
+        info->iterations = st.it;
+        info->converged = st.converged;
+        info->backward_error = st.backward;
+        info->contraction = st.contraction;
+    }
     return AFX_OK;
 }
 
@@ -1364,7 +1397,9 @@ struct afx_vlm {
            *d_normal = nullptr, *d_rhs = nullptr, *d_gamma = nullptr, *d_rforce = nullptr, *d_sforce = nullptr;
     int *d_rn = nullptr, *d_soff = nullptr, *d_rst = nullptr;
     double* d_salpha = nullptr;
+    double* stage = nullptr;   // pinned: nodes on their way in, angles and forces
     ~afx_vlm() {
+        if (stage) (void)hipHostFree(stage);
         for (void* p : {(void*)d_nodes, (void*)d_corner, (void*)d_wcorner, (void*)d_colloc, (void*)d_normal,
                         (void*)d_rhs, (void*)d_gamma, (void*)d_rforce, (void*)d_sforce, (void*)d_rn, (void*)d_soff,
                         (void*)d_rst, (void*)d_salpha})
@@ -1403,7 +1438,7 @@ int afx_dense_set(afx_dense* h, const double* a) {
     if (!h || !a) return api_fail(AFX_EARG, "null argument");
     VCHK(hipMemcpyAsync(h->A64, a, (size_t)h->n * h->n * sizeof(double), hipMemcpyHostToDevice, h->s));
     VCHK(hipStreamSynchronize(h->s));
-    h->anorm = -1.0;
+    h->anorm_known = false;
     h->factored = false;
     return AFX_OK;
 }
@@ -1485,6 +1520,9 @@ int afx_vlm_create(int32_t n_nodes, const double* xyz, int32_t n_stations, const
     VCHK_C(dalloc(&h->d_soff, n_stations + 1));
     VCHK_C(dalloc(&h->d_rst, nr));
     VCHK_C(dalloc(&h->d_salpha, n_stations));
+    VCHK_C(hipHostMalloc((void**)&h->stage,
+                         sizeof(double) * std::max(3 * (size_t)n_nodes, 3 * ((size_t)nr + n_stations) + n_stations),
+                         hipHostMallocDefault));
     std::vector<int> rst(nr);
     for (int st = 0; st < n_stations; ++st)
         for (int k = soff[st]; k < soff[st + 1]; ++k) rst[k] = st;
@@ -1527,8 +1565,9 @@ int afx_vlm_set_flow(afx_vlm* h, const afx_vlm_flow* f) {
 int afx_vlm_set_nodes(afx_vlm* h, const double* xyz) {
     if (!h || !xyz) return api_fail(AFX_EARG, "null argument");
     std::copy(xyz, xyz + 3 * (size_t)h->nn, h->xyz.begin());
-    VCHK(hipMemcpyAsync(h->d_nodes, xyz, 3 * (size_t)h->nn * sizeof(double), hipMemcpyHostToDevice, h->dense->s));
-    VCHK(hipStreamSynchronize(h->dense->s));
+    VCHK(hipStreamSynchronize(h->dense->s));   // the stage is free
+    std::copy(h->xyz.begin(), h->xyz.end(), h->stage);
+    VCHK(hipMemcpyAsync(h->d_nodes, h->stage, 3 * (size_t)h->nn * sizeof(double), hipMemcpyHostToDevice, h->dense->s));
     h->built = h->solved = false;
     return AFX_OK;
 }
@@ -1565,8 +1604,7 @@ int afx_vlm_build(afx_vlm* h) {
     k_aic_wake<<<(unsigned)((nw + 255) / 256), 256, 0, s>>>(h->d_colloc, h->d_normal, h->d_wcorner, h->d_soff, ns,
                                                             nr, f.core_radius, h->dense->A64);
     VCHK(hipGetLastError());
-    VCHK(hipStreamSynchronize(s));
-    h->dense->anorm = -1.0;
+    h->dense->anorm_known = false;
     h->built = true;
     h->solved = false;
     return AFX_OK;
@@ -1604,12 +1642,14 @@ int afx_vlm_forces(afx_vlm* h, double* ring_force, double* station_force, double
     k_forces<<<(h->ns + 127) / 128, 128, 0, s>>>(h->d_corner, h->d_gamma, h->d_soff, h->ns, f.rho, vx, 0.0, vz,
                                                  h->d_rforce, h->d_sforce);
     VCHK(hipGetLastError());
-    std::vector<double> sf(3 * (size_t)h->ns);
-    VCHK(hipMemcpyAsync(sf.data(), h->d_sforce, sf.size() * sizeof(double), hipMemcpyDeviceToHost, s));
+    const size_t nsf = 3 * (size_t)h->ns, nrf = 3 * (size_t)h->nr;
+    const double *sf = h->stage, *rf = h->stage + nsf;
+    VCHK(hipMemcpyAsync(h->stage, h->d_sforce, nsf * sizeof(double), hipMemcpyDeviceToHost, s));
     if (ring_force)
-        VCHK(hipMemcpyAsync(ring_force, h->d_rforce, 3 * (size_t)h->nr * sizeof(double), hipMemcpyDeviceToHost, s));
+        VCHK(hipMemcpyAsync(h->stage + nsf, h->d_rforce, nrf * sizeof(double), hipMemcpyDeviceToHost, s));
     VCHK(hipStreamSynchronize(s));
-    if (station_force) std::copy(sf.begin(), sf.end(), station_force);
+    if (ring_force) std::copy(rf, rf + nrf, ring_force);
+    if (station_force) std::copy(sf, sf + nsf, station_force);
     if (coeffs) {
         // lift axis = freestream x unit-y (input.cpp:46-52), stream axis = freestream
         const double q = 0.5 * f.rho * f.vinf * f.vinf;
@@ -1713,7 +1753,9 @@ int afx_vlm_nonlinear_solve(afx_vlm* h, const afx_polar* P, double relaxation, d
     }
     for (int st = ns - 1; st >= 0; --st) spanloc[st] = (spanloc[st] - spanloc[0]) / span;
     const double q = 0.5 * f.rho * f.vinf * f.vinf;
-    std::vector<double> alpha(ns, f.alpha_deg), sf(3 * (size_t)ns), clinv(ns);
+    std::vector<double> alpha(ns, f.alpha_deg), clinv(ns);
+    double *sf = h->stage, *angles = h->stage + 3 * (size_t)ns;   // (free after each wait of the loop)
+    VCHK(hipStreamSynchronize(h->dense->s));
     hipStream_t s = h->dense->s;
     auto lift_axis = [&](int st, double* ax) {   // unit(V(alpha_s) x dl_LE)
         const double a = alpha[st] * M_PI / 180.0, vx = std::cos(a), vz = std::sin(a);
@@ -1728,7 +1770,8 @@ int afx_vlm_nonlinear_solve(afx_vlm* h, const afx_polar* P, double relaxation, d
     int iter = 0;
     double residual = 0.0;
     do {
-        VCHK(hipMemcpyAsync(h->d_salpha, alpha.data(), ns * sizeof(double), hipMemcpyHostToDevice, s));
+        std::copy(alpha.begin(), alpha.end(), angles);
+        VCHK(hipMemcpyAsync(h->d_salpha, angles, ns * sizeof(double), hipMemcpyHostToDevice, s));
         k_rhs_stations<<<(h->nr + 127) / 128, 128, 0, s>>>(h->d_normal, h->d_rst, h->nr, f.vinf, h->d_salpha, h->d_rhs);
         VCHK(hipGetLastError());
         afx_solve_info si{};
@@ -1738,7 +1781,7 @@ int afx_vlm_nonlinear_solve(afx_vlm* h, const afx_polar* P, double relaxation, d
         k_forces_stations<<<(ns + 127) / 128, 128, 0, s>>>(h->d_corner, h->d_gamma, h->d_soff, ns, f.rho, f.vinf,
                                                            h->d_salpha, h->d_sforce);
         VCHK(hipGetLastError());
-        VCHK(hipMemcpyAsync(sf.data(), h->d_sforce, sf.size() * sizeof(double), hipMemcpyDeviceToHost, s));
+        VCHK(hipMemcpyAsync(sf, h->d_sforce, 3 * (size_t)ns * sizeof(double), hipMemcpyDeviceToHost, s));
         VCHK(hipStreamSynchronize(s));
         residual = 0.0;
         for (int st = 0; st < ns; ++st) {

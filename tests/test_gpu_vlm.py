@@ -110,6 +110,30 @@ def test_first_panel_takes_the_plain_right_looking_steps(vlm, n, ties):
     assert np.array_equal(lu[nb:, :nb], P[perm[nb:]])
 
 
+# block rows of one row, whole and ragged; the steps are queued in pairs, so the
+# limit on them falls inside a pair and at its end
+@pytest.mark.parametrize("n", [1, 2, 127, 128, 129, 256, 257, 640])
+def test_refined_solve_at_the_edges_of_blocks_and_pairs(vlm, n):
+    rng = np.random.default_rng(n)
+    A = rng.normal(size=(n, n)) + 2.0 * math.sqrt(n) * np.eye(n)
+    b = rng.normal(size=n)
+    d = vlm.Dense(n)
+    d.set(A)
+    d.factor()
+    x, info = d.solve(b)
+    assert info.converged
+    # normwise: |x - A^-1 b| <= |A^-1| (2 sqrt(n) eps |A| |x|), twice for numpy's own
+    Ai = np.linalg.inv(A)
+    bound = 4 * math.sqrt(n) * 1.12e-16 * np.linalg.norm(Ai, np.inf) * np.linalg.norm(A, np.inf) * np.abs(x).max()
+    assert np.abs(x - Ai @ b).max() <= bound + n * 1.12e-16 * np.abs(Ai).sum(1).max() * np.abs(b).max()
+    for most in (1, 2, 3):
+        y, few = d.solve(b, tol=1e-30, max_iter=most)
+        # (a residual of one or two rows can be exactly zero)
+        assert few.converged == (few.backward_error <= 1e-30)
+        assert few.iterations == most or few.converged
+        assert np.isfinite(y).all()
+
+
 @pytest.mark.parametrize("n,cond", [(300, 1e2), (700, 1e6), (1537, 1e3)])
 def test_refined_solve_matches_fp64(vlm, n, cond):
     print(f"[vlm] refine n={n} cond={cond:g}", flush=True)
