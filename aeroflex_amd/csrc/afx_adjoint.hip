@@ -44,36 +44,44 @@ __device__ __forceinline__ GasT<Dual1> dual_gas(const GasT<double>& g) {
     return GasT<Dual1>{Dual1(g.gamma), Dual1(g.R), Dual1(g.mu), Dual1(g.k), Dual1(g.cp), Dual1(g.PrL), Dual1(g.PrT)};
 }
 
-// b += (d face_vars(kind, qL, qbc) / d qL)^T a  (qbc is boundary data)
-__device__ __forceinline__ void face_vars_vjp(const GasT<double>& g, int kind, double nx, double ny, const double* qL,
-                                              const double* qbc, const double* a, double* b) {
+// component j of (d face_vars(kind, qL, qbc) / d qL)^T a  (qbc is boundary data)
+__device__ __forceinline__ double face_vars_vjp(const GasT<double>& g, int kind, double nx, double ny, const double* qL,
+                                                const double* qbc, const double* a, int j) {
     const GasT<Dual1> gd = dual_gas(g);
-    Dual1 bc[4], out[4];
-    for (int k = 0; k < 4; ++k) bc[k] = Dual1(qbc[k]);
-    for (int j = 0; j < 4; ++j) {
-        Dual1 in[4];
-        for (int k = 0; k < 4; ++k) in[k] = Dual1(qL[k], k == j ? 1.0 : 0.0);
-        face_vars<Dual1>(gd, kind, Dual1(nx), Dual1(ny), in, bc, out);
-        double s = 0.0;
-        for (int k = 0; k < 4; ++k) s += out[k].d * a[k];
-        b[j] += s;
+    Dual1 in[4], bc[4], out[4];
+    for (int k = 0; k < 4; ++k) {
+        in[k] = Dual1(qL[k], k == j ? 1.0 : 0.0);
+        bc[k] = Dual1(qbc[k]);
     }
+    face_vars<Dual1>(gd, kind, Dual1(nx), Dual1(ny), in, bc, out);
+    double s = 0.0;
+    for (int k = 0; k < 4; ++k) s += out[k].d * a[k];
+    return s;
 }
 
-// b += (d face_vars(kind, qL, qbc) / d qbc)^T a  (farfield boundary data)
-__device__ __forceinline__ void face_vars_vjp_bc(const GasT<double>& g, int kind, double nx, double ny,
-                                                 const double* qL, const double* qbc, const double* a, double* b) {
+// component j of (d face_vars(kind, qL, qbc) / d qbc)^T a  (farfield boundary data)
+__device__ __forceinline__ double face_vars_vjp_bc(const GasT<double>& g, int kind, double nx, double ny,
+                                                   const double* qL, const double* qbc, const double* a, int j) {
     const GasT<Dual1> gd = dual_gas(g);
-    Dual1 in[4], out[4];
-    for (int k = 0; k < 4; ++k) in[k] = Dual1(qL[k]);
-    for (int j = 0; j < 4; ++j) {
-        Dual1 bc[4];
-        for (int k = 0; k < 4; ++k) bc[k] = Dual1(qbc[k], k == j ? 1.0 : 0.0);
-        face_vars<Dual1>(gd, kind, Dual1(nx), Dual1(ny), in, bc, out);
-        double s = 0.0;
-        for (int k = 0; k < 4; ++k) s += out[k].d * a[k];
-        b[j] += s;
+    Dual1 in[4], bc[4], out[4];
+    for (int k = 0; k < 4; ++k) {
+        in[k] = Dual1(qL[k]);
+        bc[k] = Dual1(qbc[k], k == j ? 1.0 : 0.0);
     }
+    face_vars<Dual1>(gd, kind, Dual1(nx), Dual1(ny), in, bc, out);
+    double s = 0.0;
+    for (int k = 0; k < 4; ++k) s += out[k].d * a[k];
+    return s;
+}
+
+__device__ __forceinline__ double pick4(const double* v, int k) {
+    return k == 0 ? v[0] : k == 1 ? v[1] : k == 2 ? v[2] : v[3];
+}
+
+// sum over the four lanes of a boundary face
+__device__ __forceinline__ double quad_sum(double v) {
+    v += __shfl_xor(v, 1);
+    return v + __shfl_xor(v, 2);
 }
 
 // d face_vars(kind, qL, qbc; n) / d n_dir, dir 0 = x, 1 = y
@@ -132,13 +140,29 @@ __device__ void viscous_vjp(const GasT<double>& g, double nx, double ny, const d
     }
 }
 
-// pass 1: gradients, limiters and the active branch of every (cell, variable)
+// pass 1: gradients, limiters and the active branch of every (cell, variable),
+// and in a reversed step the reverse of the stage's update.  Bound by the chain of
+// dependent loads (slot word, face, cells), so the words and cells of all four
+// slots are read first; the gradients of the step's start are formed with the
+// first stage reversed and read by the others: 15 to 13 us a stage at 56k cells,
+// with the update, which was a launch of 5 us.
 __global__ void __launch_bounds__(kBlock)
 k_adj_forward(CellsT<double> C, FacesT<double> F, const double* qg, const double* q, GasT<double> g, int second_order,
-              double limiter_k, AdjBufs A) {
+              double limiter_k, AdjBufs A, RevStage R) {
     const int c = xcd_index();
     if (c >= C.nC) return;
     const size_t nT = (size_t)C.nT, nC = (size_t)C.nC;
+    if (R.g) {   // reverse of q_s+1 = q + W_s dt coef
+        double sdt = 0.0;
+        for (int k = 0; k < 4; ++k) {
+            const size_t i = k * nT + c;
+            const double gk = R.g[i];
+            R.qbar[i] = R.first ? gk : R.qbar[i] + gk;
+            R.wseed[i] = gk * R.dt[c] * R.coef / C.area[c];
+            sdt += gk * R.W[i] * R.coef;
+        }
+        R.dtbar[c] = R.first ? sdt : R.dtbar[c] + sdt;
+    }
     // gradients and limiters of one state (qg == q): the neighbour extrema
     // come from the values the gradient loop already holds
     const bool same = qg == q;
@@ -146,11 +170,24 @@ k_adj_forward(CellsT<double> C, FacesT<double> F, const double* qg, const double
     double mn[4], mx[4];
     int jmn[4] = {-1, -1, -1, -1}, jmx[4] = {-1, -1, -1, -1};
     for (int k = 0; k < 4; ++k) { qc[k] = q[k * nT + c]; mn[k] = qc[k]; mx[k] = qc[k]; }
+    const bool have = R.g && !R.first;   // the gradients of the step's start, from its first reversed stage
+    uint32_t es[4];
+    int os[4], ns[4], ks[4];
+#pragma unroll
+    for (int s = 0; s < 4; ++s) es[s] = C.cface[(size_t)s * nC + c];
+#pragma unroll
     for (int s = 0; s < 4; ++s) {
-        const uint32_t e = C.cface[(size_t)s * nC + c];
+        const int f = es[s] == 0xFFFFFFFFu ? 0 : (int)(es[s] & 0x7FFFFFFFu);
+        os[s] = F.c0[f];
+        ns[s] = F.c1[f];
+        ks[s] = F.kind[f];
+    }
+#pragma unroll 1
+    for (int s = 0; s < 4 && !have; ++s) {
+        const uint32_t e = es[s];
         if (e == 0xFFFFFFFFu) break;
         const int f = (int)(e & 0x7FFFFFFFu);
-        const int o = F.c0[f], n = F.c1[f], kind = F.kind[f];
+        const int o = os[s], n = ns[s], kind = ks[s];
         double qo[4], qn[4], qv[4];
         for (int k = 0; k < 4; ++k) { qo[k] = qg[k * nT + o]; qn[k] = qg[k * nT + n]; }
         face_vars<double>(g, kind, F.nx[f], F.ny[f], qo, qn, qv);
@@ -170,21 +207,28 @@ k_adj_forward(CellsT<double> C, FacesT<double> F, const double* qg, const double
         }
     }
     const double Ar = C.area[c];
+    double gx[4], gy[4];
     for (int k = 0; k < 4; ++k) {
-        A.gx[k * nT + c] = sx[k] / Ar;
-        A.gy[k * nT + c] = sy[k] / Ar;
+        if (have) {
+            gx[k] = A.gx[k * nT + c];
+            gy[k] = A.gy[k * nT + c];
+        } else {
+            A.gx[k * nT + c] = gx[k] = sx[k] / Ar;
+            A.gy[k * nT + c] = gy[k] = sy[k] / Ar;
+        }
     }
     if (!second_order) return;
-    if (!same)
+    if (!same || have)
+#pragma unroll
         for (int s = 0; s < 4; ++s) {
-            const uint32_t e = C.cface[(size_t)s * nC + c];
-            if (e == 0xFFFFFFFFu) break;
-            const int f = (int)(e & 0x7FFFFFFFu);
-            const int kind = F.kind[f];
-            if (kind == K_WALL || kind == K_SLIP) continue;   // ghost = owner copy
-            const int other = (e >> 31) ? F.c0[f] : F.c1[f];
+            const uint32_t e = es[s];
+            const int kind = ks[s];
+            const int other = (e >> 31) ? os[s] : ns[s];
+            double qv[4];
+            for (int k = 0; k < 4; ++k) qv[k] = q[k * nT + other];
+            if (e == 0xFFFFFFFFu || kind == K_WALL || kind == K_SLIP) continue;   // ghost = owner copy
             for (int k = 0; k < 4; ++k) {
-                const double v = q[k * nT + other];
+                const double v = qv[k];
                 if (v < mn[k]) { mn[k] = v; jmn[k] = other; }
                 if (mx[k] < v) { mx[k] = v; jmx[k] = other; }
             }
@@ -192,13 +236,14 @@ k_adj_forward(CellsT<double> C, FacesT<double> F, const double* qg, const double
     const double Ka = limiter_k * sqrt(Ar), K3a = Ka * Ka * Ka;
     double lm[4] = {1, 1, 1, 1};
     int act[4] = {-1, -1, -1, -1};
+#pragma unroll
     for (int s = 0; s < 4; ++s) {
-        const uint32_t e = C.cface[(size_t)s * nC + c];
+        const uint32_t e = es[s];
         if (e == 0xFFFFFFFFu) break;
         const int f = (int)(e & 0x7FFFFFFFu);
         const double dx = F.xf[f] - C.xc[c], dy = F.yf[f] - C.yc[c];
         for (int k = 0; k < 4; ++k) {
-            const double dqg = sx[k] / Ar * dx + sy[k] / Ar * dy;
+            const double dqg = gx[k] * dx + gy[k] * dy;
             const double l = limiter_phi<double>(dqg, mx[k] - qc[k], mn[k] - qc[k], K3a);
             if (l < lm[k]) { lm[k] = l; act[k] = s; }
         }
@@ -211,23 +256,37 @@ k_adj_forward(CellsT<double> C, FacesT<double> F, const double* qg, const double
     }
 }
 
-// pass 2: per face, adjoints of the reconstructed states.  PART 1 takes the
-// interior faces (boundary code compiled out, so the kernel needs far fewer
-// registers), PART 2 the boundary faces from the list A.bface.  LAM compiles
-// the laminar terms in (interior faces of the laminar residual, A.vgx set);
-// without them the inviscid instances need far fewer registers.
+// The face passes take the interior faces (PART 1) a thread each and the boundary
+// faces (PART 2), from the list A.bface, four lanes each, in one launch: blocks
+// below `nbb` the boundary faces, the rest the interior ones in XCD-aware order.
+// The lanes share a boundary face's forward-mode sweeps, a direction per lane.  A
+// thread per boundary face in a launch of its own took 30 us for the 500 faces of
+// a 56k-cell mesh (15 in pass 4) behind the 19 (10) of its 84k interior faces,
+// where the joint launch takes 24 (11).  The joint kernel holds two waves per SIMD
+// where the interior one holds three, yet is no slower at any size: the inviscid
+// adjoint of 115k and 500k cells takes 69 and 217 us with it, 75 and 220 with
+// launches apart.
+constexpr int kBndLanes = 4;
+inline int bnd_blocks(const AdjBufs& A) {   // a multiple of 8, so that the interior blocks keep their XCDs
+    return (((kBndLanes * A.nbf + kBlock - 1) / kBlock) + 7) & ~7;
+}
+
+// pass 2: per face, adjoints of the reconstructed states.  LAM compiles the
+// laminar terms in (interior faces of the laminar residual, A.vgx set); without
+// them the inviscid instances need far fewer registers.
 template <bool GEO, bool GHOST, int PART, bool LAM>
-__global__ void __launch_bounds__(kBlock) k_adj_face(CellsT<double> C, FacesT<double> F, const double* __restrict__ q,
-                                                     const double* __restrict__ w, GasT<double> g, int second_order,
-                                                     AdjBufs A, GeoBufs G, double* __restrict__ ghost) {
-    const int i = PART == 1 ? xcd_index() : (int)(blockIdx.x * blockDim.x + threadIdx.x);
+__device__ __forceinline__ void adj_face_body(const CellsT<double>& C, const FacesT<double>& F,
+                                              const double* __restrict__ q, const double* __restrict__ w,
+                                              const GasT<double>& g, int second_order, const AdjBufs& A,
+                                              const GeoBufs& G, double* __restrict__ ghost, int i) {
     int f;
+    const int lane = PART == 1 ? 0 : (int)(threadIdx.x & (kBndLanes - 1));
     if constexpr (PART == 1) {
         f = i;
         if (f >= F.nF || F.kind[f] != K_INTERNAL) return;
     } else {
-        if (i >= A.nbf) return;
-        f = A.bface[i];
+        if (i / kBndLanes >= A.nbf) return;
+        f = A.bface[i / kBndLanes];
     }
     const size_t nT = (size_t)C.nT, nF = (size_t)F.nF;
     const int o = F.c0[f], n = F.c1[f];
@@ -279,20 +338,27 @@ __global__ void __launch_bounds__(kBlock) k_adj_face(CellsT<double> C, FacesT<do
         double qb[4], bB[4];
         face_vars<double>(g, kind, nx, ny, qL, qR, qb);
         roe_flux_vjp<double>(g.gamma, nx, ny, qL, qb, bF, bL, bB);
-        face_vars_vjp(g, kind, nx, ny, qL, qR, bB, bL);
-        for (int k = 0; k < 4; ++k) bR[k] = 0.0;
+        bL[0] = pick4(bL, lane) + face_vars_vjp(g, kind, nx, ny, qL, qR, bB, lane);   // this lane's component
         if (GHOST && kind == K_FARFIELD) {   // the ghost's first adjoint write of this evaluation
-            double gb[4] = {0.0, 0.0, 0.0, 0.0};
-            face_vars_vjp_bc(g, kind, nx, ny, qL, qR, bB, gb);
-            for (int k = 0; k < 4; ++k) ghost[k * nT + n] = gb[k];
+            const double gb = face_vars_vjp_bc(g, kind, nx, ny, qL, qR, bB, lane);
+            ghost[lane * nT + n] = A.add ? ghost[lane * nT + n] + gb : gb;
         }
     }
-    for (int k = 0; k < 4; ++k) {
-        A.bL[k * nF + f] = bL[k];
-        A.bR[k * nF + f] = bR[k];
+    if constexpr (PART == 1) {
+        for (int k = 0; k < 4; ++k) {
+            A.bL[k * nF + f] = bL[k];
+            A.bR[k * nF + f] = bR[k];
+        }
+    } else {
+        A.bL[lane * nF + f] = bL[0];
+        A.bR[lane * nF + f] = 0.0;
     }
     if (!GEO) return;
     // metric adjoints of F(qL, qR; n) len: length, normal, reconstruction offsets
+    auto put = [&](int plane, double v) {
+        double* to = G.fbar + plane * nF + f;
+        *to = G.add ? *to + v : v;
+    };
     double fl[4], qRuse[4];
     if (kind == K_INTERNAL) {
         for (int k = 0; k < 4; ++k) qRuse[k] = qR[k];
@@ -302,29 +368,52 @@ __global__ void __launch_bounds__(kBlock) k_adj_face(CellsT<double> C, FacesT<do
     roe_flux<double>(g, nx, ny, qL, qRuse, false, nullptr, nullptr, fl);
     double lb = 0.0;
     for (int k = 0; k < 4; ++k) lb += (kind == K_INTERNAL ? w[k * nT + n] - w[k * nT + o] : -w[k * nT + o]) * fl[k];
-    const double nbx = roe_dn(g, kind, nx, ny, qL, qR, bF, 0), nby = roe_dn(g, kind, nx, ny, qL, qR, bF, 1);
     double d0b[2] = {0.0, 0.0}, d1b[2] = {0.0, 0.0};
-    if (second_order) {
-        for (int k = 0; k < 4; ++k) {
-            const double ph = A.lim[k * nT + o] * bL[k];
-            d0b[0] += ph * A.gx[k * nT + o];
-            d0b[1] += ph * A.gy[k * nT + o];
-        }
-        if (kind == K_INTERNAL)
+    if constexpr (PART == 1) {
+        const double nbx = roe_dn(g, kind, nx, ny, qL, qR, bF, 0), nby = roe_dn(g, kind, nx, ny, qL, qR, bF, 1);
+        if (second_order)
             for (int k = 0; k < 4; ++k) {
-                const double ph = A.lim[k * nT + n] * bR[k];
-                d1b[0] += ph * A.gx[k * nT + n];
-                d1b[1] += ph * A.gy[k * nT + n];
+                const double p0 = A.lim[k * nT + o] * bL[k], p1 = A.lim[k * nT + n] * bR[k];
+                d0b[0] += p0 * A.gx[k * nT + o];
+                d0b[1] += p0 * A.gy[k * nT + o];
+                d1b[0] += p1 * A.gx[k * nT + n];
+                d1b[1] += p1 * A.gy[k * nT + n];
             }
+        put(0, nbx);
+        put(1, nby);
+        put(2, lb);
+        put(3, 0.0);
+        put(4, d0b[0]);
+        put(5, d0b[1]);
+        put(6, d1b[0]);
+        put(7, d1b[1]);
+    } else {
+        const double nb = roe_dn(g, kind, nx, ny, qL, qR, bF, lane & 1);
+        if (second_order) {
+            const double p0 = A.lim[lane * nT + o] * bL[0];
+            d0b[0] = quad_sum(p0 * A.gx[lane * nT + o]);
+            d0b[1] = quad_sum(p0 * A.gy[lane * nT + o]);
+        }
+        if (lane < 2) {
+            put(lane, nb);
+            put(4 + lane, lane == 0 ? d0b[0] : d0b[1]);
+        } else {
+            put(lane, lane == 2 ? lb : 0.0);
+            put(4 + lane, 0.0);
+        }
     }
-    G.fbar[0 * nF + f] = nbx;
-    G.fbar[1 * nF + f] = nby;
-    G.fbar[2 * nF + f] = lb;
-    G.fbar[3 * nF + f] = 0.0;
-    G.fbar[4 * nF + f] = d0b[0];
-    G.fbar[5 * nF + f] = d0b[1];
-    G.fbar[6 * nF + f] = d1b[0];
-    G.fbar[7 * nF + f] = d1b[1];
+}
+
+template <bool GEO, bool GHOST, bool LAM>
+__global__ void __launch_bounds__(kBlock) k_adj_face(CellsT<double> C, FacesT<double> F, const double* __restrict__ q,
+                                                     const double* __restrict__ w, GasT<double> g, int second_order,
+                                                     AdjBufs A, GeoBufs G, double* __restrict__ ghost, int nbb) {
+    const int b = (int)blockIdx.x;
+    if (b < nbb)
+        adj_face_body<GEO, GHOST, 2, false>(C, F, q, w, g, second_order, A, G, ghost, b * kBlock + (int)threadIdx.x);
+    else
+        adj_face_body<GEO, GHOST, 1, LAM>(C, F, q, w, g, second_order, A, G, ghost,
+                                          xcd_tile(b - nbb, (int)gridDim.x - nbb) * kBlock + (int)threadIdx.x);
 }
 
 // pass 3: per cell, state / gradient / limiter adjoints
@@ -341,13 +430,21 @@ __global__ void __launch_bounds__(kBlock) k_adj_cell1(CellsT<double> C, FacesT<d
     for (int k = 0; k < 4; ++k) { gx[k] = A.gx[k * nT + c]; gy[k] = A.gy[k * nT + c]; ph[k] = A.lim[k * nT + c]; }
     uint32_t es[4] = {0xFFFFFFFFu, 0xFFFFFFFFu, 0xFFFFFFFFu, 0xFFFFFFFFu};   // the slots' words and offsets, kept
     double dxs[4] = {0, 0, 0, 0}, dys[4] = {0, 0, 0, 0};                   // for the limiter's active slot
+#pragma unroll
+    for (int s = 0; s < 4; ++s) es[s] = C.cface[(size_t)s * nC + c];
+#pragma unroll
+    for (int s = 0; s < 4; ++s) {   // the offsets of all slots in one round trip
+        const int f = es[s] == 0xFFFFFFFFu ? 0 : (int)(es[s] & 0x7FFFFFFFu);
+        dxs[s] = F.xf[f] - C.xc[c];
+        dys[s] = F.yf[f] - C.yc[c];
+    }
+#pragma unroll
     for (int s = 0; s < 4; ++s) {
-        const uint32_t e = C.cface[(size_t)s * nC + c];
+        const uint32_t e = es[s];
         if (e == 0xFFFFFFFFu) break;
         const int f = (int)(e & 0x7FFFFFFFu);
         const bool nb = (e >> 31) != 0;
-        const double dx = F.xf[f] - C.xc[c], dy = F.yf[f] - C.yc[c];
-        es[s] = e; dxs[s] = dx; dys[s] = dy;
+        const double dx = dxs[s], dy = dys[s];
         for (int k = 0; k < 4; ++k) {
             const double b = nb ? A.bR[k * nF + f] : A.bL[k * nF + f];
             lq[k] += b;
@@ -397,8 +494,8 @@ __global__ void __launch_bounds__(kBlock) k_adj_cell1(CellsT<double> C, FacesT<d
             }
         }
         lam[k * nT + c] = lq[k];
-        A.lgx[k * nT + c] = lgx[k];
-        A.lgy[k * nT + c] = lgy[k];
+        A.lgx[k * nT + c] = A.add_lg ? A.lgx[k * nT + c] + lgx[k] : lgx[k];
+        A.lgy[k * nT + c] = A.add_lg ? A.lgy[k * nT + c] + lgy[k] : lgy[k];
         A.nbv[k * nC + c] = nbv;
         A.nbj[k * nC + c] = nbj;
     }
@@ -406,25 +503,23 @@ __global__ void __launch_bounds__(kBlock) k_adj_cell1(CellsT<double> C, FacesT<d
         // gradient = S / A
         if (second_order)
             for (int k = 0; k < 4; ++k) abar -= (lgx[k] * gx[k] + lgy[k] * gy[k]) / C.area[c];
-        G.abar[c] = abar;
+        G.abar[c] = G.add ? G.abar[c] + abar : abar;
     }
 }
 
-// pass 4: transpose of the Green-Gauss face values.  PART 1 takes the
-// interior faces (the boundary face values' reverse compiled out, so the
-// kernel needs far fewer registers), PART 2 the boundary faces of A.bface.
+// pass 4: transpose of the Green-Gauss face values
 template <bool GEO, bool GHOST, int PART>
-__global__ void __launch_bounds__(kBlock) k_adj_face2(CellsT<double> C, FacesT<double> F, const double* __restrict__ q,
-                                                      GasT<double> g, AdjBufs A, GeoBufs G,
-                                                      double* __restrict__ ghost) {
+__device__ __forceinline__ void adj_face2_body(const CellsT<double>& C, const FacesT<double>& F,
+                                               const double* __restrict__ q, const GasT<double>& g, const AdjBufs& A,
+                                               const GeoBufs& G, double* __restrict__ ghost, int i) {
     int f;
+    const int lane = PART == 1 ? 0 : (int)(threadIdx.x & (kBndLanes - 1));
     if constexpr (PART == 1) {
-        f = xcd_index();
+        f = i;
         if (f >= F.nF || F.kind[f] != K_INTERNAL) return;
     } else {
-        const int i = blockIdx.x * blockDim.x + threadIdx.x;
-        if (i >= A.nbf) return;
-        f = A.bface[i];
+        if (i / kBndLanes >= A.nbf) return;
+        f = A.bface[i / kBndLanes];
     }
     const size_t nT = (size_t)C.nT, nF = (size_t)F.nF;
     const int o = F.c0[f], n = F.c1[f];
@@ -437,28 +532,21 @@ __global__ void __launch_bounds__(kBlock) k_adj_face2(CellsT<double> C, FacesT<d
         if (two) v -= (A.lgx[k * nT + n] * nx + A.lgy[k * nT + n] * ny) * L / C.area[n];
         lfv[k] = v;
     }
-    double co[4], cn[4];
-    if (two) {   // face value q_o (1 - gw) + (q_o + q_n) gw / 2
-        for (int k = 0; k < 4; ++k) { co[k] = lfv[k] * (1.0 - 0.5 * gw); cn[k] = lfv[k] * (0.5 * gw); }
+    if constexpr (two) {   // face value q_o (1 - gw) + (q_o + q_n) gw / 2
+        for (int k = 0; k < 4; ++k) {
+            A.co[k * nF + f] = lfv[k] * (1.0 - 0.5 * gw);
+            A.cn[k * nF + f] = lfv[k] * (0.5 * gw);
+        }
     } else {     // q_o (1 - gw) + face_vars(q_o, q_ghost) gw
         double a[4], qo[4], qn[4];
         for (int k = 0; k < 4; ++k) {
             a[k] = lfv[k] * gw;
-            co[k] = lfv[k] * (1.0 - gw);
-            cn[k] = 0.0;
             qo[k] = q[k * nT + o];
             qn[k] = q[k * nT + n];
         }
-        face_vars_vjp(g, kind, nx, ny, qo, qn, a, co);
-        if (GHOST && kind == K_FARFIELD) {
-            double gb[4] = {0.0, 0.0, 0.0, 0.0};
-            face_vars_vjp_bc(g, kind, nx, ny, qo, qn, a, gb);
-            for (int k = 0; k < 4; ++k) ghost[k * nT + n] += gb[k];
-        }
-    }
-    for (int k = 0; k < 4; ++k) {
-        A.co[k * nF + f] = co[k];
-        A.cn[k * nF + f] = cn[k];
+        A.co[lane * nF + f] = pick4(lfv, lane) * (1.0 - gw) + face_vars_vjp(g, kind, nx, ny, qo, qn, a, lane);
+        A.cn[lane * nF + f] = 0.0;
+        if (GHOST && kind == K_FARFIELD) ghost[lane * nT + n] += face_vars_vjp_bc(g, kind, nx, ny, qo, qn, a, lane);
     }
     if (!GEO) return;
     // face value fv (as in pass 1) and the metric adjoints of fv n len / A
@@ -476,24 +564,29 @@ __global__ void __launch_bounds__(kBlock) k_adj_face2(CellsT<double> C, FacesT<d
         lb += fv[k] * (ax * nx + ay * ny);
         gb += lfv[k] * (qv[k] - qo[k]);
     }
-    if (!two) {
-        double dvx[4], dvy[4];
-        face_vars_dn(g, kind, nx, ny, qo, qn, 0, dvx);
-        face_vars_dn(g, kind, nx, ny, qo, qn, 1, dvy);
-        for (int k = 0; k < 4; ++k) {
-            nbx += lfv[k] * gw * dvx[k];
-            nby += lfv[k] * gw * dvy[k];
-        }
+    if constexpr (two) {
+        G.fbar[0 * nF + f] += nbx;
+        G.fbar[1 * nF + f] += nby;
+        G.fbar[2 * nF + f] += lb;
+        G.fbar[3 * nF + f] += gb;
+    } else {
+        double dv[4], nb = lane == 0 ? nbx : nby;
+        face_vars_dn(g, kind, nx, ny, qo, qn, lane & 1, dv);
+        for (int k = 0; k < 4; ++k) nb += lfv[k] * gw * dv[k];
+        G.fbar[lane * nF + f] += lane < 2 ? nb : lane == 2 ? lb : gb;
     }
-    G.fbar[0 * nF + f] += nbx;
-    G.fbar[1 * nF + f] += nby;
-    G.fbar[2 * nF + f] += lb;
-    G.fbar[3 * nF + f] += gb;
 }
 
-__global__ void k_fill0(double* __restrict__ x, int n) {
-    const int i = blockIdx.x * blockDim.x + threadIdx.x;
-    if (i < n) x[i] = 0.0;
+template <bool GEO, bool GHOST>
+__global__ void __launch_bounds__(kBlock) k_adj_face2(CellsT<double> C, FacesT<double> F, const double* __restrict__ q,
+                                                      GasT<double> g, AdjBufs A, GeoBufs G,
+                                                      double* __restrict__ ghost, int nbb) {
+    const int b = (int)blockIdx.x;
+    if (b < nbb)
+        adj_face2_body<GEO, GHOST, 2>(C, F, q, g, A, G, ghost, b * kBlock + (int)threadIdx.x);
+    else
+        adj_face2_body<GEO, GHOST, 1>(C, F, q, g, A, G, ghost,
+                                      xcd_tile(b - nbb, (int)gridDim.x - nbb) * kBlock + (int)threadIdx.x);
 }
 
 // pass 6: face metrics -> face ends and centroids (mesh.h:378-453, 744-787;
@@ -613,33 +706,55 @@ __global__ void __launch_bounds__(kBlock) k_geo_node(CellsT<double> C, FacesT<do
     G.xbar[2 * (size_t)v + 1] = y;
 }
 
-// pass 5: gather of the Green-Gauss transpose and the neighbours' limiter parts
-// lam gets the state part (pass 3 + neighbours' limiter parts), lam_g the
-// Green-Gauss part (the gradient's source state); with lam_g == lam both add
+// pass 5: gather of the Green-Gauss transpose (gg) and the neighbours' limiter
+// parts.  lam gets the state part (pass 3 + neighbours' limiter parts), lam_g the
+// Green-Gauss part (the gradient's source state); with lam_g == lam both add.  In
+// a reversed step the state part is the next stage's seed (R.g), or with the
+// step's last stage joins the Green-Gauss part in R.qbar.
 __global__ void __launch_bounds__(kBlock) k_adj_cell2(CellsT<double> C, FacesT<double> F, AdjBufs A,
-                                                      double* __restrict__ lam, double* lam_g) {
+                                                      double* __restrict__ lam, double* lam_g, int gg, RevStage R) {
     const int c = xcd_index();
     if (c >= C.nC) return;
     const size_t nT = (size_t)C.nT, nC = (size_t)C.nC, nF = (size_t)F.nF;
     double acc[4], accg[4] = {0.0, 0.0, 0.0, 0.0};
     for (int k = 0; k < 4; ++k) acc[k] = lam[k * nT + c];
+    // the four slots' words, then their neighbours, then those cells' limiting
+    // neighbours: each in one round trip (slot by slot, 13 us at 56k cells)
+    uint32_t e[4];
+    int other[4], j[4][4];
+#pragma unroll
+    for (int s = 0; s < 4; ++s) e[s] = C.cface[(size_t)s * nC + c];
+#pragma unroll
     for (int s = 0; s < 4; ++s) {
-        const uint32_t e = C.cface[(size_t)s * nC + c];
-        if (e == 0xFFFFFFFFu) break;
-        const int f = (int)(e & 0x7FFFFFFFu);
-        const bool nb = (e >> 31) != 0;
-        const int other = nb ? F.c0[f] : F.c1[f];
-        for (int k = 0; k < 4; ++k) {
-            accg[k] += nb ? A.cn[k * nF + f] : A.co[k * nF + f];
-            if (other < C.nC && A.nbj[k * nC + other] == c) acc[k] += A.nbv[k * nC + other];
-        }
+        const int f = e[s] == 0xFFFFFFFFu ? 0 : (int)(e[s] & 0x7FFFFFFFu);
+        other[s] = (e[s] >> 31) ? F.c0[f] : F.c1[f];
+        if (e[s] == 0xFFFFFFFFu || other[s] >= C.nC) other[s] = -1;
     }
-    if (lam_g == lam) {
-        for (int k = 0; k < 4; ++k) lam[k * nT + c] = acc[k] + accg[k];
-    } else {
-        for (int k = 0; k < 4; ++k) {
-            lam[k * nT + c] = acc[k];
-            lam_g[k * nT + c] = accg[k];
+#pragma unroll
+    for (int s = 0; s < 4; ++s)
+#pragma unroll
+        for (int k = 0; k < 4; ++k) j[s][k] = A.nbj[k * nC + max(other[s], 0)];
+#pragma unroll
+    for (int s = 0; s < 4; ++s) {
+        if (gg && e[s] != 0xFFFFFFFFu) {
+            const int f = (int)(e[s] & 0x7FFFFFFFu);
+            const double* from = (e[s] >> 31) ? A.cn : A.co;
+            for (int k = 0; k < 4; ++k) accg[k] += from[k * nF + f];
+        }
+#pragma unroll
+        for (int k = 0; k < 4; ++k)
+            if (other[s] >= 0 && j[s][k] == c) acc[k] += A.nbv[k * nC + other[s]];
+    }
+    for (int k = 0; k < 4; ++k) {
+        const size_t i = k * nT + c;
+        if (R.g) {
+            if (R.last) R.qbar[i] += accg[k] + acc[k];
+            else R.g[i] = acc[k];
+        } else if (lam_g == lam) {
+            lam[i] = acc[k] + accg[k];
+        } else {
+            lam[i] = acc[k];
+            lam_g[i] = accg[k];
         }
     }
 }
@@ -681,16 +796,26 @@ __global__ void __launch_bounds__(kBlock) k_dt_bar_face(CellsT<double> C, FacesT
 // per cell: the faces on which this cell's state gives max(eig_o, eig_n)
 __global__ void __launch_bounds__(kBlock) k_dt_bar_cell(CellsT<double> C, FacesT<double> F, const double* __restrict__ q,
                                                         GasT<double> g, const double* __restrict__ ebar,
-                                                        double* __restrict__ qbar) {
+                                                        const double* __restrict__ qbar, double* __restrict__ out) {
     const int c = blockIdx.x * blockDim.x + threadIdx.x;
     if (c >= C.nC) return;
     const size_t nT = (size_t)C.nT, nC = (size_t)C.nC;
     double acc[4] = {0.0, 0.0, 0.0, 0.0};
+    uint32_t es[4];
+    int os[4], ns[4];
+#pragma unroll
+    for (int s = 0; s < 4; ++s) es[s] = C.cface[(size_t)s * nC + c];
+#pragma unroll
     for (int s = 0; s < 4; ++s) {
-        const uint32_t e = C.cface[(size_t)s * nC + c];
-        if (e == 0xFFFFFFFFu) break;
-        const int f = (int)(e & 0x7FFFFFFFu);
-        const int o = F.c0[f], n = F.c1[f];
+        const int f = es[s] == 0xFFFFFFFFu ? 0 : (int)(es[s] & 0x7FFFFFFFu);
+        os[s] = F.c0[f];
+        ns[s] = F.c1[f];
+    }
+#pragma unroll
+    for (int s = 0; s < 4; ++s) {
+        if (es[s] == 0xFFFFFFFFu) break;
+        const int f = (int)(es[s] & 0x7FFFFFFFu);
+        const int o = os[s], n = ns[s];
         const double nx = F.nx[f], ny = F.ny[f];
         double qo[4], d[4];
         for (int k = 0; k < 4; ++k) qo[k] = q[k * nT + o];
@@ -705,46 +830,7 @@ __global__ void __launch_bounds__(kBlock) k_dt_bar_cell(CellsT<double> C, FacesT
         if (active != c) continue;
         for (int k = 0; k < 4; ++k) acc[k] += ebar[f] * d[k];
     }
-    for (int k = 0; k < 4; ++k) qbar[k * nT + c] += acc[k];
-}
-
-// reverse of qk_s+1 = q + W_s dt coef for the real cells: qbar += g,
-// wseed = g dt coef / A (the seed of the undivided residual), dtbar += g . W coef
-__global__ void __launch_bounds__(kBlock) k_rev_stage(const double* __restrict__ gk, const double* __restrict__ W,
-                                                      const double* __restrict__ dt, const double* __restrict__ area,
-                                                      double coef, int32_t nC, int32_t nT, double* __restrict__ wseed,
-                                                      double* __restrict__ dtbar, double* __restrict__ qbar) {
-    const int c = blockIdx.x * blockDim.x + threadIdx.x;
-    if (c >= nC) return;
-    double sdt = 0.0;
-    for (int k = 0; k < 4; ++k) {
-        const size_t i = (size_t)k * nT + c;
-        qbar[i] += gk[i];
-        wseed[i] = gk[i] * dt[c] * coef / area[c];
-        sdt += gk[i] * W[i] * coef;
-    }
-    dtbar[c] += sdt;
-}
-
-// y (+)= a x over the real-cell rows of 4 planes
-__global__ void __launch_bounds__(kBlock) k_axpy4(const double* __restrict__ x, double a, int32_t nC, int32_t nT,
-                                                  int overwrite, double* __restrict__ y) {
-    const int c = blockIdx.x * blockDim.x + threadIdx.x;
-    if (c >= nC) return;
-    for (int k = 0; k < 4; ++k) {
-        const size_t i = (size_t)k * nT + c;
-        y[i] = overwrite ? a * x[i] : y[i] + a * x[i];
-    }
-}
-
-// Facc += G.fbar (8 planes over faces), Aacc += G.abar (real cells)
-__global__ void __launch_bounds__(kBlock) k_acc_metrics(const double* __restrict__ fbar, const double* __restrict__ abar,
-                                                        int32_t nF, int32_t nC, double* __restrict__ facc,
-                                                        double* __restrict__ aacc) {
-    const int i = blockIdx.x * blockDim.x + threadIdx.x;
-    if (i < nF)
-        for (int k = 0; k < 8; ++k) facc[(size_t)k * nF + i] += fbar[(size_t)k * nF + i];
-    if (i < nC) aacc[i] += abar[i];
+    for (int k = 0; k < 4; ++k) out[k * nT + c] = qbar[k * nT + c] + acc[k];
 }
 
 // metric part of the local time step's VJP: dt_c = cfl A_c / S_c with
@@ -792,13 +878,6 @@ __global__ void __launch_bounds__(kBlock) k_ghost_acc(const double* __restrict__
 
 }  // namespace
 
-hipError_t launch_acc_metrics(hipStream_t s, const GeoBufs& G, int32_t nF, int32_t nC, double* facc, double* aacc) {
-    const int n = nF > nC ? nF : nC;
-    hipLaunchKernelGGL(k_acc_metrics, dim3((n + kBlock - 1) / kBlock), dim3(kBlock), 0, s, G.fbar, G.abar, nF, nC,
-                       facc, aacc);
-    return hipGetLastError();
-}
-
 hipError_t launch_dt_vjp_geo(hipStream_t s, CellsT<double> C, FacesT<double> F, const double* q, GasT<double> g,
                              const double* dt, const double* dtbar, double cfl, double* facc) {
     hipLaunchKernelGGL(k_dt_bar_geo, dim3((F.nF + kBlock - 1) / kBlock), dim3(kBlock), 0, s, C, F, q, g, dt, dtbar,
@@ -813,18 +892,6 @@ hipError_t launch_geo_to_nodes(hipStream_t s, CellsT<double> C, FacesT<double> F
     return hipGetLastError();
 }
 
-hipError_t launch_rev_stage(hipStream_t s, const double* gk, const double* W, const double* dt, const double* area,
-                            double coef, int32_t nC, int32_t nT, double* wseed, double* dtbar, double* qbar) {
-    hipLaunchKernelGGL(k_rev_stage, dim3((nC + kBlock - 1) / kBlock), dim3(kBlock), 0, s, gk, W, dt, area, coef, nC,
-                       nT, wseed, dtbar, qbar);
-    return hipGetLastError();
-}
-
-hipError_t launch_axpy4(hipStream_t s, const double* x, double a, int32_t nC, int32_t nT, int overwrite, double* y) {
-    hipLaunchKernelGGL(k_axpy4, dim3((nC + kBlock - 1) / kBlock), dim3(kBlock), 0, s, x, a, nC, nT, overwrite, y);
-    return hipGetLastError();
-}
-
 hipError_t launch_ghost_acc(hipStream_t s, const double* ghost, const int32_t* cells, int32_t n, int32_t nT,
                             double* acc) {
     if (n <= 0) return hipSuccess;
@@ -833,42 +900,40 @@ hipError_t launch_ghost_acc(hipStream_t s, const double* ghost, const int32_t* c
 }
 
 hipError_t launch_dt_vjp(hipStream_t s, CellsT<double> C, FacesT<double> F, const double* q, GasT<double> g,
-                         const double* dt, const double* dtbar, double cfl, double* ebar, double* qbar) {
+                         const double* dt, const double* dtbar, double cfl, double* ebar, const double* qbar,
+                         double* out) {
     hipLaunchKernelGGL(k_dt_bar_face, dim3((F.nF + kBlock - 1) / kBlock), dim3(kBlock), 0, s, C, F, dt, dtbar, cfl,
                        ebar);
-    hipLaunchKernelGGL(k_dt_bar_cell, dim3((C.nC + kBlock - 1) / kBlock), dim3(kBlock), 0, s, C, F, q, g, ebar, qbar);
+    hipLaunchKernelGGL(k_dt_bar_cell, dim3((C.nC + kBlock - 1) / kBlock), dim3(kBlock), 0, s, C, F, q, g, ebar, qbar, out);
     return hipGetLastError();
 }
 
 namespace {
+// R.g null: the adjoint of one residual; otherwise one stage of a reversed step,
+// whose Green-Gauss transpose (linear in the gradient adjoints, and of the
+// step's start in every stage) is applied once, to the sum over the stages
 template <bool GEO, bool GHOST>
 void adjoint_passes(hipStream_t s, CellsT<double> C, FacesT<double> F, const double* qg, const double* q,
                     const double* w, GasT<double> g, int second_order, double limiter_k, AdjBufs A, double* lam,
-                    double* lam_g, double* ghost, const GeoBufs& G, bool to_nodes = true) {
-    // the pass kernels index cells and faces in XCD-aware block order
-    const int nbc = xcd_grid(C.nC), nbf = xcd_grid(F.nF);
-    hipLaunchKernelGGL(k_adj_forward, dim3(nbc), dim3(kBlock), 0, s, C, F, qg, q, g, second_order, limiter_k, A);
+                    double* lam_g, double* ghost, const GeoBufs& G, const RevStage& R = RevStage{}) {
+    // the pass kernels index cells and interior faces in XCD-aware block order
+    const int nbc = xcd_grid(C.nC), nbf = xcd_grid(F.nF), nbb = bnd_blocks(A);
+    const bool gradients = second_order || A.vgx;   // they enter the residual (reconstruction or laminar terms)
+    const bool gg = gradients && (!R.g || R.last);
+    hipLaunchKernelGGL(k_adj_forward, dim3(nbc), dim3(kBlock), 0, s, C, F, qg, q, g, second_order, limiter_k, A, R);
     if (A.vgx)
-        hipLaunchKernelGGL((k_adj_face<GEO, GHOST, 1, true>), dim3(nbf), dim3(kBlock), 0, s, C, F, q, w, g,
-                           second_order, A, G, ghost);
+        hipLaunchKernelGGL((k_adj_face<GEO, GHOST, true>), dim3(nbb + nbf), dim3(kBlock), 0, s, C, F, q, w, g,
+                           second_order, A, G, ghost, nbb);
     else
-        hipLaunchKernelGGL((k_adj_face<GEO, GHOST, 1, false>), dim3(nbf), dim3(kBlock), 0, s, C, F, q, w, g,
-                           second_order, A, G, ghost);
-    if (A.nbf > 0)
-        hipLaunchKernelGGL((k_adj_face<GEO, GHOST, 2, false>), dim3((A.nbf + kBlock - 1) / kBlock), dim3(kBlock), 0, s, C, F,
-                           q, w, g, second_order, A, G, ghost);
+        hipLaunchKernelGGL((k_adj_face<GEO, GHOST, false>), dim3(nbb + nbf), dim3(kBlock), 0, s, C, F, q, w, g,
+                           second_order, A, G, ghost, nbb);
     hipLaunchKernelGGL((k_adj_cell1<GEO, GHOST>), dim3(nbc), dim3(kBlock), 0, s, C, F, q, second_order, limiter_k, A,
                        lam, G, ghost);
-    if (second_order || A.vgx) {   // gradients enter the residual (reconstruction or laminar terms)
-        hipLaunchKernelGGL((k_adj_face2<GEO, GHOST, 1>), dim3(nbf), dim3(kBlock), 0, s, C, F, qg, g, A, G, ghost);
-        if (A.nbf > 0)
-            hipLaunchKernelGGL((k_adj_face2<GEO, GHOST, 2>), dim3((A.nbf + kBlock - 1) / kBlock), dim3(kBlock), 0, s,
-                               C, F, qg, g, A, G, ghost);
-        hipLaunchKernelGGL(k_adj_cell2, dim3(nbc), dim3(kBlock), 0, s, C, F, A, lam, lam_g);
-    } else if (lam_g != lam) {
-        hipLaunchKernelGGL(k_fill0, dim3((4 * C.nT + kBlock - 1) / kBlock), dim3(kBlock), 0, s, lam_g, 4 * C.nT);
-    }
-    if (GEO && to_nodes) {
+    if (gg)
+        hipLaunchKernelGGL((k_adj_face2<GEO, GHOST>), dim3(nbb + nbf), dim3(kBlock), 0, s, C, F, qg, g, A, G, ghost, nbb);
+    if (gradients || R.g)
+        hipLaunchKernelGGL(k_adj_cell2, dim3(nbc), dim3(kBlock), 0, s, C, F, A, lam, lam_g, gg ? 1 : 0, R);
+    if (GEO && !R.g) {
         hipLaunchKernelGGL(k_geo_face, dim3(nbf), dim3(kBlock), 0, s, C, F, G);
         hipLaunchKernelGGL(k_geo_cell, dim3(nbc), dim3(kBlock), 0, s, C, F, G);
         hipLaunchKernelGGL(k_geo_node, dim3((G.nN + kBlock - 1) / kBlock), dim3(kBlock), 0, s, C, F, G);
@@ -876,28 +941,25 @@ void adjoint_passes(hipStream_t s, CellsT<double> C, FacesT<double> F, const dou
 }
 }  // namespace
 
-hipError_t launch_adjoint_stage(hipStream_t s, CellsT<double> C, FacesT<double> F, const double* qg, const double* q,
-                                const double* w, GasT<double> g, int second_order, double limiter_k, AdjBufs A,
-                                double* lam, double* lam_g, double* ghost, const GeoBufs* Gp) {
-    const GeoBufs G = Gp ? *Gp : GeoBufs{};
-    if (Gp && ghost) return hipErrorInvalidValue;   // no caller needs both
-    if (Gp) adjoint_passes<true, false>(s, C, F, qg, q, w, g, second_order, limiter_k, A, lam, lam_g, nullptr, G);
-    else if (ghost) adjoint_passes<false, true>(s, C, F, qg, q, w, g, second_order, limiter_k, A, lam, lam_g, ghost, G);
-    else adjoint_passes<false, false>(s, C, F, qg, q, w, g, second_order, limiter_k, A, lam, lam_g, nullptr, G);
-    return hipGetLastError();
-}
-
-hipError_t launch_adjoint_stage_metrics(hipStream_t s, CellsT<double> C, FacesT<double> F, const double* qg,
-                                        const double* q, const double* w, GasT<double> g, int second_order,
-                                        double limiter_k, AdjBufs A, double* lam, double* lam_g, const GeoBufs& G) {
-    adjoint_passes<true, false>(s, C, F, qg, q, w, g, second_order, limiter_k, A, lam, lam_g, nullptr, G, false);
+hipError_t launch_reverse_stage(hipStream_t s, CellsT<double> C, FacesT<double> F, const double* qg, const double* q,
+                                GasT<double> g, int second_order, double limiter_k, AdjBufs A, double* lam,
+                                const RevStage& R, double* ghost, const GeoBufs* Gp) {
+    if (!ghost == !Gp) return hipErrorInvalidValue;   // the boundary data's adjoints or the metrics'
+    A.add = 1;
+    A.add_lg = R.first ? 0 : 1;
+    GeoBufs G = Gp ? *Gp : GeoBufs{};
+    G.add = 1;
+    if (Gp) adjoint_passes<true, false>(s, C, F, qg, q, R.wseed, g, second_order, limiter_k, A, lam, lam, nullptr, G, R);
+    else adjoint_passes<false, true>(s, C, F, qg, q, R.wseed, g, second_order, limiter_k, A, lam, lam, ghost, G, R);
     return hipGetLastError();
 }
 
 hipError_t launch_adjoint_state(hipStream_t s, CellsT<double> C, FacesT<double> F, const double* q, const double* w,
                                 GasT<double> g, int second_order, double limiter_k, AdjBufs A, double* lam,
                                 const GeoBufs* Gp) {
-    return launch_adjoint_stage(s, C, F, q, q, w, g, second_order, limiter_k, A, lam, lam, nullptr, Gp);
+    if (Gp) adjoint_passes<true, false>(s, C, F, q, q, w, g, second_order, limiter_k, A, lam, lam, nullptr, *Gp);
+    else adjoint_passes<false, false>(s, C, F, q, q, w, g, second_order, limiter_k, A, lam, lam, nullptr, GeoBufs{});
+    return hipGetLastError();
 }
 
 // ------------------------------------------------------------------ tangent --

@@ -46,6 +46,8 @@ struct AdjBufs {
     double* vgx;     // [4][nF]
     double* vgy;
     double* vdq;
+    int add;         // the ghost rows' adjoints are added to
+    int add_lg;      // lgx, lgy are added to
 };
 
 // work arrays of the adjoint with respect to the mesh nodes
@@ -63,6 +65,21 @@ struct GeoBufs {
     const int32_t* n_ent;    // 2 f + end (face ends) or -(1 + 4 c + slot) (cell vertices)
     int32_t nN;
     double* xbar;            // [nN][2] output: (x, y) adjoint per node
+    int add;                 // fbar, abar are added to
+};
+
+// One stage of a reversed explicit step, real cells: q_s+1 = q + W dt coef with
+// q_s+1's adjoint g.  qbar and dtbar start with the step's first reversed stage;
+// g becomes the adjoint of q_s, which the last one adds to qbar.
+struct RevStage {
+    double* g = nullptr;          // null: no reversed step
+    const double* W = nullptr;    // the stage's residual
+    const double* dt = nullptr;
+    double coef = 0.0;
+    double* wseed = nullptr;      // g dt coef / A, the seed of the undivided residual
+    double* dtbar = nullptr;
+    double* qbar = nullptr;
+    int first = 0, last = 0;
 };
 
 // lam[k*nT + i] (real cells) = ((dR/dq)^T w)[i, k] for the inviscid residual
@@ -83,37 +100,26 @@ hipError_t launch_adjoint_state_sa(hipStream_t s, CellsT<double> C, FacesT<doubl
 
 // The explicit stage residual of explicitSolver::solve (solver.h:802-828)
 // takes its gradients from the step's start state qg and everything else
-// from the stage state q (A3).  lam = (dR/dq)^T w, lam_g = (dR/dqg)^T w; with
-// ghost non-null the adjoints of the farfield ghost states (boundary data)
-// are written into its ghost rows [k*nT + ghost cell].
-hipError_t launch_adjoint_stage(hipStream_t s, CellsT<double> C, FacesT<double> F, const double* qg, const double* q,
-                                const double* w, GasT<double> g, int second_order, double limiter_k, AdjBufs A,
-                                double* lam, double* lam_g, double* ghost, const GeoBufs* G = nullptr);
-
-// launch_adjoint_stage with the metric adjoints of the stage left in G.fbar /
-// G.abar (overwritten) and not converted to node adjoints
-hipError_t launch_adjoint_stage_metrics(hipStream_t s, CellsT<double> C, FacesT<double> F, const double* qg,
-                                        const double* q, const double* w, GasT<double> g, int second_order,
-                                        double limiter_k, AdjBufs A, double* lam, double* lam_g, const GeoBufs& G);
-// facc += G.fbar (8 x nF), aacc += G.abar (nC)
-hipError_t launch_acc_metrics(hipStream_t s, const GeoBufs& G, int32_t nF, int32_t nC, double* facc, double* aacc);
+// from the stage state q (A3); one stage of the reversed step, with the
+// adjoints of the farfield ghost states (boundary data) added to the ghost rows
+// [k*nT + ghost cell] of `ghost`, or the metric adjoints to G->fbar and G->abar
+// (one of the two).  lam is scratch.
+hipError_t launch_reverse_stage(hipStream_t s, CellsT<double> C, FacesT<double> F, const double* qg, const double* q,
+                                GasT<double> g, int second_order, double limiter_k, AdjBufs A, double* lam,
+                                const RevStage& R, double* ghost, const GeoBufs* G);
 // facc += metric adjoints (n, len) of the local time step for dtbar
 hipError_t launch_dt_vjp_geo(hipStream_t s, CellsT<double> C, FacesT<double> F, const double* q, GasT<double> g,
                              const double* dt, const double* dtbar, double cfl, double* facc);
 // G.xbar from the metric adjoints in G.fbar / G.abar
 hipError_t launch_geo_to_nodes(hipStream_t s, CellsT<double> C, FacesT<double> F, const GeoBufs& G);
 
-// reverse of one explicit stage update qk_s+1 = q + W_s dt coef (real cells)
-hipError_t launch_rev_stage(hipStream_t s, const double* gk, const double* W, const double* dt, const double* area,
-                            double coef, int32_t nC, int32_t nT, double* wseed, double* dtbar, double* qbar);
-// y = a x (overwrite) or y += a x, over the real-cell rows of the 4 planes
-hipError_t launch_axpy4(hipStream_t s, const double* x, double a, int32_t nC, int32_t nT, int overwrite, double* y);
 // acc[k][j] += ghost[k*nT + cells[j]]
 hipError_t launch_ghost_acc(hipStream_t s, const double* ghost, const int32_t* cells, int32_t n, int32_t nT,
                             double* acc);
 
-// dt = cfl A / sum_f max(eig_o, eig_n) len (solver.h:308-356): qbar += (d dt / d q)^T dtbar
+// dt = cfl A / sum_f max(eig_o, eig_n) len (solver.h:308-356): out = qbar + (d dt / d q)^T dtbar
 hipError_t launch_dt_vjp(hipStream_t s, CellsT<double> C, FacesT<double> F, const double* q, GasT<double> g,
-                         const double* dt, const double* dtbar, double cfl, double* ebar, double* qbar);
+                         const double* dt, const double* dtbar, double cfl, double* ebar, const double* qbar,
+                         double* out);
 
 }  // namespace afx

@@ -2403,12 +2403,12 @@ int afx_rans_dcl_dalpha(afx_rans* h, const char* patch, int32_t steps, int32_t e
             dfar.push_back(rho * v[0] * c * std::cos(v[1]));
         }
     const int32_t nfar = (int32_t)far.size();
-    DBuf<double> ck, seg, keepb, g, qb, lam, lamg, wseed, dtb, eb, gh, gacc;
+    DBuf<double> ck, seg, keepb, g, qb, lam, wseed, dtb, eb, gh, gacc;
     DBuf<int32_t> dfarc;
     HIPCHK(ck.alloc(nck * nq));
     HIPCHK(seg.alloc((size_t)std::min(every, steps) * nq));
     HIPCHK(keepb.alloc(5 * nq));
-    for (DBuf<double>* b : {&g, &qb, &lam, &lamg, &wseed, &gh}) HIPCHK(b->alloc(nq));
+    for (DBuf<double>* b : {&g, &qb, &lam, &wseed, &gh}) HIPCHK(b->alloc(nq));
     HIPCHK(dtb.alloc(nT));
     HIPCHK(eb.alloc(h->nF));
     HIPCHK(gacc.alloc(4 * (size_t)std::max(nfar, 1)));
@@ -2416,6 +2416,7 @@ int afx_rans_dcl_dalpha(afx_rans* h, const char* patch, int32_t steps, int32_t e
     if (nfar) HIPCHK(dfarc.upload(far, s));
     HIPCHK(hipMemsetAsync(wseed.p, 0, nq * 8, s));
     HIPCHK(hipMemsetAsync(gacc.p, 0, 4 * (size_t)std::max(nfar, 1) * 8, s));
+    HIPCHK(hipMemsetAsync(gh.p, 0, nq * 8, s));
     double* keep[5];
     for (int k = 0; k < 5; ++k) keep[k] = keepb.p + k * nq;
 
@@ -2443,22 +2444,17 @@ int afx_rans_dcl_dalpha(afx_rans* h, const char* patch, int32_t steps, int32_t e
         for (int32_t n = end - 1; n >= start; --n) {
             double* qn = seg.p + (size_t)(n - start) * nq;
             if ((rc = explicit_step64(h, qn, h->qk.p, relaxation, keep))) return rc;   // dt, W_s, qk_1, qk_2
-            HIPCHK(hipMemsetAsync(qb.p, 0, nq * 8, s));
-            HIPCHK(hipMemsetAsync(dtb.p, 0, (size_t)nT * 8, s));
             for (int st = 2; st >= 0; --st) {
-                HIPCHK(launch_rev_stage(s, g.p, keep[st], h->dt.p, h->area.p, alpha[st] * relaxation, nC, nT,
-                                        wseed.p, dtb.p, qb.p));
-                const double* qs = st == 0 ? qn : keep[2 + st];
-                HIPCHK(launch_adjoint_stage(s, h->cells64(), h->faces64(), qn, qs, wseed.p, h->gas64(),
-                                            h->opts.second_order, h->opts.limiter_k, A, lam.p, lamg.p, gh.p));
-                HIPCHK(launch_ghost_acc(s, gh.p, dfarc.p, nfar, nT, gacc.p));
-                HIPCHK(launch_axpy4(s, lamg.p, 1.0, nC, nT, 0, qb.p));
-                HIPCHK(launch_axpy4(s, lam.p, 1.0, nC, nT, st > 0 ? 1 : 0, st > 0 ? g.p : qb.p));
+                const RevStage R{g.p,   keep[st], h->dt.p, alpha[st] * relaxation, wseed.p, dtb.p, qb.p,
+                                 st == 2, st == 0};
+                HIPCHK(launch_reverse_stage(s, h->cells64(), h->faces64(), qn, st == 0 ? qn : keep[2 + st], h->gas64(),
+                                            h->opts.second_order, h->opts.limiter_k, A, lam.p, R, gh.p, nullptr));
             }
-            HIPCHK(launch_dt_vjp(s, h->cells64(), h->faces64(), qn, h->gas64(), h->dt.p, dtb.p, h->cfl, eb.p, qb.p));
-            HIPCHK(launch_copy(s, qb.p, g.p, (int64_t)nq));
+            HIPCHK(launch_dt_vjp(s, h->cells64(), h->faces64(), qn, h->gas64(), h->dt.p, dtb.p, h->cfl, eb.p, qb.p,
+                                 g.p));
         }
     }
+    HIPCHK(launch_ghost_acc(s, gh.p, dfarc.p, nfar, nT, gacc.p));
     std::vector<double> ga(4 * (size_t)std::max(nfar, 1));
     HIPCHK(hipMemcpyAsync(ga.data(), gacc.p, ga.size() * 8, hipMemcpyDeviceToHost, s));
     HIPCHK(hipStreamSynchronize(s));
@@ -2482,11 +2478,11 @@ int afx_rans_dcl_dnodes(afx_rans* h, const char* patch, int32_t steps, int32_t e
     const int32_t nC = h->nC, nT = h->nT, nF = h->nF;
     const size_t nq = (size_t)NV * nT;
     const int nck = (steps + every - 1) / every;
-    DBuf<double> ck, seg, keepb, g, qb, lam, lamg, wseed, dtb, eb, facc, aacc;
+    DBuf<double> ck, seg, keepb, g, qb, lam, wseed, dtb, eb, facc, aacc;
     HIPCHK(ck.alloc(nck * nq));
     HIPCHK(seg.alloc((size_t)std::min(every, steps) * nq));
     HIPCHK(keepb.alloc(5 * nq));
-    for (DBuf<double>* b : {&g, &qb, &lam, &lamg, &wseed}) HIPCHK(b->alloc(nq));
+    for (DBuf<double>* b : {&g, &qb, &lam, &wseed}) HIPCHK(b->alloc(nq));
     HIPCHK(dtb.alloc(nT));
     HIPCHK(eb.alloc(nF));
     HIPCHK(facc.alloc(8 * (size_t)nF));
@@ -2546,6 +2542,9 @@ int afx_rans_dcl_dnodes(afx_rans* h, const char* patch, int32_t steps, int32_t e
     const AdjBufs A = adj_bufs(h);
     GeoBufs G{h->g_fbar.p, h->g_abar.p, h->g_fnode.p, h->g_cnode.p, h->g_nodex.p, h->g_nodey.p, h->g_fend.p,
               h->g_fcen.p, h->g_cvert.p, h->g_noff.p, h->g_nent.p, h->nN, h->g_xbar.p};
+    GeoBufs sums = G;   // over all stages and steps
+    sums.fbar = facc.p;
+    sums.abar = aacc.p;
     for (int k = nck - 1; k >= 0; --k) {
         const int32_t start = k * every, end = std::min(steps, start + every);
         HIPCHK(launch_copy(s, ck.p + (size_t)k * nq, seg.p, (int64_t)nq));
@@ -2556,22 +2555,16 @@ int afx_rans_dcl_dnodes(afx_rans* h, const char* patch, int32_t steps, int32_t e
         for (int32_t n = end - 1; n >= start; --n) {
             double* qn = seg.p + (size_t)(n - start) * nq;
             if ((rc = explicit_step64(h, qn, h->qk.p, relaxation, keep))) return rc;   // dt, W_s, qk_1, qk_2
-            HIPCHK(hipMemsetAsync(qb.p, 0, nq * 8, s));
-            HIPCHK(hipMemsetAsync(dtb.p, 0, (size_t)nT * 8, s));
             for (int st = 2; st >= 0; --st) {
-                HIPCHK(launch_rev_stage(s, g.p, keep[st], h->dt.p, h->area.p, alpha[st] * relaxation, nC, nT,
-                                        wseed.p, dtb.p, qb.p));
-                const double* qs = st == 0 ? qn : keep[2 + st];
-                HIPCHK(launch_adjoint_stage_metrics(s, h->cells64(), h->faces64(), qn, qs, wseed.p, h->gas64(),
-                                                    h->opts.second_order, h->opts.limiter_k, A, lam.p, lamg.p, G));
-                HIPCHK(launch_acc_metrics(s, G, nF, nC, facc.p, aacc.p));
-                HIPCHK(launch_axpy4(s, lamg.p, 1.0, nC, nT, 0, qb.p));
-                HIPCHK(launch_axpy4(s, lam.p, 1.0, nC, nT, st > 0 ? 1 : 0, st > 0 ? g.p : qb.p));
+                const RevStage R{g.p,   keep[st], h->dt.p, alpha[st] * relaxation, wseed.p, dtb.p, qb.p,
+                                 st == 2, st == 0};
+                HIPCHK(launch_reverse_stage(s, h->cells64(), h->faces64(), qn, st == 0 ? qn : keep[2 + st], h->gas64(),
+                                            h->opts.second_order, h->opts.limiter_k, A, lam.p, R, nullptr, &sums));
             }
-            HIPCHK(launch_dt_vjp(s, h->cells64(), h->faces64(), qn, h->gas64(), h->dt.p, dtb.p, h->cfl, eb.p, qb.p));
+            HIPCHK(launch_dt_vjp(s, h->cells64(), h->faces64(), qn, h->gas64(), h->dt.p, dtb.p, h->cfl, eb.p, qb.p,
+                                 g.p));
             HIPCHK(launch_dt_vjp_geo(s, h->cells64(), h->faces64(), qn, h->gas64(), h->dt.p, dtb.p, h->cfl,
                                      facc.p));
-            HIPCHK(launch_copy(s, qb.p, g.p, (int64_t)nq));
         }
     }
     HIPCHK(launch_copy(s, facc.p, G.fbar, 8 * (int64_t)nF));
