@@ -980,8 +980,8 @@ __global__ void __launch_bounds__(kBlock) k_residual_tile(TilesT<T> S, const T* 
 // LDS, and the gradients, which A3 takes from the step's start, are formed once
 // per step.  Bound by the latency of one tile's FP64 chain on small meshes and
 // by FP64 issue on large ones.  A step of a 16k-cell inviscid mesh with its
-// norm went from 109 to 93 us, six SA steps of 250k cells with their transfers
-// from 3.18 to 2.94 ms.
+// norm went from 109 to 93 us (62 with the tiles of 128 cells that such a mesh
+// takes now), six SA steps of 250k cells with their transfers from 3.18 to 2.94 ms.
 template <typename T, int NV, int MODE>
 __global__ void __launch_bounds__(kBlock) k_stage_tile(TilesT<T> S, const T* __restrict__ q, int32_t nT, int32_t nC,
                                                        const T* __restrict__ area, const T* __restrict__ lsq,

@@ -635,8 +635,8 @@ int afx_aeroelastic_solve(afx_aeroelastic* h, const afx_coupling_opts* o, afx_co
             const V3 u = follow(b, h->disp, h->na[k], h->nb[k], h->nw[k], p);
             for (int d = 0; d < 3; ++d) xyz[3 * k + d] = p[d] + u[d];
         }
-        if ((rc = afx_vlm_set_nodes(h->v, xyz.data()))) return rc;
-        if ((rc = afx_vlm_build(h->v))) return rc;
+        if ((rc = afx::vlm_queue_nodes(h->v, xyz.data()))) return rc;
+        if ((rc = afx::vlm_queue_build(h->v))) return rc;
         if (!h->have_factor) {
             if ((rc = afx_vlm_factor(h->v))) return rc;
             h->have_factor = true;

@@ -122,10 +122,10 @@ __device__ inline int wave_winner(unsigned hi, unsigned lo) {
 // Bound by the latency of that exchange (a word takes about 0.55 us from one
 // compute unit to another) and, with one workgroup, by the column's chain of
 // maximum, LDS exchange, division and update.  Keys go to a mailbox of each
-// reader: polled by all, one row of keys cost 4.4 us a column at 64 workgroups
-// where this costs 2.8.  A panel of 256, 2 048 and 16 384 rows takes 140, 320
-// and 370 us; with a row's 128 columns exchanged and updated per column, 120
-// rows to a workgroup, it took 590, 560 and 690.
+// reader: one row of keys polled by all cost 1.1 us more a column at 64
+// workgroups.  A panel of 256, 2 048 and 16 384 rows takes 133, 320 and 352 us
+// alone; with a row's 128 columns exchanged and updated per column, 120 rows to a
+// workgroup, it took 520, 554 and 554.
 __device__ inline unsigned long long tagged(unsigned seq, float v) {
     return ((unsigned long long)seq << 32) | (unsigned long long)__float_as_uint(v);
 }
@@ -1563,6 +1563,15 @@ int afx_vlm_set_flow(afx_vlm* h, const afx_vlm_flow* f) {
 }
 
 int afx_vlm_set_nodes(afx_vlm* h, const double* xyz) {
+    const int rc = afx::vlm_queue_nodes(h, xyz);
+    if (rc) return rc;
+    VCHK(hipStreamSynchronize(h->dense->s));
+    return AFX_OK;
+}
+
+}  // extern "C"
+
+int afx::vlm_queue_nodes(afx_vlm* h, const double* xyz) {
     if (!h || !xyz) return api_fail(AFX_EARG, "null argument");
     std::copy(xyz, xyz + 3 * (size_t)h->nn, h->xyz.begin());
     VCHK(hipStreamSynchronize(h->dense->s));   // the stage is free
@@ -1571,6 +1580,8 @@ int afx_vlm_set_nodes(afx_vlm* h, const double* xyz) {
     h->built = h->solved = false;
     return AFX_OK;
 }
+
+extern "C" {
 
 int afx_vlm_get_nodes(const afx_vlm* h, double* xyz) {
     if (!h || !xyz) return api_fail(AFX_EARG, "null argument");
@@ -1586,6 +1597,15 @@ int afx_vlm_get_rings(const afx_vlm* h, int32_t* ring_nodes, int32_t* soff) {
 }
 
 int afx_vlm_build(afx_vlm* h) {
+    const int rc = afx::vlm_queue_build(h);
+    if (rc) return rc;
+    VCHK(hipStreamSynchronize(h->dense->s));
+    return AFX_OK;
+}
+
+}  // extern "C"
+
+int afx::vlm_queue_build(afx_vlm* h) {
     if (!h) return api_fail(AFX_EARG, "null argument");
     if (!h->flow_set) return api_fail(AFX_ESTATE, "flow not set");
     const afx_vlm_flow& f = h->flow;
@@ -1609,6 +1629,8 @@ int afx_vlm_build(afx_vlm* h) {
     h->solved = false;
     return AFX_OK;
 }
+
+extern "C" {
 
 int afx_vlm_factor(afx_vlm* h) {
     if (!h) return api_fail(AFX_EARG, "null argument");
@@ -1721,7 +1743,7 @@ int afx_vlm_nonlinear_solve(afx_vlm* h, const afx_polar* P, double relaxation, d
             return api_fail(AFX_EARG, "section airfoil index out of range");
     const afx_vlm_flow& f = h->flow;
     const int ns = h->ns;
-    int rc = afx_vlm_build(h);
+    int rc = afx::vlm_queue_build(h);
     if (rc) return rc;
     if ((rc = afx_vlm_factor(h))) return rc;
     // station geometry (wingStation / wing, surface.cpp): area = sum of ring
