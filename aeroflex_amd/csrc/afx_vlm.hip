@@ -116,8 +116,11 @@ __device__ inline int wave_winner(unsigned hi, unsigned lo) {
 // j + 2 before every workgroup has posted j + 1, which each does only after
 // reading column j's words; the published rows alternate by sub-panel alike.
 // With one workgroup (m <= R) nothing is exchanged.  Every wait is bounded: a
-// wave that polls longer than SPIN_LIMIT raises `abort` and every workgroup
-// returns.
+// wave that polls longer than spin_limit raises `abort` and every workgroup
+// returns.  What is queued behind the panel then runs on an unfinished one:
+// src and dst of rows that were not placed keep an earlier panel's values, all
+// of them rows of the panel, so every access stays inside the matrix, and the
+// host refuses the factor.
 //
 // Bound by the latency of that exchange (a word takes about 0.55 us from one
 // compute unit to another) and, with one workgroup, by the column's chain of
@@ -130,11 +133,11 @@ __device__ inline unsigned long long tagged(unsigned seq, float v) {
     return ((unsigned long long)seq << 32) | (unsigned long long)__float_as_uint(v);
 }
 // wait (bounded) for a value | sequence word of this sequence; false on timeout
-__device__ inline bool wait_tagged(const unsigned long long* p, unsigned seq, float& v) {
+__device__ inline bool wait_tagged(const unsigned long long* p, unsigned seq, unsigned limit, float& v) {
     unsigned spins = 0;
     unsigned long long w;
     while (((w = __hip_atomic_load(p, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT)) >> 32) != seq) {
-        if (++spins > SPIN_LIMIT) { v = 0.f; return false; }
+        if (++spins > limit) { v = 0.f; return false; }
         __builtin_amdgcn_s_sleep(1);
     }
     v = __uint_as_float((unsigned)(w & 0xFFFFFFFFull));
@@ -145,7 +148,8 @@ __global__ __launch_bounds__(256, 1) void k_panel_lu(float* __restrict__ A, int 
                                                      int* __restrict__ ipiv, int* __restrict__ src,
                                                      int* __restrict__ dst, unsigned long long* keys,
                                                      unsigned long long* vals, unsigned long long* prow,
-                                                     unsigned* abort_flag, int* __restrict__ info) {
+                                                     unsigned* abort_flag, unsigned spin_limit,
+                                                     int* __restrict__ info) {
     __shared__ float4 slab4[LU_NB * PANEL_R / 4];     // panel column c at slab[c * PANEL_R]
     __shared__ float4 U4[(LU_NB - SUB) * SUB / 4];    // U of the sub-panel's rows, column by column
     __shared__ float4 Ls4[SUB * SUB / 4];             // L of the sub-panel's rows
@@ -244,7 +248,7 @@ __global__ __launch_bounds__(256, 1) void k_panel_lu(float* __restrict__ A, int 
                             kk = k > kk ? k : kk;
                         }
                         if (__all(ok)) break;
-                        if (++spins > SPIN_LIMIT ||
+                        if (++spins > spin_limit ||
                             ((spins & 63u) == 0u &&
                              __hip_atomic_load(abort_flag, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) != 0u)) {
                             late = true;
@@ -260,7 +264,7 @@ __global__ __launch_bounds__(256, 1) void k_panel_lu(float* __restrict__ A, int 
                         const unsigned lo = (unsigned)__builtin_amdgcn_readlane((int)(unsigned)kk, wl);
                         const unsigned hi = (unsigned)__builtin_amdgcn_readlane((int)(unsigned)(kk >> 32), wl);
                         float f = 0.f;
-                        if (lane < SUB) late = !wait_tagged(&vbox[2 * wq * SUB + lane], seq, f);
+                        if (lane < SUB) late = !wait_tagged(&vbox[2 * wq * SUB + lane], seq, spin_limit, f);
                         if (lane < SUB) reinterpret_cast<float*>(urow4[par])[lane] = f;
                         if (lane == 0) s_win[par] = ((unsigned long long)hi << 32) | lo;
                     }
@@ -329,7 +333,7 @@ __global__ __launch_bounds__(256, 1) void k_panel_lu(float* __restrict__ A, int 
             float l = 0.f;
             if (i < k) {
                 if (nwg == 1) l = slab[(c0 + i) * PANEL_R + lrow[k]];
-                else ok = wait_tagged(&rest[k * LU_NB + i], (unsigned)(j0 + c0 + k + 1), l);
+                else ok = wait_tagged(&rest[k * LU_NB + i], (unsigned)(j0 + c0 + k + 1), spin_limit, l);
             }
             Ls[t] = l;
         }
@@ -346,7 +350,8 @@ __global__ __launch_bounds__(256, 1) void k_panel_lu(float* __restrict__ A, int 
                 for (int k = 0; k < SUB; ++k) {
                     const unsigned seq = (unsigned)(j0 + c0 + k + 1);
                     v[k] = __uint_as_float((unsigned)x[k]);
-                    if ((unsigned)(x[k] >> 32) != seq) ok = wait_tagged(&rest[k * LU_NB + SUB + t], seq, v[k]) && ok;
+                    if ((unsigned)(x[k] >> 32) != seq)
+                        ok = wait_tagged(&rest[k * LU_NB + SUB + t], seq, spin_limit, v[k]) && ok;
                 }
             }
         }
@@ -1127,14 +1132,19 @@ hipError_t launch_gemm_sub_f32(hipStream_t s, const float* A, const float* B, fl
 }
 
 __global__ void k_panel_reset(unsigned long long* keys, unsigned long long* vals, unsigned long long* prow, int* perm,
-                              int n, int nwg, unsigned* abort_flag, unsigned* trsv_abort, int* info) {
+                              int* src, int* dst, int n, int nwg, unsigned* abort_flag, unsigned* trsv_abort,
+                              int* info) {
     const int stride = gridDim.x * blockDim.x, i0 = blockIdx.x * blockDim.x + threadIdx.x;
     // the words carry the column sequence j0 + j + 1, which repeats from one
     // factorisation to the next
     for (int q = i0; q < 2 * KEY_STRIDE * nwg; q += stride) keys[q] = 0ull;
     for (int q = i0; q < 2 * SUB * nwg; q += stride) vals[q] = 0ull;
     for (int q = i0; q < 2 * SUB * LU_NB; q += stride) prow[q] = 0ull;
-    for (int q = i0; q < n; q += stride) perm[q] = q;
+    // no interchanges in any panel, for one that gives up before it writes its own
+    for (int q = i0; q < n; q += stride) {
+        perm[q] = q;
+        src[q] = dst[q] = q % LU_NB;
+    }
     if (i0 == 0) {
         *abort_flag = 0u;
         *trsv_abort = 0u;   // a new factorisation also re-arms the triangular solves
@@ -1181,6 +1191,7 @@ struct afx_dense {
         int info;
         unsigned aborted;
     }* host = nullptr;
+    unsigned spin_limit = SPIN_LIMIT;   // of the panel's waits
     bool factored = false;
     ~afx_dense() {
         for (void* p : {(void*)A64, (void*)A32, (void*)ipiv, (void*)perm, (void*)b, (void*)x, (void*)r,
@@ -1255,7 +1266,8 @@ int dense_factor(afx_dense* h, int32_t* info_out) {
     dim3 tg((n + 63) / 64, (n + 63) / 64);
     k_to_cm32<<<tg, 256, 0, s>>>(h->A64, n, h->A32, lda);
     VCHK(hipGetLastError());
-    k_panel_reset<<<64, 256, 0, s>>>(h->keys, h->vals, h->prow, h->perm, n, (n + PANEL_R - 1) / PANEL_R, h->pabort, h->abort, h->info);
+    k_panel_reset<<<64, 256, 0, s>>>(h->keys, h->vals, h->prow, h->perm, h->src, h->dst, n,
+                                     (n + PANEL_R - 1) / PANEL_R, h->pabort, h->abort, h->info);
     VCHK(hipGetLastError());
     // Right-looking blocked LU with a look-ahead of one panel.  After panel
     // k (columns [j0, c1)) is factored on s, s2 interchanges the rows of the
@@ -1277,12 +1289,13 @@ int dense_factor(afx_dense* h, int32_t* info_out) {
         const int nwg = (m + PANEL_R - 1) / PANEL_R;
         if (nwg == 1) {   // waits for no other workgroup: needs no cooperative launch
             k_panel_lu<<<1, 256, 0, s>>>(A, lda, m, nbc, j0, h->ipiv, h->src, h->dst, h->keys, h->vals, h->prow,
-                                         h->pabort, h->info);
+                                         h->pabort, h->spin_limit, h->info);
             VCHK(hipGetLastError());
         } else {
             int ldai = lda, mi = m, nbci = nbc, j0i = j0;
             void* args[] = {&A,       &ldai,    &mi,      &nbci,    &j0i,       &h->ipiv, &h->src,
-                            &h->dst,  &h->keys, &h->vals, &h->prow, &h->pabort, &h->info};
+                            &h->dst,  &h->keys, &h->vals, &h->prow, &h->pabort, &h->spin_limit,
+                            &h->info};
             VCHK(hipLaunchCooperativeKernel((const void*)k_panel_lu, dim3(nwg), dim3(256), args, 0, s));
         }
         const int c1 = j0 + nbc, c2 = std::min(n, c1 + LU_NB), rest = n - c1;
@@ -1468,6 +1481,15 @@ int afx_dense_raise_abort(afx_dense* h) {
     const unsigned one = 1u;
     VCHK(hipMemcpyAsync(h->abort, &one, sizeof(unsigned), hipMemcpyHostToDevice, h->s));
     VCHK(hipStreamSynchronize(h->s));
+    return AFX_OK;
+}
+
+// Test hook: the panels' waits give up after `polls` polls (0: the kernels' own
+// limit), so that a factorisation takes the way of a timed-out wait with every
+// kernel still ending normally.
+int afx_dense_limit_polls(afx_dense* h, uint32_t polls) {
+    if (!h) return api_fail(AFX_EARG, "null argument");
+    h->spin_limit = polls ? std::min(polls, SPIN_LIMIT) : SPIN_LIMIT;
     return AFX_OK;
 }
 

@@ -95,6 +95,7 @@ def _load():
         "afx_dense_solve": (C.c_int, [_P, _dp, _f64, _i32, _dp, C.POINTER(SolveInfo)]),
         "afx_dense_get_lu": (C.c_int, [_P, C.POINTER(C.c_float), ip]),
         "afx_dense_raise_abort": (C.c_int, [_P]),
+        "afx_dense_limit_polls": (C.c_int, [_P, C.c_uint32]),
         "afx_beam_create": (C.c_int, [_i32, _dp, _i32, ip, _dp, _i32, ip, C.POINTER(_P)]),
         "afx_beam_destroy": (C.c_int, [_P]),
         "afx_beam_solve": (C.c_int, [_P, _dp, _dp]),
@@ -245,6 +246,11 @@ class Dense(Handle):
         """Test hook: raise the triangular solves' abort flag, as a timed-out
         wait does."""
         _chk(_lib.afx_dense_raise_abort(self.h))
+
+    def limit_polls(self, polls):
+        """Test hook: the factorisation's waits give up after this many polls
+        (0: the kernels' own limit)."""
+        _chk(_lib.afx_dense_limit_polls(self.h, polls))
 
     def lu(self):
         lu = np.zeros((self.n, self.n), np.float32, order="F")

@@ -170,6 +170,11 @@ int afx_dense_get_lu(afx_dense* h, float* lu_colmajor, int32_t* ipiv);
  * afx_dense_solve then fails (AFX_EHIP) and discards the factorisation; the
  * next afx_dense_factor clears the flag. */
 int afx_dense_raise_abort(afx_dense* h);
+/* Test hook (no counterpart in the reference): the bounded waits of
+ * afx_dense_factor give up after this many polls (0: the kernels' own limit),
+ * so that a factorisation of more than 256 rows fails as one whose wait timed
+ * out (AFX_EHIP). */
+int afx_dense_limit_polls(afx_dense* h, uint32_t polls);
 
 /* --------------------------------------------------------------- beam --- */
 

@@ -193,6 +193,37 @@ def test_solve_after_a_timed_out_wait(vlm):
     np.testing.assert_allclose(x2, x, rtol=0, atol=1e-13 * np.abs(xr).max())
 
 
+# a first factorisation, whose interchange tables no panel has written yet, and
+# one after another factor; a panel of one tall stretch and ragged rows
+@pytest.mark.parametrize("n", [257, 600])
+@pytest.mark.parametrize("before", [False, True])
+def test_factor_after_a_timed_out_wait(vlm, n, before):
+    """A panel whose waits give up (forced from the host by a limit of one poll:
+    the words of another workgroup take hundreds of cycles) leaves its tables
+    unwritten, while the kernels queued behind it go on: they stay inside the
+    matrix, the factor is refused, and the next one is right again."""
+    print(f"[vlm] timed-out panel n={n} before={before}", flush=True)
+    rng = np.random.default_rng(n)
+    A = rng.normal(size=(n, n)) + n * np.eye(n)
+    A = A[rng.permutation(n)]   # interchanges in every panel
+    b = rng.normal(size=n)
+    d = vlm.Dense(n)
+    d.set(A)
+    if before:
+        d.factor()
+    d.limit_polls(1)
+    with pytest.raises(vlm.VlmError, match="pivot exchange timed out"):
+        d.factor()
+    with pytest.raises(vlm.VlmError, match="no factorisation"):
+        d.solve(b)
+    d.limit_polls(0)
+    assert d.factor() == 0
+    x, info = d.solve(b)
+    assert info.converged
+    xr = np.linalg.solve(A, b)
+    np.testing.assert_allclose(x, xr, rtol=0, atol=1e-12 * np.abs(xr).max())
+
+
 @pytest.mark.parametrize("alpha", [2.0, 8.0])
 def test_gamma_forces_cl_match_oracle(vlm, ov, alpha):
     print(f"[vlm] solve alpha={alpha}", flush=True)
