@@ -1907,6 +1907,64 @@ int afx_rans_precond_apply(afx_rans* h, const double* x, double* y) {
     return afx_rans_precond_apply_nu(h, x, nullptr, y, nullptr);
 }
 
+// Test hook: the end of one Arnoldi step on the caller's basis and vector, in the
+// order of the process (nv planes of the real cells by colour position with
+// DILU, otherwise one row of nv planes of all cells).  basis: m columns of n,
+// orthonormal; w: what the product would have left.  Pass 1's sums are taken on
+// the host; pass 2, the step and the next vector run as in the solve.
+int afx_rans_arnoldi_step(afx_rans* h, int32_t m, int64_t n, const double* basis, const double* w, double* next,
+                          double* norm, int32_t* flags) {
+    int rc = check_handle(h);
+    if (rc) return rc;
+    if (!h->lhs_ready || h->mf) return fail(AFX_ESTATE, "call afx_rans_implicit_fill first");
+    const bool colour = h->precond == 1;
+    const int nv = h->nv, N = colour ? nv : 1, cap = h->gm_restart + 1;
+    const int64_t len = colour ? h->nC : (int64_t)nv * h->nT;
+    if (m < 1 || m >= h->gm_restart || n != N * len || !basis || !w || !next || !norm || !flags)
+        return fail(AFX_EARG, "bad Arnoldi step");
+    hipStream_t s = h->stream;
+    std::vector<double> V(basis_doubles((size_t)len, N, h->gm_restart), 0.0), g((size_t)m, 0.0), dots((size_t)m, 0.0);
+    auto at = [&](int64_t i, int k) {   // entry i of column k
+        const int64_t r = i / len, p = i % len;
+        return (size_t)(((p >> 6) * N + r) * cap * 64 + (p & 63) + 64 * k);
+    };
+    for (int k = 0; k < m; ++k)
+        for (int64_t i = 0; i < n; ++i) {
+            V[at(i, k)] = basis[(size_t)k * n + i];
+            dots[k] += basis[(size_t)k * n + i] * w[i];
+        }
+    GmDev G = h->gm_dev(nullptr);
+    G.tol = 0.0;
+    const std::vector<double> ones((size_t)m, 1.0), zeros((size_t)m, 0.0);
+    g[m - 1] = 1.0;
+    const double hdr[4] = {1.0, 1.0, 1.0, 0.0};
+    const int on[4] = {1, 0, 0, 0};
+    auto up = [&](void* to, const void* from, size_t bytes) {
+        return hipMemcpyAsync(to, from, bytes, hipMemcpyHostToDevice, s);
+    };
+    HIPCHK(up(h->kV.p, V.data(), V.size() * 8));
+    HIPCHK(up(h->kw.p, w, (size_t)n * 8));
+    HIPCHK(up(G.sums, dots.data(), dots.size() * 8));
+    HIPCHK(up(G.hdr, hdr, sizeof(hdr)));
+    HIPCHK(up(G.cs, ones.data(), (size_t)m * 8));   // no rotations before this one
+    HIPCHK(up(G.sn, zeros.data(), (size_t)m * 8));
+    HIPCHK(up(G.g, g.data(), (size_t)m * 8));
+    HIPCHK(up(G.flags, on, sizeof(on)));
+    HIPCHK(hipStreamSynchronize(s));
+    const ColourOrder O = h->colours();
+    HIPCHK(launch_gm_step(s, G, colour ? &O : nullptr, nv, h->kV.p, n, m - 1, false, h->kw.p, 1));
+    if (colour) HIPCHK(launch_dilu_apply_next(s, nv, O, h->colour_matrix(), G, h->kw.p, h->kV.p, m, h->kz.p));
+    else HIPCHK(launch_next_vector(s, G, h->kw.p, h->kV.p, m, h->ktmp.p, n));
+    double back[3];
+    HIPCHK(hipMemcpyAsync(V.data(), h->kV.p, V.size() * 8, hipMemcpyDeviceToHost, s));
+    HIPCHK(hipMemcpyAsync(back, G.hdr, sizeof(back), hipMemcpyDeviceToHost, s));
+    HIPCHK(hipMemcpyAsync(flags, G.flags, sizeof(on), hipMemcpyDeviceToHost, s));
+    HIPCHK(hipStreamSynchronize(s));
+    for (int64_t i = 0; i < n; ++i) next[i] = flags[0] ? V[at(i, m)] : 0.0;
+    *norm = flags[0] ? 1.0 / back[2] : 0.0;
+    return AFX_OK;
+}
+
 int afx_rans_cell_colours(afx_rans* h, int32_t* colours, int32_t* ncolours) {
     int rc = check_handle(h, false);
     if (rc) return rc;

@@ -842,7 +842,8 @@ __global__ void __launch_bounds__(kBlock) k_colour_update(int32_t nC, int32_t nT
 //   (2) every block adds h1 up, then w -= V h1, and h2 = V^T w and |w|^2 of the
 //       result, block sums in the second half of partial;
 //   (3) one block: h2, |w - V h2|^2 = |w|^2 - |h2|^2 (V orthonormal, h2 only the
-//       rounding of pass 1), the Givens step, flags and scale;
+//       rounding of pass 1; at a breakdown, where w is rounding too, summed from
+//       the vector), the Givens step, flags and scale;
 //   (4) the next basis vector a (w - V h2), formed where it is first read (the
 //       forward sweeps).
 // So the basis is read three times and a step of two colours is six launches.
@@ -1019,8 +1020,12 @@ __global__ void __launch_bounds__(64 * N) k_gs_update_small(const double* __rest
 // column and rotation i, and the chain of rotations runs on lane reads (from
 // memory, one thread's chain took 7.8 us for 30 columns).  show: the host
 // reads the flags next (the write to its memory costs about a microsecond).
-__global__ void __launch_bounds__(576) k_gm_step(GmDev G, int j, int show, const double* __restrict__ sums2, int nblk) {
-    __shared__ double h2[kGsMax + 4];
+// The vectors are N rows of len positions.
+constexpr int kStepWaves = 9;
+__global__ void __launch_bounds__(64 * kStepWaves) k_gm_step(GmDev G, int j, int show, const double* __restrict__ sums2,
+                                                             int nblk, const double* __restrict__ V, int N, int64_t len,
+                                                             const double* __restrict__ w) {
+    __shared__ double h2[kGsMax + 4], left[kStepWaves];
     const int k = threadIdx.x / 16, part = threadIdx.x % 16, lane = threadIdx.x;
     const int m = G.m;
     const int on = G.flags[0], total = G.flags[2] + 1;
@@ -1033,13 +1038,37 @@ __global__ void __launch_bounds__(576) k_gm_step(GmDev G, int j, int show, const
     if (!on) return;
     if (part == 0 && k <= j + 1) h2[k] = t;
     __syncthreads();
-    if (!first) return;
-    const double c2 = lane <= j ? h2[lane] : 0.0;
+    const int at = lane & 63;
+    const double c2 = at <= j ? h2[at] : 0.0;
     if (lane <= j) G.h2[lane] = c2;
     double hh = c2 * c2;
 #pragma unroll
     for (int off = 32; off > 0; off >>= 1) hh += __shfl_xor(hh, off, 64);
-    const double ww = h2[j + 1] - hh;
+    double ww = h2[j + 1] - hh;
+    // A breakdown: most of what pass 1 left lies in the basis' span, so it is
+    // rounding and the difference has few digits or none.  Every wave sees the
+    // same sums and goes the same way.
+    if (ww < 0.25 * h2[j + 1]) {
+        double sum = 0.0;
+        const int64_t tiles = (len + 63) / 64 * N;
+        for (int64_t q = lane >> 6; q < tiles; q += kStepWaves) {
+            const int r = (int)(q % N);
+            const int64_t p = q / N * 64 + at;
+            if (p >= len) continue;
+            const double* Ve = V + basis_at((size_t)p, r, N, m + 1);
+            double v = 0.0;
+            for (int i = 0; i <= j; ++i) v += h2[i] * Ve[64 * i];
+            v = w[r * len + p] - v;
+            sum += v * v;
+        }
+#pragma unroll
+        for (int off = 32; off > 0; off >>= 1) sum += __shfl_xor(sum, off, 64);
+        if (at == 0) left[lane >> 6] = sum;
+        __syncthreads();
+        ww = 0.0;
+        for (int q = 0; q < kStepWaves; ++q) ww += left[q];
+    }
+    if (!first) return;
     const double nrm = __builtin_sqrt(ww > 0.0 ? ww : 0.0);
     const double h = h1 + c2;
     double mine = 0.0, a = lane_value(h, 0);
@@ -1462,7 +1491,8 @@ hipError_t launch_gm_step(hipStream_t s, const GmDev& G, const ColourOrder* O, i
         e = gs_update<1, kTiles>(s, G, span_of(off, 1), V, (size_t)n, m, w, nblk1, sums2, &nblk);
     }
     if (e != hipSuccess) return e;
-    hipLaunchKernelGGL(k_gm_step, dim3(1), dim3(576), 0, s, G, j, show ? 1 : 0, sums2, nblk);
+    hipLaunchKernelGGL(k_gm_step, dim3(1), dim3(64 * kStepWaves), 0, s, G, j, show ? 1 : 0, sums2, nblk, V, O ? nv : 1,
+                       O ? (int64_t)O->off[O->ncolours] : n, w);
     return hipGetLastError();
 }
 hipError_t launch_next_vector(hipStream_t s, const GmDev& G, const double* w, double* V, int cols, double* v,

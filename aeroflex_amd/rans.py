@@ -92,6 +92,7 @@ def _load():
         "afx_rans_set_preconditioner": (C.c_int, [P, i32]),
         "afx_rans_precond_apply": (C.c_int, [P, P, P]),
         "afx_rans_cell_colours": (C.c_int, [P, P, P]),
+        "afx_rans_arnoldi_step": (C.c_int, [P, i32, i64, dp, dp, dp, dp, P]),
         "afx_rans_implicit_fill": (C.c_int, [P]),
         "afx_rans_implicit_compute": (C.c_int, [P, C.POINTER(i32)]),
         "afx_rans_implicit_solve": (C.c_int, [P, f64, f64, i32, i32, dp]),
@@ -470,6 +471,20 @@ class Solver(Handle):
         n = C.c_int32()
         _check(lib.afx_rans_cell_colours(self.h, col.ctypes.data_as(C.c_void_p), C.byref(n)))
         return col, n.value
+
+    def arnoldi_step(self, basis, w):
+        """(next vector, its length before scaling, flags) at the end of one
+        Arnoldi step of the linear solver on an orthonormal basis (one row per
+        vector) and w, in the order of the process (test hook)."""
+        basis = np.ascontiguousarray(basis, dtype=np.float64)
+        w = np.ascontiguousarray(w, dtype=np.float64)
+        if basis.ndim != 2 or w.shape != basis.shape[1:]:
+            raise RansError("basis and vector differ in length")
+        nxt, norm = np.empty_like(w), C.c_double()
+        flags = np.zeros(4, dtype=np.int32)
+        _check(lib.afx_rans_arnoldi_step(self.h, basis.shape[0], len(w), _dptr(basis), _dptr(w), _dptr(nxt),
+                                         C.byref(norm), flags.ctypes.data_as(C.c_void_p)))
+        return nxt, norm.value, flags
 
     def set_matrix_free(self, enable=True):
         """The RANS_MATRIX_FREE build of implicitSolver (solver.h:863-925):

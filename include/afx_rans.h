@@ -229,6 +229,15 @@ int afx_rans_precond_apply_nu(afx_rans* h, const double* x, const double* x_nu, 
 /* colour of each real cell (reference order, n_real entries, nullable) in the
  * DILU sweeps and the number of colours; for tests */
 int afx_rans_cell_colours(afx_rans* h, int32_t* colours, int32_t* ncolours);
+/* Test hook (no counterpart in the reference): the end of one Arnoldi step of
+ * the linear solver, with the preconditioner of the last fill, on the caller's
+ * m < restart orthonormal basis vectors and vector w, each of n entries: with
+ * DILU the planes of the real cells in the sweeps' order (n = nv n_real),
+ * otherwise nv n_cells.  next: the vector the basis goes on with; norm: its
+ * length before scaling; flags (4): active, converged, steps, columns.  norm
+ * and next are zero where the process has ended. */
+int afx_rans_arnoldi_step(afx_rans* h, int32_t m, int64_t n, const double* basis, const double* w, double* next,
+                          double* norm, int32_t* flags);
 /* The RANS_MATRIX_FREE build of implicitSolver (solver.h:863-868, 911-914,
  * 920-925): enable = 1 replaces the assembled matrix by the matrix-free
  * operator RansMatrix (ransMatrix.h:138-178) and the preconditioned GMRES by

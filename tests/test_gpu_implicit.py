@@ -379,3 +379,44 @@ def test_colour_order_solve_at_the_variants_edges(ni, nj, model):
     bound = tol * np.linalg.norm(R) + 4 * np.finfo(float).eps * 100 * size
     assert np.linalg.norm((left - R)[keep]) <= bound
     assert its > 8
+
+
+# what pass 1 leaves of a vector: nothing lost (0.5), rounding of the basis' span
+# above it by 4, 8 and 9 orders.  Rows split over threads (and one tile), whole
+# rows; both layouts of the basis.
+@pytest.mark.parametrize("left", [0.5, 1e-6, 1e-12, 1e-20, 1e-24, 1e-25])
+@pytest.mark.parametrize("ni,nj,model,kind", [(16, 4, "inviscid", "dilu"), (61, 40, "spalart-allmaras", "dilu"),
+                                              (160, 129, "inviscid", "dilu"), (160, 129, "spalart-allmaras", "dilu"),
+                                              (16, 4, "inviscid", "block-jacobi"),
+                                              (61, 40, "spalart-allmaras", "block-jacobi")])
+def test_basis_goes_on_with_a_unit_vector_at_a_breakdown(ni, nj, model, kind, left):
+    """w = V c + left e with |c| = 1 and V spanning 8 coordinates that e is not
+    among: the step's norm is that of w - V h2 after two passes, left to within
+    the second pass's rounding (eps^2 |c|), and the next vector has length 1."""
+    from aeroflex_amd import rans
+    m = rans.Mesh.jittered(ni, nj, r_far=20.0 if nj > 10 else 3.0, first_h=2e-3 if nj > 10 else 0.3, seed=3,
+                           quad_frac=0.0)
+    sa = model == "spalart-allmaras"
+    s = rans.Solver(m, gas=rans.Gas(mu_L=1e-6 if sa else 1e-5), viscosity_model=model)
+    far = rans.BoundaryVariables(mach=0.5, angle=0.03)
+    s.set_bcs({"farfield": rans.BoundaryCondition("farfield", far),
+               "wall": rans.BoundaryCondition("wall" if sa else "slip-wall")})
+    s.init()
+    s.refill_bcs()
+    s.set_cfl(5.0)
+    s.set_preconditioner(kind)
+    s.fill()
+    rng = np.random.default_rng(ni)
+    n = (5 if sa else 4) * (s.n_real if kind == "dilu" else s.n_cells)
+    at = rng.choice(n, 9, replace=False)
+    Q = np.linalg.qr(rng.standard_normal((8, 8)))[0]
+    V = np.zeros((8, n))
+    V[:, at[:8]] = Q
+    c = rng.standard_normal(8)
+    w = V.T @ (c / np.linalg.norm(c))
+    w[at[8]] = left
+    nxt, norm, flags = s.arnoldi_step(V, w)
+    assert list(flags[:2]) == [1, 0]
+    assert abs(norm - left) <= 1e-12 * left + 64 * np.finfo(float).eps ** 2
+    assert abs(np.linalg.norm(nxt) - 1.0) <= 1e-12
+    assert abs(nxt[at[8]]) > 0.99
