@@ -2149,6 +2149,12 @@ int afx_rans_save_vtu(afx_rans* h, const char* path) {
     return AFX_OK;
 }
 
+// Test hook: see afx_rans.h
+int afx_no_pinned(int32_t on) {
+    t_no_pinned = on != 0;
+    return AFX_OK;
+}
+
 int afx_rans_set_turbulence(afx_rans* h, double nu_ratio) {
     int rc = check_handle(h, false);
     if (rc) return rc;

@@ -177,21 +177,26 @@ StagingPool& pool() {
     return *p;
 }
 }  // namespace
+thread_local bool t_no_pinned = false;
+
 void staging_retain() { pool().retain(); }
 void staging_release() { pool().release(); }
 
 Staging::Staging() {
     int dev = 0;
     if ((err_ = hipGetDevice(&dev)) != hipSuccess) return;
-    if ((b_ = pool().take(dev))) return;
+    if (!t_no_pinned && (b_ = pool().take(dev))) return;
     b_ = new Buf();
     b_->device = dev;
-    err_ = hipHostMalloc((void**)&b_->pin, kSlots * kSlotBytes + kScalars * sizeof(double), hipHostMallocDefault);
+    const size_t bytes = t_no_pinned ? size_t(1) << 60 : kSlots * kSlotBytes + kScalars * sizeof(double);
+    err_ = hipHostMalloc((void**)&b_->pin, bytes, hipHostMallocDefault);
     for (int k = 0; k < kSlots && err_ == hipSuccess; ++k)
         err_ = hipEventCreateWithFlags(&b_->ev[k], hipEventDisableTiming);
     if (err_ != hipSuccess) {
         delete b_;
         b_ = nullptr;
+        // the call goes on without: the error must not reach its launches' checks
+        (void)hipGetLastError();
     }
 }
 Staging::~Staging() {

@@ -43,6 +43,8 @@ private:
 };
 // The pool keeps buffers while any solver handle lives: every handle holds one
 // reference, and the last one to go frees the idle buffers.
+// Test hook, per thread: Staging asks for more pinned memory than there is.
+extern thread_local bool t_no_pinned;
 void staging_retain();
 void staging_release();
 

@@ -80,6 +80,10 @@ typedef struct afx_opts {
 } afx_opts;
 
 const char* afx_last_error(void);
+/* Test hook (no counterpart in the reference): on = 1 lets the calling thread's
+ * requests for pinned staging memory fail, as when the host has none to give;
+ * vectors then cross without it. */
+int afx_no_pinned(int32_t on);
 void afx_default_gas(afx_gas* g);
 void afx_default_opts(afx_opts* o);
 

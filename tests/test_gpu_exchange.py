@@ -65,3 +65,44 @@ def test_threads_do_not_mix_their_vectors():
     for t in team:
         t.join()
     assert not bad
+
+
+# direct and pieced vectors, one and two norms, both operators of the implicit
+# step: without pinned memory the same values cross
+@pytest.mark.parametrize("model,nj", [("inviscid", 16), ("spalart-allmaras", 16), ("spalart-allmaras", 1100)])
+def test_vectors_cross_without_pinned_memory(model, nj):
+    from aeroflex_amd import rans
+    ni = 64
+
+    def values():
+        s = make(ni, nj, True, model)
+        s.init()
+        s.refill_bcs()
+        s.set_cfl(2.0)
+        q = s.get_q().reshape(-1, 4)
+        q[:s.n_real] *= 1.0 + 1e-3 * np.random.default_rng(nj).standard_normal((s.n_real, 4))
+        s.set_q(q.ravel())
+        out = [s.get_q(), s.calc_dt()]
+        for precision in (rans.AFX_FP64, rans.AFX_FP32):
+            out += s.fillRhoRHS(precision)
+        if model != "inviscid":
+            s.set_nu(s.get_nu() * 1.5)
+            out += [s.get_nu(), s.nu_residual()]
+        err = s.explicit_solve(0.5)
+        if nj < 100:
+            for matrix_free in (False,) if model != "inviscid" else (False, True):
+                s.set_matrix_free(matrix_free)
+                s.fill()
+                assert s.compute() == 0
+                assert s.solve(relaxation=0.5, tol=0.0, rhs_iterations=2) >= 0
+                out.append(s.linear_iterations())
+        return out + [err, s.get_q()]
+    want = values()
+    try:
+        assert rans.lib.afx_no_pinned(1) == 0
+        got = values()
+    finally:
+        rans.lib.afx_no_pinned(0)
+    assert len(got) == len(want)
+    for a, b in zip(got, want):
+        assert np.array_equal(a, b)
