@@ -39,11 +39,20 @@ int fail(int code, const std::string& msg) {
     return code;
 }
 
-#define HIPCHK(x)                                                                              \
-    do {                                                                                       \
-        hipError_t e_ = (x);                                                                   \
-        if (e_ != hipSuccess) return fail(AFX_EHIP, std::string(#x) + ": " + hipGetErrorString(e_)); \
+// the runtime keeps an error until it is read, and the launch checks read it: one
+// that is reported must not be left for the next call's first launch
+int hip_fail(const char* what, hipError_t e) {
+    (void)hipGetLastError();
+    return fail(AFX_EHIP, std::string(what) + ": " + hipGetErrorString(e));
+}
+
+#define HIPCHK(x)                                            \
+    do {                                                     \
+        hipError_t e_ = (x);                                 \
+        if (e_ != hipSuccess) return hip_fail(#x, e_);       \
     } while (0)
+
+thread_local int t_fail_alloc = 0;   // test hook: the n-th allocation from now fails (afx_fail_alloc)
 
 template <typename T>
 struct DBuf {
@@ -55,7 +64,8 @@ struct DBuf {
     ~DBuf() { if (p) (void)hipFree(p); }
     hipError_t alloc(size_t count) {
         n = count;
-        return hipMalloc(&p, std::max<size_t>(count, 1) * sizeof(T));
+        const bool too_much = t_fail_alloc > 0 && --t_fail_alloc == 0;
+        return hipMalloc(&p, too_much ? size_t(1) << 60 : std::max<size_t>(count, 1) * sizeof(T));
     }
     hipError_t upload(const T* h, size_t count, hipStream_t s) {
         return hipMemcpyAsync(p, h, count * sizeof(T), hipMemcpyHostToDevice, s);
@@ -1065,7 +1075,7 @@ int create_impl(const Mesh& mesh_in, const afx_gas* g, const afx_opts* o, const 
 #define HIPCHK_C(x)                                                                                   \
     do {                                                                                              \
         hipError_t e_ = (x);                                                                          \
-        if (e_ != hipSuccess) return bail(fail(AFX_EHIP, std::string(#x) + ": " + hipGetErrorString(e_))); \
+        if (e_ != hipSuccess) return bail(hip_fail(#x, e_));                                              \
     } while (0)
 
     HIPCHK_C(hipStreamCreateWithFlags(&h->stream, hipStreamNonBlocking));
@@ -2149,7 +2159,11 @@ int afx_rans_save_vtu(afx_rans* h, const char* path) {
     return AFX_OK;
 }
 
-// Test hook: see afx_rans.h
+// Test hooks: see afx_rans.h
+int afx_fail_alloc(int32_t nth) {
+    t_fail_alloc = nth > 0 ? nth : 0;
+    return AFX_OK;
+}
 int afx_no_pinned(int32_t on) {
     t_no_pinned = on != 0;
     return AFX_OK;
@@ -2881,7 +2895,7 @@ int afx_batch_create(int32_t n, afx_rans* const* members, double relaxation, afx
         if (!rc && !h->q32v_b.p) {   // the two further FP32 stage buffers
             if (h->q32v_b.alloc(h->nT) != hipSuccess || h->q32v_c.alloc(h->nT) != hipSuccess ||
                 (h->sa() && (h->q32n_b.alloc(h->nT) != hipSuccess || h->q32n_c.alloc(h->nT) != hipSuccess)))
-                rc = fail(AFX_EHIP, "hipMalloc of the batch stage buffers failed");
+                rc = hip_fail("batch stage buffers", hipErrorOutOfMemory);
         }
         if (rc) { delete b; return rc; }
         b->mem.push_back(h);
@@ -3009,7 +3023,7 @@ int afx_mapper_create(const afx_rans* coarse, const afx_rans* fine, afx_mapper**
 #define HIPCHK_M(x)                                                                                   \
     do {                                                                                              \
         hipError_t e_ = (x);                                                                          \
-        if (e_ != hipSuccess) return bail(fail(AFX_EHIP, std::string(#x) + ": " + hipGetErrorString(e_))); \
+        if (e_ != hipSuccess) return bail(hip_fail(#x, e_));                                              \
     } while (0)
     mp->coarse = coarse;
     mp->fine = fine;

@@ -31,10 +31,15 @@ using afx::api_fail;
 
 namespace {
 
-#define VCHK(x)                                                                                     \
-    do {                                                                                            \
-        hipError_t e_ = (x);                                                                        \
-        if (e_ != hipSuccess) return api_fail(AFX_EHIP, std::string(#x) + ": " + hipGetErrorString(e_)); \
+// (the error is read, or the next call's launch check would report it again)
+int hip_fail(const char* what, hipError_t e) {
+    (void)hipGetLastError();
+    return api_fail(AFX_EHIP, std::string(what) + ": " + hipGetErrorString(e));
+}
+#define VCHK(x)                                              \
+    do {                                                     \
+        hipError_t e_ = (x);                                 \
+        if (e_ != hipSuccess) return hip_fail(#x, e_);       \
     } while (0)
 
 constexpr int LU_NB = 128;          // panel width = trailing-update depth = solve block
@@ -1527,7 +1532,7 @@ int afx_vlm_create(int32_t n_nodes, const double* xyz, int32_t n_stations, const
 #define VCHK_C(x)                                                                                    \
     do {                                                                                             \
         hipError_t e_ = (x);                                                                         \
-        if (e_ != hipSuccess) return bail(api_fail(AFX_EHIP, std::string(#x) + ": " + hipGetErrorString(e_))); \
+        if (e_ != hipSuccess) return bail(hip_fail(#x, e_));                                         \
     } while (0)
     VCHK_C(dalloc(&h->d_nodes, 3 * (size_t)n_nodes));
     VCHK_C(dalloc(&h->d_corner, 12 * (size_t)nr));

@@ -70,6 +70,7 @@ def _load():
         "afx_mesh_boundary_name": (C.c_int, [P, i64, C.c_char_p, i32]),
         "afx_mesh_rcm": (C.c_int, [P, P]),
         "afx_no_pinned": (C.c_int, [i32]),
+        "afx_fail_alloc": (C.c_int, [i32]),
         "afx_mesh_tile_stats": (C.c_int, [P, i32, C.POINTER(i64)]),
         "afx_mesh_destroy": (None, [P]),
         "afx_rans_create": (C.c_int, [P, C.POINTER(AfxGas), C.POINTER(AfxOpts), C.POINTER(P)]),

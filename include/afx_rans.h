@@ -84,6 +84,10 @@ const char* afx_last_error(void);
  * requests for pinned staging memory fail, as when the host has none to give;
  * vectors then cross without it. */
 int afx_no_pinned(int32_t on);
+/* Test hook (no counterpart in the reference): the nth device allocation that a
+ * solver makes from now on, on the calling thread, asks for more memory than
+ * there is and fails (0: none). */
+int afx_fail_alloc(int32_t nth);
 void afx_default_gas(afx_gas* g);
 void afx_default_opts(afx_opts* o);
 

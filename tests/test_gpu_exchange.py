@@ -106,3 +106,17 @@ def test_vectors_cross_without_pinned_memory(model, nj):
     assert len(got) == len(want)
     for a, b in zip(got, want):
         assert np.array_equal(a, b)
+
+
+def test_a_failed_allocation_is_reported_once():
+    """The state's first large transfer allocates its device rows; where that
+    fails, the next call goes through."""
+    from aeroflex_amd import rans
+    s, t = make(64, 1100, True), make(64, 1100, True)
+    s.init()
+    t.init()
+    rans.lib.afx_fail_alloc(1)
+    with pytest.raises(rans.RansError, match="out of memory"):
+        s.get_q()
+    rans.lib.afx_fail_alloc(0)
+    assert np.array_equal(s.get_q(), t.get_q())
