@@ -62,10 +62,18 @@ struct DBuf {
     DBuf(const DBuf&) = delete;
     DBuf& operator=(const DBuf&) = delete;
     ~DBuf() { if (p) (void)hipFree(p); }
+    // an array of count; one of that size is kept, another freed first; empty on
+    // failure, so that a set-up that failed halfway can be run again
     hipError_t alloc(size_t count) {
-        n = count;
+        if (p && n == count) return hipSuccess;
+        if (p) (void)hipFree(p);
+        p = nullptr;
+        n = 0;
         const bool too_much = t_fail_alloc > 0 && --t_fail_alloc == 0;
-        return hipMalloc(&p, too_much ? size_t(1) << 60 : std::max<size_t>(count, 1) * sizeof(T));
+        const hipError_t e = hipMalloc(&p, too_much ? size_t(1) << 60 : std::max<size_t>(count, 1) * sizeof(T));
+        if (e == hipSuccess) n = count;
+        else p = nullptr;
+        return e;
     }
     hipError_t upload(const T* h, size_t count, hipStream_t s) {
         return hipMemcpyAsync(p, h, count * sizeof(T), hipMemcpyHostToDevice, s);
@@ -198,6 +206,9 @@ struct afx_rans {
         return G;
     }
     static size_t gm_doubles(int m) { return 8 + (size_t)(m + 1) * m + 2 * (size_t)m + (m + 1) + m + 2 * (size_t)(m + 1); }
+    // set-ups of the implicit step, the adjoints, those with respect to the mesh
+    // nodes and the tangent: every array allocated and filled
+    bool implicit_ready = false, adjoint_ready = false, geo_ready = false, tangent_ready = false;
     bool lhs_ready = false;
     int lhs_bad = 0;
     bool mf = false;             // matrix-free operator (RANS_MATRIX_FREE build)
@@ -295,11 +306,7 @@ std::vector<T> to_device_order_faces(const afx_rans* h, const std::vector<double
 }
 
 int ensure_rows(afx_rans* h, int nv) {
-    if (h->xrows.n >= (size_t)nv * h->nT) return AFX_OK;
-    if (h->xrows.p) { (void)hipFree(h->xrows.p); h->xrows.p = nullptr; h->xrows.n = 0; }
-    const hipError_t e = h->xrows.alloc((size_t)nv * h->nT);
-    if (e != hipSuccess) { h->xrows.p = nullptr; h->xrows.n = 0; }
-    HIPCHK(e);
+    if (h->xrows.n < (size_t)nv * h->nT) HIPCHK(h->xrows.alloc((size_t)nv * h->nT));
     return AFX_OK;
 }
 // device cells (planes of double or float, or one float4 per cell) -> nv values
@@ -447,7 +454,7 @@ int compute_wall_distance(afx_rans* h) {
     HIPCHK(launch_wall_dist(h->stream, h->xc.p, h->yc.p, h->nT, dwx.p, dwy.p, (int32_t)wx.size(), h->wall_d.p));
     DBuf<double4> dseg;
     if (h->sa()) {
-        if (!h->sa_wd.p) HIPCHK(h->sa_wd.alloc(h->nT));
+        HIPCHK(h->sa_wd.alloc(h->nT));
         HIPCHK(dseg.alloc(seg.size())); HIPCHK(dseg.upload(seg, h->stream));
         HIPCHK(launch_wall_dist_seg(h->stream, h->xc.p, h->yc.p, h->nT, dseg.p, (int32_t)seg.size(), h->sa_wd.p));
     }
@@ -638,14 +645,14 @@ std::vector<uint8_t> colour_cells(const std::vector<int32_t>& nbr, int32_t nC, i
 }
 
 int ensure_implicit(afx_rans* h) {
-    if (h->mf && !h->mfFb.p) HIPCHK(h->mfFb.alloc((size_t)4 * h->nF));
-    if (!h->mf && h->precond == 0 && !h->ellE.p) {   // the product in cell order
+    if (h->mf) HIPCHK(h->mfFb.alloc((size_t)4 * h->nF));
+    if (!h->mf && h->precond == 0) {   // the product in cell order
         const size_t nn = (size_t)h->nv * h->nv;
         HIPCHK(h->ellD.alloc(nn * h->nC));
         HIPCHK(h->ellN.alloc(4 * (size_t)h->nC));
         HIPCHK(h->ellE.alloc(4 * nn * h->nC));
     }
-    if (!h->mf && h->precond == 1 && !h->dilE.p) {   // sweeps and product in colour order
+    if (!h->mf && h->precond == 1) {   // sweeps and product in colour order
         const size_t nn = (size_t)h->nv * h->nv;
         HIPCHK(h->Dti.alloc(nn * h->nC));
         HIPCHK(h->dilD.alloc(nn * h->nC));
@@ -653,7 +660,7 @@ int ensure_implicit(afx_rans* h) {
         HIPCHK(h->dilN.alloc(4 * (size_t)h->nC));
         HIPCHK(h->dilE.alloc(4 * nn * h->nC));
     }
-    if (h->Jf.p) return AFX_OK;
+    if (h->implicit_ready) return AFX_OK;
     // blocks of nv x nv (five with the Spalart-Allmaras model), vectors of nv planes
     const int nv = h->nv;
     const size_t nn = (size_t)nv * nv;
@@ -709,6 +716,7 @@ int ensure_implicit(afx_rans* h) {
         HIPCHK(h->col_pos.upload(where, h->stream));
         HIPCHK(hipStreamSynchronize(h->stream));
     }
+    h->implicit_ready = true;
     return AFX_OK;
 }
 
@@ -1672,7 +1680,7 @@ int explicit_step_tiles(afx_rans* h, const double* qin, double* qout, double rel
     static const double alpha[3] = {0.25, 0.5, 1.};
     hipStream_t s = h->stream;
     const int64_t nq = (int64_t)h->nv * h->nT;
-    if (!h->qk2.p) HIPCHK(h->qk2.alloc((size_t)NV_MAX * h->nT));
+    HIPCHK(h->qk2.alloc((size_t)NV_MAX * h->nT));
     double* a = keep ? keep[3] : h->qk2.p;
     double* b = keep ? keep[4] : h->qk.p;
     // the last stage writes beside its input and, when viscous fluxes read qin
@@ -1754,7 +1762,7 @@ int afx_rans_set_linear_solver(afx_rans* h, int32_t restart, double tol, int32_t
     if (rc) return rc;
     if (restart < 1 || restart > 32 || !(tol > 0) || maxit < 1)
         return fail(AFX_EARG, "bad linear solver settings (restart 1..32, tol > 0, maxit >= 1)");
-    if (h->Jf.p && restart != h->gm_restart) return fail(AFX_ESTATE, "restart length is fixed after the first fill");
+    if (h->implicit_ready && restart != h->gm_restart) return fail(AFX_ESTATE, "restart length is fixed after the first fill");
     h->gm_restart = restart;
     h->gm_tol = tol;
     h->gm_maxit = maxit;
@@ -1978,7 +1986,7 @@ int afx_rans_arnoldi_step(afx_rans* h, int32_t m, int64_t n, const double* basis
 int afx_rans_cell_colours(afx_rans* h, int32_t* colours, int32_t* ncolours) {
     int rc = check_handle(h, false);
     if (rc) return rc;
-    if (!h->colour.p) return fail(AFX_ESTATE, "no colouring before the first afx_rans_implicit_fill");
+    if (!h->implicit_ready) return fail(AFX_ESTATE, "no colouring before the first afx_rans_implicit_fill");
     std::vector<uint8_t> col(h->nC);
     HIPCHK(hipMemcpyAsync(col.data(), h->colour.p, col.size(), hipMemcpyDeviceToHost, h->stream));
     HIPCHK(hipStreamSynchronize(h->stream));
@@ -2047,10 +2055,8 @@ static int gather_patch(afx_rans* h, const char* patch, std::vector<int32_t>& bs
         }
     if (bsel.empty()) return fail(AFX_EARG, std::string("no boundary faces on patch '") + patch + "'");
     if (h->patch_cells.n < cells.size()) {
-        if (h->patch_cells.p) { (void)hipFree(h->patch_cells.p); h->patch_cells.p = nullptr; }
-        if (h->states.p) { (void)hipFree(h->states.p); h->states.p = nullptr; }
-        HIPCHK(h->patch_cells.alloc(cells.size()));
         HIPCHK(h->states.alloc(cells.size() * NV));
+        HIPCHK(h->patch_cells.alloc(cells.size()));
     }
     HIPCHK(h->patch_cells.upload(cells, h->stream));
     HIPCHK(launch_gather_states(h->stream, h->q.p, h->nT, NV, h->patch_cells.p, (int32_t)cells.size(), h->states.p));
@@ -2265,7 +2271,7 @@ int adjoint_check(afx_rans* h, bool state_adjoint = false) {
         int rc = compute_wall_distance(h);
         if (rc) return rc;
     }
-    if (!h->a_w.p) {
+    if (!h->adjoint_ready) {
         // planes: one per variable (five with the Spalart-Allmaras model)
         const size_t c4 = (size_t)h->nv * h->nC, t4 = (size_t)h->nv * h->nT, f4 = (size_t)h->nv * h->nF;
         for (DBuf<double>* b : {&h->a_w, &h->a_lam, &h->a_lgx, &h->a_lgy}) HIPCHK(b->alloc(t4));
@@ -2280,8 +2286,9 @@ int adjoint_check(afx_rans* h, bool state_adjoint = false) {
         std::sort(bf.begin(), bf.end());
         if (!bf.empty()) { HIPCHK(h->a_bface.alloc(bf.size())); HIPCHK(h->a_bface.upload(bf, h->stream)); }
         HIPCHK(hipStreamSynchronize(h->stream));
+        h->adjoint_ready = true;
     }
-    if (h->opts.viscosity != 0 && !h->a_vgx.p) {
+    if (h->opts.viscosity != 0) {
         const size_t f4 = (size_t)h->nv * h->nF;
         for (DBuf<double>* b : {&h->a_vgx, &h->a_vgy, &h->a_vdq}) HIPCHK(b->alloc(f4));
     }
@@ -2295,7 +2302,7 @@ AdjBufs adj_bufs(const afx_rans* h) {
                    lam ? h->a_vgy.p : nullptr, lam ? h->a_vdq.p : nullptr};
 }
 int geo_check(afx_rans* h) {
-    if (h->g_fbar.p) return AFX_OK;
+    if (h->geo_ready) return AFX_OK;
     const Mesh& m = h->m;
     const int32_t nC = h->nC, nF = h->nF;
     const int32_t nN = (int32_t)m.nodesX.size();
@@ -2341,6 +2348,7 @@ int geo_check(afx_rans* h) {
     HIPCHK(h->g_noff.alloc(off.size())); HIPCHK(h->g_noff.upload(off, h->stream));
     HIPCHK(h->g_nent.alloc(ent.size())); HIPCHK(h->g_nent.upload(ent, h->stream));
     HIPCHK(hipStreamSynchronize(h->stream));
+    h->geo_ready = true;
     return AFX_OK;
 }
 int enqueue_adjoint(afx_rans* h) {
@@ -2678,7 +2686,7 @@ int tangent_prepare(afx_rans* h) {
     if (h->sa() && !h->wd_ready && (rc = compute_wall_distance(h))) return rc;
     hipStream_t s = h->stream;
     const int64_t nT = h->nT;
-    if (!h->tg_q.p) {
+    if (!h->tangent_ready) {
         HIPCHK(h->tg_geo.alloc(h->t_geo64.n));
         HIPCHK(h->tg_area.alloc(h->area.n));
         HIPCHK(h->tg_lsq.alloc(h->lsq.n));
@@ -2697,6 +2705,7 @@ int tangent_prepare(afx_rans* h) {
         HIPCHK(hipMemsetAsync(h->tg_v.p, 0, (size_t)nv * nT * 8, s));
         // the tile kernel writes the real rows only: ghost rows of J v stay 0
         HIPCHK(hipMemsetAsync(h->tg_R.p, 0, (size_t)nv * nT * sizeof(Dual1), s));
+        h->tangent_ready = true;
     }
     if (h->sa())   // follows the BCs
         HIPCHK(launch_to_dual(s, h->sa_wd.p, (int64_t)h->sa_wd.n, h->tg_wd.p));
@@ -2892,7 +2901,7 @@ int afx_batch_create(int32_t n, afx_rans* const* members, double relaxation, afx
             rc = fail(AFX_EARG, "batch members must share the viscosity model, gradient scheme and order "
                                 "(one kernel instantiation per launch)");
         if (!rc && h->sa() && !h->wd_ready) rc = compute_wall_distance(h);
-        if (!rc && !h->q32v_b.p) {   // the two further FP32 stage buffers
+        if (!rc) {   // the two further FP32 stage buffers
             if (h->q32v_b.alloc(h->nT) != hipSuccess || h->q32v_c.alloc(h->nT) != hipSuccess ||
                 (h->sa() && (h->q32n_b.alloc(h->nT) != hipSuccess || h->q32n_c.alloc(h->nT) != hipSuccess)))
                 rc = hip_fail("batch stage buffers", hipErrorOutOfMemory);

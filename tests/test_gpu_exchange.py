@@ -1,6 +1,7 @@
 """Vectors crossing the C ABI (afx_exchange.hip): the device permutation, the
 direct and the pieced transfer on both sides of their limits, and calls from
 several threads at once."""
+import ctypes as C
 import threading
 
 import numpy as np
@@ -120,3 +121,76 @@ def test_a_failed_allocation_is_reported_once():
         s.get_q()
     rans.lib.afx_fail_alloc(0)
     assert np.array_equal(s.get_q(), t.get_q())
+
+
+def _free_bytes():
+    """Free device memory, from the runtime that the library is linked with."""
+    from aeroflex_amd import rans
+    free, total = C.c_size_t(), C.c_size_t()
+    assert C.CDLL(rans.LIB_PATH).hipMemGetInfo(C.byref(free), C.byref(total)) == 0
+    return free.value
+
+
+def _implicit(s, kind):
+    s.set_preconditioner(kind)
+    s.set_cfl(2.0)
+    s.fill()
+    s.compute()
+    s.solve(relaxation=0.5, tol=0.0, rhs_iterations=1)
+    return s.get_q()
+
+
+def _batch(s):
+    from aeroflex_amd import rans
+    s.set_cfl(0.1)
+    b = rans.Batch([s])
+    b.run(2, 0)
+    b.close()
+    return s.get_q()
+
+
+# every set-up that a first call makes: each of its allocations fails once, and
+# the call after that goes through with the same result.  Once the solver is closed
+# nothing of them is left, to a few of the runtime's chunks of 2 MB; an array of the
+# set-ups kept by mistake is 4 MB and more.
+@pytest.mark.parametrize("model,call", [
+    ("inviscid", lambda s: _implicit(s, "dilu")), ("inviscid", lambda s: _implicit(s, "block-jacobi")),
+    ("spalart-allmaras", lambda s: _implicit(s, "dilu")), ("inviscid", lambda s: s.explicit_solve(0.5)),
+    ("laminar", lambda s: s.adjoint(np.ones(4 * s.n_cells))), ("inviscid", lambda s: s.tangent(np.ones(4 * s.n_cells))),
+    ("inviscid", lambda s: s.adjoint_nodes(np.ones(4 * s.n_cells))[1]), ("inviscid", lambda s: s.get_wall_profile("wall")),
+    ("spalart-allmaras", _batch)])
+def test_a_set_up_that_failed_halfway_is_run_again(model, call):
+    from aeroflex_amd import rans
+
+    def prepared():
+        s = make(64, 270, True, model)
+        s.init()
+        s.refill_bcs()
+        q = s.get_q().reshape(-1, 4)
+        q[:s.n_real] *= 1.0 + 1e-3 * np.random.default_rng(7).standard_normal((s.n_real, 4))
+        s.set_q(q.ravel())
+        return s, q.ravel()
+    # (five at once: every hardware queue gets its scratch memory, which the runtime keeps)
+    warm = [prepared() for _ in range(5)]
+    want = [call(w) for w, _ in warm][0]
+    before = _free_bytes()
+    s, q = prepared()
+    failed = 0
+    for again in range(80):
+        print("attempt", again, flush=True)
+        # a solver keeps what the last attempt got, so the second allocation is a
+        # new one; a batch that could not be made starts again
+        rans.lib.afx_fail_alloc(again + 1 if call is _batch else min(again, 1) + 1)
+        try:
+            s.set_q(q)
+            got = call(s)
+            break
+        except rans.RansError as e:
+            assert "out of memory" in str(e)
+            failed += 1
+        finally:
+            rans.lib.afx_fail_alloc(0)
+    assert failed > 0
+    assert np.array_equal(np.asarray(got), np.asarray(want))
+    s.close()
+    assert before - _free_bytes() <= 3 << 21
