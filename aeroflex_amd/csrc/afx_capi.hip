@@ -313,12 +313,12 @@ int ensure_rows(afx_rans* h, int nv) {
 // per reference cell in the caller's memory (nv 4: q(4*i+k)); waits.  The call's staging
 // buffer st may carry scalars that earlier kernels of the call wrote.
 template <typename T>
-int fetch_rows(afx_rans* h, const Staging& st, const T* d, int nv, double* out) {
+int fetch_rows(afx_rans* h, Staging& st, const T* d, int nv, double* out) {
     const size_t bytes = (size_t)nv * h->nT * sizeof(double);
     const bool pinned = st.status() == hipSuccess;
     if (pinned && bytes <= kDirectBytes) {
         HIPCHK(launch_export_rows(h->stream, d, h->o2n.p, h->nT, nv, reinterpret_cast<double*>(st.piece(0))));
-        HIPCHK(hipStreamSynchronize(h->stream));
+        HIPCHK(st.wait());
         std::memcpy(out, st.piece(0), bytes);
         return AFX_OK;
     }
@@ -326,7 +326,7 @@ int fetch_rows(afx_rans* h, const Staging& st, const T* d, int nv, double* out) 
     if (rc) return rc;
     HIPCHK(launch_export_rows(h->stream, d, h->o2n.p, h->nT, nv, h->xrows.p));
     if (pinned) {
-        HIPCHK(st.to_host(h->stream, h->xrows.p, out, bytes));
+        HIPCHK(st.to_host(h->xrows.p, out, bytes));
     } else {   // no pinned memory to be had
         HIPCHK(hipMemcpyAsync(out, h->xrows.p, bytes, hipMemcpyDeviceToHost, h->stream));
         HIPCHK(hipStreamSynchronize(h->stream));
@@ -334,19 +334,19 @@ int fetch_rows(afx_rans* h, const Staging& st, const T* d, int nv, double* out) 
     return AFX_OK;
 }
 // the other way: nv values per reference cell -> planes; waits
-int send_rows(afx_rans* h, const Staging& st, const double* in, int nv, double* d) {
+int send_rows(afx_rans* h, Staging& st, const double* in, int nv, double* d) {
     const size_t bytes = (size_t)nv * h->nT * sizeof(double);
     const bool pinned = st.status() == hipSuccess;
     if (pinned && bytes <= kDirectBytes) {
         std::memcpy(st.piece(0), in, bytes);
         HIPCHK(launch_import_rows(h->stream, reinterpret_cast<const double*>(st.piece(0)), h->o2n.p, h->nT, nv, d));
-        HIPCHK(hipStreamSynchronize(h->stream));
+        HIPCHK(st.wait());
         return AFX_OK;
     }
     int rc = ensure_rows(h, nv);
     if (rc) return rc;
     if (pinned)
-        HIPCHK(st.to_device(h->stream, in, h->xrows.p, bytes));
+        HIPCHK(st.to_device(in, h->xrows.p, bytes));
     else
         HIPCHK(hipMemcpyAsync(h->xrows.p, in, bytes, hipMemcpyHostToDevice, h->stream));
     HIPCHK(launch_import_rows(h->stream, h->xrows.p, h->o2n.p, h->nT, nv, d));
@@ -354,12 +354,22 @@ int send_rows(afx_rans* h, const Staging& st, const double* in, int nv, double* 
     return AFX_OK;
 }
 
+template <typename T>
+int fetch_rows(afx_rans* h, const T* d, int nv, double* out) {
+    Staging st(h->stream);
+    return fetch_rows(h, st, d, nv, out);
+}
+int send_rows(afx_rans* h, const double* in, int nv, double* d) {
+    Staging st(h->stream);
+    return send_rows(h, st, in, nv, d);
+}
+
 // device SoA [NV][nT] -> reference AoS q(4*i+k)
-int download_aos(afx_rans* h, const double* d, double* out) { return fetch_rows(h, Staging(), d, NV, out); }
-int download_aos32(afx_rans* h, const float* d, double* out) { return fetch_rows(h, Staging(), d, NV, out); }
-int download_cells(afx_rans* h, const double* d, double* out) { return fetch_rows(h, Staging(), d, 1, out); }
-int upload_aos(afx_rans* h, const double* in, double* d) { return send_rows(h, Staging(), in, NV, d); }
-int upload_cells(afx_rans* h, const double* in, double* d) { return send_rows(h, Staging(), in, 1, d); }
+int download_aos(afx_rans* h, const double* d, double* out) { return fetch_rows(h, d, NV, out); }
+int download_aos32(afx_rans* h, const float* d, double* out) { return fetch_rows(h, d, NV, out); }
+int download_cells(afx_rans* h, const double* d, double* out) { return fetch_rows(h, d, 1, out); }
+int upload_aos(afx_rans* h, const double* in, double* d) { return send_rows(h, in, NV, d); }
+int upload_cells(afx_rans* h, const double* in, double* d) { return send_rows(h, in, 1, d); }
 // the rho nu~ plane from the caller's vector, zero without one
 int upload_nu(afx_rans* h, const double* in, double* d) {
     if (in) return upload_cells(h, in, d);
@@ -394,10 +404,10 @@ int read_scalars(afx_rans* h, const Staging& st, int n, double* v) {   // after 
     return AFX_OK;
 }
 int norm_of(afx_rans* h, const double* x, int64_t ld, int nrows, double* out) {
-    Staging st;
+    Staging st(h->stream);
     int rc = enqueue_sumsq(h, x, ld, nrows, scalar_slot(h, st));
     if (rc) return rc;
-    HIPCHK(hipStreamSynchronize(h->stream));
+    HIPCHK(st.wait());
     double s = 0;
     if ((rc = read_scalars(h, st, 1, &s))) return rc;
     *out = std::sqrt(s);
@@ -743,7 +753,7 @@ int gmres(afx_rans* h, const double* b, double* dq, double relax, bool* converge
     const int m = h->gm_restart;
     hipStream_t s = h->stream;
     double* V = h->kV.p;
-    Staging st;
+    Staging st(h->stream);
     const bool pinned = st.status() == hipSuccess;
     volatile int* seen = pinned ? reinterpret_cast<volatile int*>(st.scalars()) : nullptr;
     const GmDev G = h->gm_dev(const_cast<int*>(seen));
@@ -778,7 +788,7 @@ int gmres(afx_rans* h, const double* b, double* dq, double relax, bool* converge
     int flags[4] = {0, 0, 0, 0};
     auto read_flags = [&]() -> int {
         if (!pinned) HIPCHK(hipMemcpyAsync(flags, G.flags, sizeof(flags), hipMemcpyDeviceToHost, s));
-        HIPCHK(hipStreamSynchronize(s));
+        HIPCHK(st.wait());
         if (pinned)
             for (int k = 0; k < 4; ++k) flags[k] = seen[k];
         return AFX_OK;
@@ -792,12 +802,14 @@ int gmres(afx_rans* h, const double* b, double* dq, double relax, bool* converge
     HIPCHK(launch_gm_begin(s, G, h->kr.p, n, 1));
     int rc, total_before = 0;
     for (int cycle = 0;; ++cycle) {
+        st.queueing();   // the steps leave their flags in the buffer
         int chunk = std::max(1, std::min<int>(h->gm_chunk, m));
         bool over = false;   // the flags of the finished cycle are known
         for (int j = 0; j < m; ++j) {
             if (j == chunk) {   // a chunk is enqueued: is the Arnoldi process still active?
                 if ((rc = read_flags())) return rc;
                 if ((over = !flags[0])) break;
+                st.queueing();
                 chunk += 4;
             }
             HIPCHK(advance(j == 0 ? h->kr.p : h->kw.p, j, j + 1 == chunk || j + 1 == m));
@@ -1532,7 +1544,7 @@ int afx_rans_residual(afx_rans* h, int32_t precision, double* R, double* norm2) 
     if ((rc = enqueue_residual(h, precision))) return rc;
     if (!R && !norm2) return AFX_OK;
     // norm, then R, and one wait for both
-    Staging st;
+    Staging st(h->stream);
     double* sums = scalar_slot(h, st);
     int parts = 1;
     if (norm2) {
@@ -1555,7 +1567,7 @@ int afx_rans_residual(afx_rans* h, int32_t precision, double* R, double* norm2) 
         else rc = fetch_rows(h, st, h->R32.p, NV, R);
         if (rc) return rc;
     } else {
-        HIPCHK(hipStreamSynchronize(h->stream));
+        HIPCHK(st.wait());
     }
     if (norm2) {
         double v[2] = {0, 0};
@@ -2208,7 +2220,7 @@ int afx_rans_nu_residual(afx_rans* h, double* Rnu) {
     if (!Rnu) return fail(AFX_EARG, "null residual vector");
     if (h->last_precision == AFX_FP64) return download_cells(h, h->R.p + (size_t)4 * h->nT, Rnu);
     if (h->last_precision != AFX_FP32) return fail(AFX_ESTATE, "no residual has been evaluated");
-    return fetch_rows(h, Staging(), h->R32n.p, 1, Rnu);
+    return fetch_rows(h, h->R32n.p, 1, Rnu);
 }
 
 int afx_rans_counts(afx_rans* h, int64_t c[5]) {

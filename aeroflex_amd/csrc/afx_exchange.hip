@@ -182,7 +182,7 @@ thread_local bool t_no_pinned = false;
 void staging_retain() { pool().retain(); }
 void staging_release() { pool().release(); }
 
-Staging::Staging() {
+Staging::Staging(hipStream_t s) : s_(s) {
     int dev = 0;
     if ((err_ = hipGetDevice(&dev)) != hipSuccess) return;
     if (!t_no_pinned && (b_ = pool().take(dev))) return;
@@ -200,7 +200,14 @@ Staging::Staging() {
     }
 }
 Staging::~Staging() {
-    if (b_) pool().give(b_);
+    if (!b_) return;
+    if (waited_ || hipStreamSynchronize(s_) == hipSuccess) pool().give(b_);
+    else delete b_;
+}
+hipError_t Staging::wait() {
+    const hipError_t e = hipStreamSynchronize(s_);
+    waited_ = e == hipSuccess;
+    return e;
 }
 char* Staging::piece(int k) const { return b_->pin + (size_t)k * kSlotBytes; }
 double* Staging::scalars() const { return reinterpret_cast<double*>(b_->pin + kSlots * kSlotBytes); }
@@ -213,7 +220,8 @@ double* Staging::scalars() const { return reinterpret_cast<double*>(b_->pin + kS
 // freshly allocated memory (page faults) and 28 GB/s into touched memory, the
 // PCIe copy of a pinned buffer 56 GB/s; pageable hipMemcpyAsync 4-10 GB/s down
 // into fresh memory and 30 GB/s up.
-hipError_t Staging::pieces(hipStream_t s, char* host, char* dev, size_t bytes, bool up) const {
+hipError_t Staging::pieces(char* host, char* dev, size_t bytes, bool up) {
+    const hipStream_t s = s_;
     const int n = (int)((bytes + kSlotBytes - 1) / kSlotBytes);
     // two slots per worker; one worker up to 4 MB (starting threads costs more)
     const int workers = n <= 4 ? 1 : 4, per = kSlots / workers;
@@ -263,15 +271,15 @@ hipError_t Staging::pieces(hipStream_t s, char* host, char* dev, size_t bytes, b
     for (int w = started; w < workers; ++w) work(w);
     for (std::thread& t : team) t.join();
     // the caller reuses the slots (and its own memory) after this
-    const hipError_t last = hipStreamSynchronize(s);
+    const hipError_t last = wait();
     const hipError_t e = (hipError_t)failed.load();
     return e != hipSuccess ? e : last;
 }
-hipError_t Staging::to_device(hipStream_t s, const void* host, void* dev, size_t bytes) const {
-    return pieces(s, static_cast<char*>(const_cast<void*>(host)), static_cast<char*>(dev), bytes, true);
+hipError_t Staging::to_device(const void* host, void* dev, size_t bytes) {
+    return pieces(static_cast<char*>(const_cast<void*>(host)), static_cast<char*>(dev), bytes, true);
 }
-hipError_t Staging::to_host(hipStream_t s, const void* dev, void* host, size_t bytes) const {
-    return pieces(s, static_cast<char*>(host), static_cast<char*>(const_cast<void*>(dev)), bytes, false);
+hipError_t Staging::to_host(const void* dev, void* host, size_t bytes) {
+    return pieces(static_cast<char*>(host), static_cast<char*>(const_cast<void*>(dev)), bytes, false);
 }
 
 }  // namespace afx

@@ -20,25 +20,33 @@ constexpr int kScalars = 64;                      // doubles for norms and flags
 
 // One pinned staging buffer with its events, on the device that was current
 // when it was taken.  Taken from a process-wide pool and given back by the
-// destructor; a Staging belongs to one call of one thread.
+// destructor, which waits for the stream first where the call has queued work
+// and not waited for it (an error return); a Staging belongs to one call of one
+// thread and one stream.
 class Staging {
 public:
-    Staging();
+    explicit Staging(hipStream_t s);
     ~Staging();
     Staging(const Staging&) = delete;
     Staging& operator=(const Staging&) = delete;
     hipError_t status() const { return err_; }
+    // waits for the stream; from then on nothing queued reads or writes the buffer
+    hipError_t wait();
+    // more work on the buffer is about to be queued after a wait
+    void queueing() { waited_ = false; }
     char* piece(int k) const;            // host = device address (unified addressing)
     double* scalars() const;
     // caller memory <-> device memory, in pieces; returns once done
-    hipError_t to_device(hipStream_t s, const void* host, void* dev, size_t bytes) const;
-    hipError_t to_host(hipStream_t s, const void* dev, void* host, size_t bytes) const;
+    hipError_t to_device(const void* host, void* dev, size_t bytes);
+    hipError_t to_host(const void* dev, void* host, size_t bytes);
 
 private:
-    hipError_t pieces(hipStream_t s, char* host, char* dev, size_t bytes, bool up) const;
+    hipError_t pieces(char* host, char* dev, size_t bytes, bool up);
     struct Buf;
     friend struct StagingPool;
     Buf* b_ = nullptr;
+    hipStream_t s_;
+    bool waited_ = false;
     hipError_t err_ = hipSuccess;
 };
 // The pool keeps buffers while any solver handle lives: every handle holds one

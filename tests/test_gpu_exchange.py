@@ -194,3 +194,23 @@ def test_a_set_up_that_failed_halfway_is_run_again(model, call):
     assert np.array_equal(np.asarray(got), np.asarray(want))
     s.close()
     assert before - _free_bytes() <= 3 << 21
+
+
+def test_a_call_that_fails_leaves_no_work_on_its_staging_buffer():
+    """The norm's kernels write into the pinned buffer that the call gives back
+    when the residual's device rows cannot be had: behind 20 ms of residuals on
+    the stream, they have ended by the time of the error."""
+    from aeroflex_amd import rans
+    s = make(64, 1100, True)
+    s.init()
+    hip = C.CDLL(rans.LIB_PATH)
+    stream = C.c_void_p(s.stream())
+    s.launch_stage(0, 0, 400)
+    assert hip.hipStreamQuery(stream) != 0   # (not yet done: the queue is longer than the call below)
+    rans.lib.afx_fail_alloc(1)
+    try:
+        with pytest.raises(rans.RansError, match="out of memory"):
+            s.fillRhoRHS()
+    finally:
+        rans.lib.afx_fail_alloc(0)
+    assert hip.hipStreamQuery(stream) == 0
