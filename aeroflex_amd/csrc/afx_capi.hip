@@ -1365,6 +1365,7 @@ int afx_rans_set_bcs(afx_rans* h, int32_t n, const char* const* names, const int
         if (bt[b] == AFX_BC_WALL || bt[b] == AFX_BC_SLIP) { wo.push_back(own); wg.push_back(gh); }
     }
     hipStream_t s = h->stream;
+    h->bcs_set = false;   // until every table is there: a failure below leaves some of the old ones
     HIPCHK(h->fkind.upload(kind, s));
     if (h->t_fkind.p && !h->tl.fref.empty()) {
         std::vector<int8_t> tk(h->tl.fref.size());
@@ -1392,7 +1393,6 @@ int afx_rans_set_bcs(afx_rans* h, int32_t n, const char* const* names, const int
     HIPCHK(hipStreamSynchronize(s));
     h->bface_type = bt;
     h->bface_vars = bv;
-    h->bcs_set = true;
     h->wd_ready = false;
     if (h->sa()) {
         int r2 = compute_wall_distance(h);
@@ -1406,6 +1406,7 @@ int afx_rans_set_bcs(afx_rans* h, int32_t n, const char* const* names, const int
     HIPCHK(h->uni64.upload(qf, 4, s));
     HIPCHK(h->uni32.upload(qf32, 4, s));
     HIPCHK(hipStreamSynchronize(s));
+    h->bcs_set = true;
     return AFX_OK;
 }
 

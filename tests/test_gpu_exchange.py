@@ -214,3 +214,36 @@ def test_a_call_that_fails_leaves_no_work_on_its_staging_buffer():
     finally:
         rans.lib.afx_fail_alloc(0)
     assert hip.hipStreamQuery(stream) == 0
+
+
+@pytest.mark.parametrize("model", ["inviscid", "spalart-allmaras"])
+def test_boundary_conditions_that_were_set_in_part_are_refused(model):
+    """Setting them again allocates their tables anew (here with other patches of
+    wall): where that fails the solver refuses to go on until they are set."""
+    from aeroflex_amd import rans
+    far = rans.BoundaryVariables(mach=0.5, angle=0.03)
+    one = {"farfield": rans.BoundaryCondition("farfield", far), "wall": rans.BoundaryCondition("slip-wall")}
+    both = {"farfield": rans.BoundaryCondition("wall"), "wall": rans.BoundaryCondition("slip-wall")}
+    s = make(64, 33, True, model)
+    s.init()
+    s.refill_bcs()
+    q = s.get_q()
+    want = s.fillRhoRHS()
+    failed = 0
+    for nth in range(1, 12):
+        rans.lib.afx_fail_alloc(nth)
+        try:
+            s.set_bcs(both)
+            break
+        except rans.RansError as e:
+            assert "out of memory" in str(e)
+            failed += 1
+            rans.lib.afx_fail_alloc(0)
+            with pytest.raises(rans.RansError, match="boundary conditions not set"):
+                s.fillRhoRHS()
+        finally:
+            rans.lib.afx_fail_alloc(0)
+        s.set_bcs(one)
+        s.set_q(q)
+        assert np.array_equal(s.fillRhoRHS()[0], want[0])
+    assert failed >= 2
