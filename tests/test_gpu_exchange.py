@@ -19,9 +19,10 @@ def make(ni, nj, renumber, model="inviscid"):
     return s
 
 
-# 2 ni nj cells in all: less than a block of the layout kernels, one more and
-# one less than full blocks, the last direct vector (131 072 cells, 4 MB), the
-# first pieced one, a last piece of a few rows, several pieces per worker
+# 2 ni nj cells in all: less than a block of the layout kernels (256), one full
+# block, two cells more; below the last direct vector (131 072 cells, 4 MB) and on
+# it, pieced with a last piece of 128 rows and of 6 144, several pieces per worker
+# (and the vectors of one value per cell pieced too)
 @pytest.mark.parametrize("ni,nj", [(8, 3), (8, 16), (43, 3), (64, 1023), (64, 1024), (64, 1025), (67, 1024),
                                    (128, 2050)])
 def test_rows_keep_their_cells(ni, nj):

@@ -7,8 +7,9 @@ import pytest
 pytestmark = pytest.mark.gpu
 
 
-# tiles of one, a few and many cells, a mesh of one tile, quads and triangles
-@pytest.mark.parametrize("ni,nj,tile", [(16, 4, 0), (31, 12, 16), (64, 40, 0), (64, 40, 128)])
+# a mesh of one tile, tiles of few cells, the automatic ones (a thread to a cell),
+# and tiles whose rings and faces take the threads more than one turn
+@pytest.mark.parametrize("ni,nj,tile", [(16, 4, 0), (31, 12, 16), (64, 40, 0), (64, 40, 224)])
 @pytest.mark.parametrize("model,opts", [("inviscid", {}), ("laminar", {}), ("inviscid", {"second_order": False}),
                                         ("laminar", {"second_order": False}), ("inviscid", {"limiter": "michalak"}),
                                         ("laminar", {"gradient_scheme": "least-squares"})])
