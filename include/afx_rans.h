@@ -70,7 +70,8 @@ typedef struct afx_opts {
     int32_t renumber;      /* 1: tiled RCM cell order on the device (default), 0: file order */
     int32_t tile_cells;    /* cells per tile of the fused residual kernel (0: automatic, the
                               largest of 256, 224, ... whose FP64 tile fits 64 KiB of LDS;
-                              128 for meshes below 131072 cells) */
+                              128 for meshes below 131072 cells, which suits one solver:
+                              a batch of many members steps faster with 192) */
     int32_t fused;         /* 1: fused tile kernel for the residual (default), 0: three-kernel path */
     int32_t limiter;       /* 0: the reference's default limiter (solver.h:575-583, default);
                               1: its RANS_MICHALAK_LIMITER build (solver.h:557-573, physics.h:583-592).
