@@ -4,6 +4,7 @@
 
 #include <algorithm>
 #include <atomic>
+#include <cstdlib>
 #include <cstring>
 #include <exception>
 #include <mutex>
@@ -181,6 +182,20 @@ thread_local bool t_no_pinned = false;
 
 void staging_retain() { pool().retain(); }
 void staging_release() { pool().release(); }
+
+HostMemory::~HostMemory() {
+    if (pinned_) (void)hipHostFree(p_);
+    else std::free(p_);
+}
+hipError_t HostMemory::alloc(size_t bytes) {
+    if (hipHostMalloc(&p_, t_no_pinned ? size_t(1) << 60 : bytes, hipHostMallocDefault) == hipSuccess) {
+        pinned_ = true;
+        return hipSuccess;
+    }
+    (void)hipGetLastError();
+    p_ = std::malloc(bytes);
+    return p_ ? hipSuccess : hipErrorOutOfMemory;
+}
 
 Staging::Staging(hipStream_t s) : s_(s) {
     int dev = 0;

@@ -49,9 +49,25 @@ private:
     bool waited_ = false;
     hipError_t err_ = hipSuccess;
 };
+// A handle's own host memory for asynchronous copies: pinned, or ordinary where no
+// pinned memory is to be had (the copies then go through the runtime's staging).
+class HostMemory {
+public:
+    HostMemory() = default;
+    ~HostMemory();
+    HostMemory(const HostMemory&) = delete;
+    HostMemory& operator=(const HostMemory&) = delete;
+    hipError_t alloc(size_t bytes);   // once
+    void* get() const { return p_; }
+
+private:
+    void* p_ = nullptr;
+    bool pinned_ = false;
+};
+
 // The pool keeps buffers while any solver handle lives: every handle holds one
 // reference, and the last one to go frees the idle buffers.
-// Test hook, per thread: Staging asks for more pinned memory than there is.
+// Test hook, per thread: Staging and HostMemory ask for more pinned memory than there is.
 extern thread_local bool t_no_pinned;
 void staging_retain();
 void staging_release();

@@ -25,6 +25,7 @@
 #include <vector>
 
 #include "../../include/afx_vlm.h"
+#include "afx_exchange.hpp"
 #include "afx_vlm.hpp"
 
 using afx::api_fail;
@@ -1191,11 +1192,13 @@ struct afx_dense {
     int nblk = 0;
     bool anorm_known = false;   // state->anorm is |A|inf of the current FP64 matrix
     SolveState* state = nullptr;
-    struct Results {            // pinned: what factor and solve read back
+    struct Results {            // what factor and solve read back
         SolveState solve;
         int info;
         unsigned aborted;
-    }* host = nullptr;
+    };
+    afx::HostMemory results;
+    Results* host() const { return static_cast<Results*>(results.get()); }
     unsigned spin_limit = SPIN_LIMIT;   // of the panel's waits
     bool factored = false;
     ~afx_dense() {
@@ -1204,7 +1207,6 @@ struct afx_dense {
                         (void*)info, (void*)Linv, (void*)Uinv, (void*)tk,
                         (void*)yx, (void*)abort})
             if (p) (void)hipFree(p);
-        if (host) (void)hipHostFree(host);
         if (ev_panel) (void)hipEventDestroy(ev_panel);
         if (ev_near) (void)hipEventDestroy(ev_near);
         if (ev_far) (void)hipEventDestroy(ev_far);
@@ -1243,7 +1245,7 @@ int dense_init(afx_dense* h, int n) {
     VCHK(dalloc(&h->r, nn));
     VCHK(dalloc(&h->rowabs, nn));
     VCHK(dalloc(&h->state, 1));
-    VCHK(hipHostMalloc((void**)&h->host, sizeof(afx_dense::Results), hipHostMallocDefault));
+    VCHK(h->results.alloc(sizeof(afx_dense::Results)));
     VCHK(dalloc(&h->y, nn));
     const size_t nwg = (nn + PANEL_R - 1) / PANEL_R;
     VCHK(dalloc(&h->keys, 2 * nwg * KEY_STRIDE + 2 * nwg * SUB + 2 * SUB * LU_NB));
@@ -1337,10 +1339,10 @@ int dense_factor(afx_dense* h, int32_t* info_out) {
     VCHK(hipGetLastError());
     VCHK(hipEventRecord(h->ev_far, h->s2));
     VCHK(hipStreamWaitEvent(s, h->ev_far, 0));
-    VCHK(hipMemcpyAsync(&h->host->info, h->info, 2 * sizeof(int), hipMemcpyDeviceToHost, s));
+    VCHK(hipMemcpyAsync(&h->host()->info, h->info, 2 * sizeof(int), hipMemcpyDeviceToHost, s));
     VCHK(hipStreamSynchronize(s));
-    const int info = h->host->info;
-    if (h->host->aborted) return api_fail(AFX_EHIP, "LU panel: pivot exchange timed out (workgroups not co-resident)");
+    const int info = h->host()->info;
+    if (h->host()->aborted) return api_fail(AFX_EHIP, "LU panel: pivot exchange timed out (workgroups not co-resident)");
     if (info_out) *info_out = info;
     h->factored = info == 0;
     if (info) return api_fail(AFX_EARG, "matrix is singular in FP32: zero pivot at column " + std::to_string(info - 1));
@@ -1367,7 +1369,7 @@ int dense_solve_dev(afx_dense* h, const double* b_dev, double* x_dev, double tol
         k_refine_check<<<1, 1024, 0, s>>>(h->r, x_dev, b_dev, rowabs, n, it, tol, max_iter, h->abort, h->state);
     };
     evaluate(0);
-    SolveState& st = h->host->solve;
+    SolveState& st = h->host()->solve;
     for (int it = 0;;) {
         for (int q = 0; q < 2 && it < max_iter; ++q) {
             k_trsv<true><<<nb, LU_NB * TRSV_G, 0, s>>>(h->A32, h->lda, h->Linv, h->r, h->perm, h->y, nullptr, n, nb, h->tk,
@@ -1415,9 +1417,9 @@ struct afx_vlm {
            *d_normal = nullptr, *d_rhs = nullptr, *d_gamma = nullptr, *d_rforce = nullptr, *d_sforce = nullptr;
     int *d_rn = nullptr, *d_soff = nullptr, *d_rst = nullptr;
     double* d_salpha = nullptr;
-    double* stage = nullptr;   // pinned: nodes on their way in, angles and forces
+    afx::HostMemory staged;    // nodes on their way in, angles and forces
+    double* stage() const { return static_cast<double*>(staged.get()); }
     ~afx_vlm() {
-        if (stage) (void)hipHostFree(stage);
         for (void* p : {(void*)d_nodes, (void*)d_corner, (void*)d_wcorner, (void*)d_colloc, (void*)d_normal,
                         (void*)d_rhs, (void*)d_gamma, (void*)d_rforce, (void*)d_sforce, (void*)d_rn, (void*)d_soff,
                         (void*)d_rst, (void*)d_salpha})
@@ -1547,9 +1549,8 @@ int afx_vlm_create(int32_t n_nodes, const double* xyz, int32_t n_stations, const
     VCHK_C(dalloc(&h->d_soff, n_stations + 1));
     VCHK_C(dalloc(&h->d_rst, nr));
     VCHK_C(dalloc(&h->d_salpha, n_stations));
-    VCHK_C(hipHostMalloc((void**)&h->stage,
-                         sizeof(double) * std::max(3 * (size_t)n_nodes, 3 * ((size_t)nr + n_stations) + n_stations),
-                         hipHostMallocDefault));
+    VCHK_C(h->staged.alloc(sizeof(double) *
+                           std::max(3 * (size_t)n_nodes, 3 * ((size_t)nr + n_stations) + n_stations)));
     std::vector<int> rst(nr);
     for (int st = 0; st < n_stations; ++st)
         for (int k = soff[st]; k < soff[st + 1]; ++k) rst[k] = st;
@@ -1602,8 +1603,8 @@ int afx::vlm_queue_nodes(afx_vlm* h, const double* xyz) {
     if (!h || !xyz) return api_fail(AFX_EARG, "null argument");
     std::copy(xyz, xyz + 3 * (size_t)h->nn, h->xyz.begin());
     VCHK(hipStreamSynchronize(h->dense->s));   // the stage is free
-    std::copy(h->xyz.begin(), h->xyz.end(), h->stage);
-    VCHK(hipMemcpyAsync(h->d_nodes, h->stage, 3 * (size_t)h->nn * sizeof(double), hipMemcpyHostToDevice, h->dense->s));
+    std::copy(h->xyz.begin(), h->xyz.end(), h->stage());
+    VCHK(hipMemcpyAsync(h->d_nodes, h->stage(), 3 * (size_t)h->nn * sizeof(double), hipMemcpyHostToDevice, h->dense->s));
     h->built = h->solved = false;
     return AFX_OK;
 }
@@ -1692,10 +1693,10 @@ int afx_vlm_forces(afx_vlm* h, double* ring_force, double* station_force, double
                                                  h->d_rforce, h->d_sforce);
     VCHK(hipGetLastError());
     const size_t nsf = 3 * (size_t)h->ns, nrf = 3 * (size_t)h->nr;
-    const double *sf = h->stage, *rf = h->stage + nsf;
-    VCHK(hipMemcpyAsync(h->stage, h->d_sforce, nsf * sizeof(double), hipMemcpyDeviceToHost, s));
+    const double *sf = h->stage(), *rf = sf + nsf;
+    VCHK(hipMemcpyAsync(h->stage(), h->d_sforce, nsf * sizeof(double), hipMemcpyDeviceToHost, s));
     if (ring_force)
-        VCHK(hipMemcpyAsync(h->stage + nsf, h->d_rforce, nrf * sizeof(double), hipMemcpyDeviceToHost, s));
+        VCHK(hipMemcpyAsync(h->stage() + nsf, h->d_rforce, nrf * sizeof(double), hipMemcpyDeviceToHost, s));
     VCHK(hipStreamSynchronize(s));
     if (ring_force) std::copy(rf, rf + nrf, ring_force);
     if (station_force) std::copy(sf, sf + nsf, station_force);
@@ -1803,7 +1804,7 @@ int afx_vlm_nonlinear_solve(afx_vlm* h, const afx_polar* P, double relaxation, d
     for (int st = ns - 1; st >= 0; --st) spanloc[st] = (spanloc[st] - spanloc[0]) / span;
     const double q = 0.5 * f.rho * f.vinf * f.vinf;
     std::vector<double> alpha(ns, f.alpha_deg), clinv(ns);
-    double *sf = h->stage, *angles = h->stage + 3 * (size_t)ns;   // (free after each wait of the loop)
+    double *sf = h->stage(), *angles = sf + 3 * (size_t)ns;   // (free after each wait of the loop)
     VCHK(hipStreamSynchronize(h->dense->s));
     hipStream_t s = h->dense->s;
     auto lift_axis = [&](int st, double* ax) {   // unit(V(alpha_s) x dl_LE)

@@ -224,6 +224,37 @@ def test_factor_after_a_timed_out_wait(vlm, n, before):
     np.testing.assert_allclose(x, xr, rtol=0, atol=1e-12 * np.abs(xr).max())
 
 
+def test_lattice_without_pinned_memory(vlm):
+    """Handles made where no pinned memory is to be had give the same values."""
+    from aeroflex_amd import rans
+    xyz, rn, so, ref = small_wing(vlm, 8, 24)
+    rng = np.random.default_rng(3)
+    A = rng.normal(size=(300, 300)) + 300 * np.eye(300)
+    b = rng.normal(size=300)
+
+    def values():
+        d = vlm.Dense(300)
+        d.set(A)
+        d.factor()
+        h = vlm.VLM(xyz, rn, so)
+        h.set_flow(4.0, vinf=1.3, rho=0.9, sref=ref["sref"], cref=ref["cref"])
+        out = []
+        for scale in (1.0, 1.1):
+            h.set_nodes(scale * xyz)
+            h.build()
+            h.factor()
+            out += [h.solve()[0], *h.forces()[:2]]
+        return [d.solve(b)[0]] + out
+    want = values()
+    try:
+        assert rans.lib.afx_no_pinned(1) == 0
+        got = values()
+    finally:
+        rans.lib.afx_no_pinned(0)
+    for x, y in zip(got, want):
+        assert np.array_equal(x, y)
+
+
 @pytest.mark.parametrize("alpha", [2.0, 8.0])
 def test_gamma_forces_cl_match_oracle(vlm, ov, alpha):
     print(f"[vlm] solve alpha={alpha}", flush=True)
